@@ -385,8 +385,7 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, const WorkItem<T>& w,
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const float h = acc[tt][4 * c4 + e][v] + rq4[e];
-              dot += glu_fwd(gt4[e], up4[e], a.act_kind) * h;
-              glu_bwd(tw * h, gt4[e], up4[e], a.act_kind, dg[e], du[e]);
+              dot += glu_bwd(tw * h, gt4[e], up4[e], a.act_kind, dg[e], du[e]) * h;
             }
 #pragma unroll
             for (int e = 0; e < 4; e += 2) {
@@ -743,8 +742,7 @@ __device__ __forceinline__ void bwd_group_item(const BwdArgs& a, int expert, int
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const float h = acc[tt][4 * c4 + e][v] + rq4[e];
-              dot += glu_fwd(gt4[e], up4[e], a.act_kind) * h;
-              glu_bwd(tw * h, gt4[e], up4[e], a.act_kind, dg[e], du[e]);
+              dot += glu_bwd(tw * h, gt4[e], up4[e], a.act_kind, dg[e], du[e]) * h;
             }
             const uint32_t g0 = pack_bf16(dg[0], dg[1]), g1 = pack_bf16(dg[2], dg[3]);
             const uint32_t u0 = pack_bf16(du[0], du[1]), u1 = pack_bf16(du[2], du[3]);
