@@ -153,6 +153,41 @@ struct Cfg {
   static constexpr int kChunkBytes = kChunk * T * 2 * 1024;
 };
 
+// Orders this wave's LDS writes before its later LDS reads (and the other way round): the lanes of
+// one wave exchange data through LDS without a work-group barrier (LDS operations of a wave
+// complete in order; this keeps the compiler's order).
+MX_DEV void wave_lds_fence()
+{
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Four staged columns of the W2 transposed product: h = g . W2 (with the LoRA term) at columns col ..
+// col + 3 of pair row p, against the saved gate | up: writes the bf16 hi + lo gradients of gate and
+// up (where ok) and returns grad_w's partial dot of the row over the 64 columns of the lane's 16
+// lanes. The stores are non-temporal: measured faster than write-back stores for these rows.
+MX_DEV float down_t_quad(const BwdArgs& a, int p, int col, bool ok, f32x4 h, f32x4 gt, f32x4 up, float tw)
+{
+  float dg[4], du[4], dot = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) dot += glu_bwd(tw * h[e], gt[e], up[e], a.act_kind, dg[e], du[e]) * h[e];
+  const float part = group16_sum(ok ? dot : 0.f);
+  if (ok) {
+    auto st = [&](const float (&d)[4], long long o) {
+      const uint32_t h0 = pack_bf16(d[0], d[1]), h1 = pack_bf16(d[2], d[3]);
+      __builtin_nontemporal_store(u32x2{h0, h1}, reinterpret_cast<u32x2*>(a.d_hi + o));
+      __builtin_nontemporal_store(u32x2{pack_bf16(d[0] - bf16_lo(h0), d[1] - bf16_hi(h0)),
+                                        pack_bf16(d[2] - bf16_lo(h1), d[3] - bf16_hi(h1))},
+                                  reinterpret_cast<u32x2*>(a.d_lo + o));
+    };
+    const long long o = (long long)p * 2 * a.C + col;
+    st(dg, o);
+    st(du, o + a.C);
+  }
+  return part;
+}
+MX_DEV float lane_f(float v, int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l)); }
+
 // BL: the weights come from the backward layout (launch_backward_layout): each 32-row step of
 // a stripe is 4 KiB of codes read by four 16-byte loads per lane (each instruction 1 KiB
 // contiguous) and 256 B of scales read by one 8-byte load per lane, instead of eight 8-byte
@@ -353,88 +388,74 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, const WorkItem<T>& w,
     }
   }
 
-  // epilogue, tile by tile: lane (n, g) holds rows 4g..4g+3 of columns col .. col + 15 (the
-  // tile index is a compile-time constant in each call, so acc is only ever indexed statically
-  // and stays in registers)
-  const bool col_ok = stripe_ok && col < a.C;  // C is a multiple of 32: all 16 columns or none
-  auto epilogue = [&](auto ttc) {
-    constexpr int tt = decltype(ttc)::value;
-    const bool live = tt < w.ntl;  // uniform
-    const int row0 = w.row0[tt], nrows = live ? w.nrows[tt] : 0;
-    if (MODE == kBwdDownT) {
-      const int F = a.C;
+  // Epilogue through LDS. A lane's accumulators hold 16 columns of 4 rows; written from there, every
+  // global access would be 16-byte pieces 64 bytes apart and the whole tile's GLU derivatives one
+  // straight run of code (several times the instruction cache). Instead each wave stages 8 rows x
+  // 256 columns at a time in its 8 KiB of the (now idle) A buffer and takes them back row by row,
+  // lane l columns 4l .. 4l + 3: whole-line accesses, and one short loop over rows. The 16-byte
+  // pieces of a row are swizzled (piece 4n + c4 at 4n + (c4 ^ (n / 2 % 4))) so that the eight
+  // lanes of one LDS pass hit all banks. With the grouped kernel's the same way: W2 transposed of
+  // 16,000 pairs in large buckets (3584 x 3072, SiTU) 1.07 -> 0.90 ms, the Zipf
+  // step 3.10 -> 3.00 ms; uniform buckets of 9 rows unchanged (bound by the weights).
+  static_assert(T == 1, "one tile per item");
+  static_assert(NW * 8192 <= 2 * kChunkBytes, "the staged rows fit the A buffers");
+  __syncthreads();  // every wave is done with the last chunk's A operands
+  f32x4* const stage = reinterpret_cast<f32x4*>(abuf + wave * 8192);
+  const int lcol = c0 + 4 * lane;
+  const bool lcol_ok = stripe_ok && lcol < a.C;  // C is a multiple of 32: all 4 columns or none
+  const int row0 = w.row0[0], nrows = stripe_ok ? w.nrows[0] : 0;
+  static_for<2>([&](auto hc) {
+    constexpr int half = decltype(hc)::value;
+    if ((g >> 1) == half)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = 4 * g + v;
-        const bool row_ok = i < nrows;
-        const int p = row0 + (row_ok ? i : 0);
-        float dot = 0.f;
-        if (col_ok) {
-          const float tw = a.row_w[p];
-          const float* sv = a.saved + (long long)p * 2 * F + col;
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int c4 = 0; c4 < 4; ++c4)
+          stage[((g & 1) * 4 + v) * 64 + 4 * n + (c4 ^ ((n >> 1) & 3))] =
+              f32x4{acc[0][4 * c4][v], acc[0][4 * c4 + 1][v], acc[0][4 * c4 + 2][v], acc[0][4 * c4 + 3][v]};
+    wave_lds_fence();
+    const int left = nrows - 8 * half;
+    auto staged = [&](int r) { return stage[r * 64 + (lane ^ ((lane >> 3) & 3))]; };
+    if constexpr (MODE == kBwdDownT) {
+      constexpr int kB = 4;  // rows whose gate | up loads are in flight together
+#pragma unroll 1
+      for (int r0 = 0; r0 < 8; r0 += kB) {
+        if (r0 >= left) break;
+        f32x4 gt[kB], up[kB], rq[kB];
+        float tw[kB];
+#pragma unroll
+        for (int b = 0; b < kB; ++b) {
+          const int p = row0 + 8 * half + min(r0 + b, left - 1);
+          const int cc = lcol_ok ? lcol : 0;
+          tw[b] = a.row_w[p];
+          gt[b] = *reinterpret_cast<const f32x4*>(a.saved + (long long)p * 2 * a.C + cc);
+          up[b] = *reinterpret_cast<const f32x4*>(a.saved + (long long)p * 2 * a.C + a.C + cc);
           // LoRA: the down adapter's A_d^T q of the row's token joins g . W2
-          const float* rq = a.lora_rq ? a.lora_rq + (long long)a.a_row_map[p] * F + col : nullptr;
-          uint32_t dh[8], dl[8], uh[8], ul[8];
-#pragma unroll
-          for (int c4 = 0; c4 < 4; ++c4) {
-            const f32x4 gt4 = *reinterpret_cast<const f32x4*>(sv + 4 * c4);
-            const f32x4 up4 = *reinterpret_cast<const f32x4*>(sv + F + 4 * c4);
-            f32x4 rq4 = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (rq) rq4 = *reinterpret_cast<const f32x4*>(rq + 4 * c4);
-            float dg[4], du[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float h = acc[tt][4 * c4 + e][v] + rq4[e];
-              dot += glu_bwd(tw * h, gt4[e], up4[e], a.act_kind, dg[e], du[e]) * h;
-            }
-#pragma unroll
-            for (int e = 0; e < 4; e += 2) {
-              const uint32_t gh = pack_bf16(dg[e], dg[e + 1]);
-              const uint32_t hh = pack_bf16(du[e], du[e + 1]);
-              dh[2 * c4 + e / 2] = gh;
-              dl[2 * c4 + e / 2] = pack_bf16(dg[e] - bf16_lo(gh), dg[e + 1] - bf16_hi(gh));
-              uh[2 * c4 + e / 2] = hh;
-              ul[2 * c4 + e / 2] = pack_bf16(du[e] - bf16_lo(hh), du[e + 1] - bf16_hi(hh));
-            }
-          }
-          if (row_ok) {
-            const long long o = (long long)p * 2 * F + col;
-#pragma unroll
-            for (int h2 = 0; h2 < 2; ++h2) {
-              const int b = 4 * h2;
-              // non-temporal: measured faster than write-back stores for these rows
-              auto st = [&](const uint32_t* v, uint16_t* dst) {
-                __builtin_nontemporal_store(i32x4{(int)v[b], (int)v[b + 1], (int)v[b + 2], (int)v[b + 3]},
-                                            reinterpret_cast<i32x4*>(dst));
-              };
-              st(dh, a.d_hi + o + 8 * h2);
-              st(dl, a.d_lo + o + 8 * h2);
-              st(uh, a.d_hi + o + F + 8 * h2);
-              st(ul, a.d_lo + o + F + 8 * h2);
-            }
-          }
+          rq[b] = a.lora_rq ? *reinterpret_cast<const f32x4*>(a.lora_rq + (long long)a.a_row_map[p] * a.C + cc)
+                            : f32x4{0.f, 0.f, 0.f, 0.f};
         }
-        // this stripe's part of grad_w = <act, h> for the row: the 16 lanes of the row group
-        const float d = group16_sum(dot);
-        if (n == 0 && row_ok && stripe_ok) a.gw_part[(long long)(row0 + i) * a.n_ct + ct] = d;
+#pragma unroll
+        for (int b = 0; b < kB; ++b) {
+          if (r0 + b >= left) break;  // uniform
+          const int p = row0 + 8 * half + r0 + b;
+          const float d = down_t_quad(a, p, lcol, lcol_ok, staged(r0 + b) + rq[b], gt[b], up[b], tw[b]);
+          // this stripe's part of grad_w = <act, h>: the four 16-lane parts in a fixed order
+          const float sum = (lane_f(d, 0) + lane_f(d, 16)) + (lane_f(d, 32) + lane_f(d, 48));
+          if (lane == 0) a.gw_part[(long long)p * a.n_ct + ct] = sum;
+        }
       }
     } else {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = 4 * g + v;
-        if (i < nrows && col_ok) {
-          float* yr = a.y + (long long)(row0 + i) * a.ldy + col;
-#pragma unroll
-          for (int c4 = 0; c4 < 4; ++c4) {
-            f32x4 o = f32x4{acc[tt][4 * c4][v], acc[tt][4 * c4 + 1][v], acc[tt][4 * c4 + 2][v], acc[tt][4 * c4 + 3][v]};
-            if (a.accumulate) o += *reinterpret_cast<const f32x4*>(yr + 4 * c4);
-            *reinterpret_cast<f32x4*>(yr + 4 * c4) = o;
-          }
-        }
+      for (int r = 0; r < 8; ++r) {
+        if (r >= left || !lcol_ok) continue;
+        f32x4 o = staged(r);
+        f32x4* const dst = reinterpret_cast<f32x4*>(a.y + (long long)(row0 + 8 * half + r) * a.ldy + lcol);
+        if (a.accumulate) o += *dst;
+        *dst = o;
       }
     }
-  };
-  static_for<T>(epilogue);
+    wave_lds_fence();  // the rows are read before the next half is staged over them
+  });
 }
 
 // One work-group of kWaves waves per item (one row tile x kWaves stripes); the grid covers
@@ -714,69 +735,67 @@ __device__ __forceinline__ void bwd_group_item(const BwdArgs& a, int expert, int
     }
   }
 
-  // epilogue: lane (n, g) holds rows 4g..4g+3 of columns col .. col + NC - 1 of every tile
-  const bool col_ok = stripe_ok && col < a.C;
-  auto epilogue = [&](auto ttc) {
+  // epilogue through LDS, as in bwd_item: each wave stages one tile's 16 rows x 128 columns at a
+  // time in its 8 KiB of the A buffers and takes them back two rows at a time, lane l columns
+  // 4 (l % 32) .. + 3 of row l / 32 (pieces 2n + c4 at 2n + (c4 ^ (n / 4 % 2)))
+  static_assert(NC == 8 && kWaves * 8192 <= 2 * kGChunkBytes, "a staged tile is 8 KiB per wave");
+  __syncthreads();  // every wave is done with the last chunk's A operands
+  f32x4* const stage = reinterpret_cast<f32x4*>(abuf + wave * 8192);
+  const int lrow = lane >> 5, lcol = c0w + 4 * (lane & 31);
+  const bool lcol_ok = stripe_ok && lcol < a.C;
+  static_for<T>([&](auto ttc) {
     constexpr int tt = decltype(ttc)::value;
-    const int r0 = row0[tt], nr = nrows[tt];
-    if (MODE == kBwdDownT) {
-      const int F = a.C;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = 4 * g + v;
-        const bool row_ok = i < nr;
-        const int p = r0 + (row_ok ? i : 0);
-        float dot = 0.f;
-        if (col_ok && row_ok) {
-          const float tw = a.row_w[p];
-          const float* sv = a.saved + (long long)p * 2 * F + col;
-          const float* rq = a.lora_rq ? a.lora_rq + (long long)a.a_row_map[p] * F + col : nullptr;
-          const long long o = (long long)p * 2 * F + col;
+    for (int v = 0; v < 4; ++v)
 #pragma unroll
-          for (int c4 = 0; c4 < NC / 4; ++c4) {
-            const f32x4 gt4 = *reinterpret_cast<const f32x4*>(sv + 4 * c4);
-            const f32x4 up4 = *reinterpret_cast<const f32x4*>(sv + F + 4 * c4);
-            f32x4 rq4 = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (rq) rq4 = *reinterpret_cast<const f32x4*>(rq + 4 * c4);
-            float dg[4], du[4];
+      for (int c4 = 0; c4 < 2; ++c4)
+        stage[(4 * g + v) * 32 + 2 * n + (c4 ^ ((n >> 2) & 1))] =
+            f32x4{acc[tt][4 * c4][v], acc[tt][4 * c4 + 1][v], acc[tt][4 * c4 + 2][v], acc[tt][4 * c4 + 3][v]};
+    wave_lds_fence();
+    const int nr = nrows[tt];
+    auto staged = [&](int i) { return stage[i * 32 + ((lane & 31) ^ ((lane >> 3) & 1))]; };
+    if constexpr (MODE == kBwdDownT) {
+      constexpr int kB = 4;  // row pairs whose gate | up loads are in flight together
+#pragma unroll 1
+      for (int r0 = 0; r0 < 16; r0 += 2 * kB) {
+        if (r0 >= nr) break;
+        f32x4 gt[kB], up[kB], rq[kB];
+        float tw[kB];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float h = acc[tt][4 * c4 + e][v] + rq4[e];
-              dot += glu_bwd(tw * h, gt4[e], up4[e], a.act_kind, dg[e], du[e]) * h;
-            }
-            const uint32_t g0 = pack_bf16(dg[0], dg[1]), g1 = pack_bf16(dg[2], dg[3]);
-            const uint32_t u0 = pack_bf16(du[0], du[1]), u1 = pack_bf16(du[2], du[3]);
-            __builtin_nontemporal_store(u32x2{g0, g1}, reinterpret_cast<u32x2*>(a.d_hi + o + 4 * c4));
-            __builtin_nontemporal_store(u32x2{pack_bf16(dg[0] - bf16_lo(g0), dg[1] - bf16_hi(g0)),
-                                               pack_bf16(dg[2] - bf16_lo(g1), dg[3] - bf16_hi(g1))},
-                                        reinterpret_cast<u32x2*>(a.d_lo + o + 4 * c4));
-            __builtin_nontemporal_store(u32x2{u0, u1}, reinterpret_cast<u32x2*>(a.d_hi + o + F + 4 * c4));
-            __builtin_nontemporal_store(u32x2{pack_bf16(du[0] - bf16_lo(u0), du[1] - bf16_hi(u0)),
-                                               pack_bf16(du[2] - bf16_lo(u1), du[3] - bf16_hi(u1))},
-                                        reinterpret_cast<u32x2*>(a.d_lo + o + F + 4 * c4));
-          }
+        for (int b = 0; b < kB; ++b) {
+          const int p = row0[tt] + min(r0 + 2 * b + lrow, nr - 1);
+          const int cc = lcol_ok ? lcol : 0;
+          tw[b] = a.row_w[p];
+          gt[b] = *reinterpret_cast<const f32x4*>(a.saved + (long long)p * 2 * a.C + cc);
+          up[b] = *reinterpret_cast<const f32x4*>(a.saved + (long long)p * 2 * a.C + a.C + cc);
+          rq[b] = a.lora_rq ? *reinterpret_cast<const f32x4*>(a.lora_rq + (long long)a.a_row_map[p] * a.C + cc)
+                            : f32x4{0.f, 0.f, 0.f, 0.f};
         }
-        // the stripe's part of grad_w = <act, h>: the 16 lanes of the row group, then the waves
-        const float d = group16_sum(dot);
-        if (n == 0) red[(wave * T + tt) * 16 + i] = d;
+#pragma unroll
+        for (int b = 0; b < kB; ++b) {
+          const int i = r0 + 2 * b + lrow;
+          if (r0 + 2 * b >= nr) break;  // uniform
+          const float d = down_t_quad(a, row0[tt] + i, lcol, lcol_ok && i < nr, staged(i) + rq[b], gt[b], up[b], tw[b]);
+          // the wave's part of grad_w = <act, h>: the two 16-lane parts of the row
+          const float s0 = lane_f(d, 0) + lane_f(d, 16), s1 = lane_f(d, 32) + lane_f(d, 48);
+          if ((lane & 31) == 0) red[(wave * T + tt) * 16 + i] = lrow ? s1 : s0;
+        }
       }
     } else {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = 4 * g + v;
-        if (i < nr && col_ok) {
-          float* yr = a.y + (long long)(r0 + i) * a.ldy + col;
-#pragma unroll
-          for (int c4 = 0; c4 < NC / 4; ++c4) {
-            f32x4 o = f32x4{acc[tt][4 * c4][v], acc[tt][4 * c4 + 1][v], acc[tt][4 * c4 + 2][v], acc[tt][4 * c4 + 3][v]};
-            if (a.accumulate) o += *reinterpret_cast<const f32x4*>(yr + 4 * c4);
-            *reinterpret_cast<f32x4*>(yr + 4 * c4) = o;
-          }
+      for (int r = 0; r < 16; r += 2) {
+        const int i = r + lrow;
+        if (r >= nr) break;  // uniform
+        if (i < nr && lcol_ok) {
+          f32x4 o = staged(i);
+          f32x4* const dst = reinterpret_cast<f32x4*>(a.y + (long long)(row0[tt] + i) * a.ldy + lcol);
+          if (a.accumulate) o += *dst;
+          *dst = o;
         }
       }
     }
-  };
-  static_for<T>(epilogue);
+    wave_lds_fence();  // the rows are read before the next tile is staged over them
+  });
   if (MODE == kBwdDownT) {
     // grad_w partials per 256 columns: the waves of each 256-column part, in a fixed order
     constexpr int kWavesPerPart = kBwdColsPerTile / kGS;
