@@ -740,278 +740,33 @@ __global__ __launch_bounds__(64 * NW, NW == kWavesPerGroup ? 2 : 1) void fwd_ker
 }
 
 // ---------------------------------------------------------------- large buckets
-// An expert with many rows would re-read each weight byte once per 16-row tile. Its tiles come
-// in groups of up to kGroupTiles (4). A work item is one group (up to 64 rows) x eight column
-// tiles (wave w takes column tile 8 fb + w: 512 weight rows in all); a work-group of eight waves
-// holds the CU's LDS alone. Both operands go through LDS one K-quarter (one MFMA's 128 K) at a
-// time: per quarter the work-group copies the 16 KiB of activations of its four tiles and the
-// 32 KiB of weight codes of its 512 rows, three quarters deep (the one being read and two in
-// flight), and each wave issues 4 tiles x 4 column groups x 2 terms = 32 MFMAs against them.
-// Every weight byte is read once per group and every activation byte once per 512 weight rows.
+// An expert with many rows would re-read each weight byte once per 16-row tile, so its tiles come
+// in wide groups of up to kWideGroupTiles = 8. A work item is one wide group (up to 128 rows) x
+// eight column tiles (512 weight rows, 64 per wave of an eight-wave work-group that holds the CU
+// alone). Each wave loads its own weight operands straight into registers, two quarters (one
+// MFMA's 128 K) in flight; only the activations go through LDS, one quarter (8 tiles x 4 KiB, from
+// the AT layout) at a time, double-buffered. Per quarter a wave issues up to 8 tiles x 4 column
+// groups x 2 terms = 64 MFMAs, for 64 KiB the CU reads (32 KiB of activations, 32 KiB of weights).
+// Each super-chunk's activation scales (8 tiles x 512 B) go through LDS; the weight scales of four
+// super-chunks at a time (64 B per row) through a per-wave LDS window.
 //
-// Block order: MFMA q of super-chunk c takes blocks 16c + 4q .. 16c + 4q + 3 (lane group g takes
-// block 4q + g), not the one-tile kernels' 16c + 4g + q. The quarter's weight bytes of a row are
-// then one contiguous 64 B (half a cache line, whose other half the next quarter takes) instead
-// of four 16 B pieces spread over two lines, each line requested again by all four quarters.
-// The activations keep the AT layout: a quarter's operand is gathered from it in 256 B runs
-// (every run fetched once per item), and the scale bytes of blocks 4q + g, q = 0..3, are packed
-// into one register per lane at the first quarter of each super-chunk.
-constexpr int kGmT = 4;                        // row tiles per item
-constexpr int kGmWaves = 8;                    // column tiles per item
-constexpr int kGmRows = kGmWaves * 64;         // weight rows per item
-constexpr int kGmA = kGmT * 4096;              // A bytes per quarter: [tile][plane][piece][lane][16 B]
-constexpr int kGmW = kGmRows * 64;             // W bytes per quarter: [row][block][16 B]
-constexpr int kGmRing = 3;                     // quarters in LDS: the one read and two in flight
-static_assert(kGmT >= kGroupTiles, "an item holds a whole group");
-struct GemmLds {
-  uint8_t q[kGmRing][kGmA + kGmW];             // quarter buffers
-  uint8_t sw[kGmRows * 16];                    // weight scales of a super-chunk: [row][16 B]
-  uint8_t sa[kGmT * 512];                      // activation scales of a super-chunk: [tile][512 B]
-};
-
-// FL: weight codes from the forward layout (fl0 / fl1): the same bytes land in the same LDS
-// places, each copy instruction reading four 256-byte runs instead of 16 rows' 64-byte runs
-template <int MODE, bool FL>
-__device__ __forceinline__ void fwd_gemm_item(const FwdArgs& a, int expert, int t0, int ntl, int fb, int wave,
-                                              int lane, GemmLds& lds)
-{
-  constexpr int T = kGmT;
-  const int g = lane >> 4;
-  const int nb = a.K / kGroup;
-  const int nsc = at_nchunks(a.K);
-
-  WorkItem w[T];  // slots past the group's end repeat its last tile and are not stored
-#pragma unroll
-  for (int tt = 0; tt < T; ++tt) {
-    w[tt].tile = t0 + min(tt, ntl - 1);
-    const cint_ptr tl = (cint_ptr)(a.tiles + w[tt].tile);
-    w[tt].expert = expert;
-    w[tt].row0 = tl[1];
-    w[tt].nrows = tl[2];
-    w[tt].ct0 = fb * kGmWaves;
-    const int ct = fb * kGmWaves + wave;
-    w[tt].active = ct < a.n_ct;
-    w[tt].ct = w[tt].active ? ct : a.n_ct - 1;
-  }
-
-  // weight row n of item row r (0..511): wave r / 64's column tile, column group cg = (r / 16) % 4
-  // (gate/up: groups 2, 3 are W3's rows); bases of the group's matrix
-  auto w_n = [&](int r) {
-    const int ct = min(fb * kGmWaves + (r >> 6), a.n_ct - 1), cg = (r >> 4) & 3, i = r & 15;
-    return MODE == kFwdGateUp ? min(ct * 32 + (cg & 1) * 16 + i, a.R - 1) : min(ct * kFwdColsPerTile + cg * 16 + i, a.R - 1);
-  };
-  auto w_base = [&](int cg) {
-    return (MODE == kFwdGateUp && cg >= 2 ? a.wp1 : a.wp0) + (long long)expert * a.wp_estride;
-  };
-  auto s_base = [&](int cg) {
-    return (MODE == kFwdGateUp && cg >= 2 ? a.ws1 : a.ws0) + (long long)expert * a.ws_estride;
-  };
-  // the copies of quarter q of super-chunk c into buffer buf, six per wave: blocks 4q .. 4q + 3
-  // of rows 64 wave .. + 63 of W (four instructions of 16 rows x 64 B) and the KiB units
-  // (plane wave % 2, pieces 0, 1) of tile wave / 2's operand, each gathered from four 256 B runs
-  // of the AT layout; at q = 0 also the super-chunk's weight scales of its 64 rows and half
-  // (wave % 2) of tile wave / 2's 512 B of activation scales
-  auto issue = [&](int c, int q, int buf) {
-    int l = lane;
-    asm volatile("" : "+v"(l));
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {  // instruction k: column group k of this wave's tile
-      const int r = wave * 64 + k * 16 + (l >> 2), b = l & 3;
-      if constexpr (FL) {
-        // row l / 4 of the group's 16 (row group rg of the layout), block 4q + b: piece b of its
-        // super-chunk c, lane 16 q + l / 4
-        const int ct = min(fb * kGmWaves + wave, a.n_ct - 1);
-        const int row0 = MODE == kFwdGateUp ? ct * 32 + (k & 1) * 16 : ct * kFwdColsPerTile + k * 16;
-        const uint32_t rg = (uint32_t)(min(row0, a.R - 1) / 16);
-        const uint8_t* base = (MODE == kFwdGateUp && k >= 2 ? a.fl1 : a.fl0) + (long long)expert * a.fl_estride;
-        dma16_async_s_nt(base, (rg * (uint32_t)nsc + (uint32_t)c) * 4096u + (uint32_t)(b * 1024 + (16 * q + (l >> 2)) * 16),
-                         &lds.q[buf][kGmA + (wave * 64 + k * 16) * 64]);
-      } else {
-        dma16_async_s(w_base(k), (uint32_t)w_n(r) * (uint32_t)(a.K / 2) + (uint32_t)(c * 256 + (4 * q + b) * 16),
-                      &lds.q[buf][kGmA + (wave * 64 + k * 16) * 64]);
-      }
-    }
-    {
-      const int tt = wave >> 1;
-      const uint8_t* at = a.a_tiles + (long long)(t0 + min(tt, ntl - 1)) * at_tile_bytes(a.K) +
-                          (long long)c * kAtChunkBytes;
-      const int plane = wave & 1, g = l >> 4, i = l & 15;
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        // lane (i, g) of piece k holds block 4q + 2k + g / 2, elements 16 (g % 2) .. + 15, which
-        // the AT layout keeps as logical block q of its MFMA 2k + g / 2: piece q / 2 of lane
-        // 16 (2 (q % 2) + g % 2) + i
-        const int src = ((((2 * k + (g >> 1)) * 2 + plane) * 2 + (q >> 1)) * 64 + 16 * (2 * (q & 1) + (g & 1)) + i) * 16;
-        dma16_async_s(at, (uint32_t)src, &lds.q[buf][tt * 4096 + (2 * plane + k) * 1024]);
-      }
-    }
-    if (q == 0) {  // two more copies: 8 in all
-      const int r = wave * 64 + l;
-      const uint8_t* ps = s_base((r >> 4) & 3) + (long long)w_n(r) * nb;
-      dma16_async(ps + c * 16, &lds.sw[wave * 64 * 16]);
-      const int tt = wave >> 1, h = wave & 1;
-      const uint8_t* at = a.a_tiles + (long long)(t0 + min(tt, ntl - 1)) * at_tile_bytes(a.K) +
-                          (long long)c * kAtChunkBytes + kAtCodeBytes + h * 256;
-      dma4_async(at + l * 4, &lds.sa[tt * 512 + h * 256]);
-    }
-  };
-
-  f32x4 acc[T][4];
-#pragma unroll
-  for (int tt = 0; tt < T; ++tt)
-#pragma unroll
-    for (int cg = 0; cg < 4; ++cg) acc[tt][cg] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float tw[T][4];
-  if (MODE == kFwdDown)
-#pragma unroll
-    for (int tt = 0; tt < T; ++tt)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) tw[tt][v] = a.row_w[w[tt].row0 + min(4 * g + v, w[tt].nrows - 1)];
-  // gate/up: third-term masks of the tiles (bit c: super-chunk c, rare) and their union
-  uint32_t m3[T], m3_any = 0;
-  const bool use3 = MODE == kFwdGateUp && a.x3 != nullptr && *(cint_ptr)a.x3_any != 0;
-#pragma unroll
-  for (int tt = 0; tt < T; ++tt) {
-    m3[tt] = 0;
-    if (use3 && tt < ntl) {
-      m3[tt] = x3_mask(x3_flags(a, x3_slot_row(a, w[tt].row0, w[tt].nrows, lane & 15), lane), lane);
-      m3_any |= m3[tt];
-    }
-  }
-
-  // One step per quarter s (super-chunk s / 4, MFMA q = s % 4): wait for its copies (the
-  // next quarter's stay in flight), barrier, request quarter s + 2 into the buffer step s - 1
-  // read, 32 MFMAs. At q = 0 the wave takes the super-chunk's scales into registers, which frees
-  // their single LDS copy for the next super-chunk's, requested two steps later. The scale dwords
-  // are shifted so that byte q is byte 0: the MFMAs' scale selectors stay constant and one copy
-  // of the step serves all four quarters.
-  const int ns = 4 * nsc;
-  issue(0, 0, 0);
-  if (ns > 1) issue(0, 1, 1);
-  uint32_t rw[4], ra[T][2];
-  for (int s = 0; s < ns; ++s) {
-    const int c = s >> 2, q = s & 3;
-    if (s + 1 >= ns) wait_vm0();
-    else if (((s + 1) & 3) == 0) wait_vm<8>();
-    else wait_vm<6>();
-    __syncthreads();
-    if (s + 2 < ns) issue((s + 2) >> 2, (s + 2) & 3, (s + 2) % kGmRing);
-    __builtin_amdgcn_sched_barrier(0);
-    // lane-derived LDS offsets are rebuilt here each step rather than held across the loop
-    int l = lane;
-    asm volatile("" : "+v"(l));
-    const int jl = l & 15, gl = l >> 4;
-    if (q == 0) {  // byte q of each register: the scale of block 4q + g (g = this lane's group)
-      // byte g of x, y, z, w -> bytes 0..3: two byte permutes (selector 12 gives zero) and an or
-      const uint32_t lo = 0x0C0C0000u | ((4u + gl) << 8) | (uint32_t)gl, hi = (lo << 16) | 0x0C0Cu;
-      auto gather = [&](uint32_t x, uint32_t y, uint32_t z, uint32_t w) {
-        return __builtin_amdgcn_perm(y, x, lo) | __builtin_amdgcn_perm(w, z, hi);
-      };
-#pragma unroll
-      for (int cg = 0; cg < 4; ++cg) {
-        const uint4 d = *reinterpret_cast<const uint4*>(&lds.sw[(wave * 64 + cg * 16 + jl) * 16]);
-        rw[cg] = gather(d.x, d.y, d.z, d.w);
-      }
-#pragma unroll
-      for (int tt = 0; tt < T; ++tt) {  // AT holds block 4qq + g's scales at lane 16qq + i, byte g
-        uint2 s2[4];
-#pragma unroll
-        for (int qq = 0; qq < 4; ++qq) s2[qq] = *reinterpret_cast<const uint2*>(&lds.sa[tt * 512 + (16 * qq + jl) * 8]);
-        ra[tt][0] = gather(s2[0].x, s2[1].x, s2[2].x, s2[3].x);
-        ra[tt][1] = gather(s2[0].y, s2[1].y, s2[2].y, s2[3].y);
-      }
-    }
-    const uint8_t* lq = lds.q[s % kGmRing];
-    uint32_t sb[4];
-    i32x4 b[4];
-#pragma unroll
-    for (int cg = 0; cg < 4; ++cg) {
-      const int r = wave * 64 + cg * 16 + jl;
-      sb[cg] = rw[cg] >> (8 * q);
-      b[cg] = *reinterpret_cast<const i32x4*>(lq + kGmA + (r * 4 + gl) * 16);
-      const bool dead = (sb[cg] & 0xFFu) >= 253u;  // zero block, scale 2^0
-      b[cg] = dead ? i32x4{0, 0, 0, 0} : b[cg];
-      sb[cg] = dead ? 127u : sb[cg];
-    }
-#pragma unroll
-    for (int tt = 0; tt < T; ++tt) {
-      const uint8_t* pa = lq + tt * 4096 + l * 16;
-      const i32x8 ah = cat8(*reinterpret_cast<const i32x4*>(pa), *reinterpret_cast<const i32x4*>(pa + 1024));
-      const i32x8 al = cat8(*reinterpret_cast<const i32x4*>(pa + 2048), *reinterpret_cast<const i32x4*>(pa + 3072));
-      const int sah = (int)(ra[tt][0] >> (8 * q)), sal = (int)(ra[tt][1] >> (8 * q));
-#pragma unroll
-      for (int cg = 0; cg < 4; ++cg) {
-        acc[tt][cg] = mfma_f8f4<0, 0>(ah, b[cg], acc[tt][cg], sah, (int)sb[cg]);
-        acc[tt][cg] = mfma_f8f4<0, 0>(al, b[cg], acc[tt][cg], sal, (int)sb[cg]);
-      }
-    }
-    // third-term MFMAs of flagged tiles (a slow path): in this block order MFMA q's logical
-    // block lb is block 4q + lb, so lane (i, g) takes blocks 4q + g / 2 and 4q + 2 + g / 2,
-    // elements 16 (g % 2) .., and the scale of block 4q + g
-    if (c < kX3Flags && ((m3_any >> c) & 1u)) {  // uniform
-#pragma unroll
-      for (int tt = 0; tt < T; ++tt) {
-        if (tt < ntl && ((m3[tt] >> c) & 1u)) {
-          const uint8_t* row = x3_slot_row(a, w[tt].row0, w[tt].nrows, jl);
-          const bool mine = x3_row_flag(a, row, c);
-          const uint8_t* p = mine ? row + c * 512 + q * 128 + (gl >> 1) * 32 + (gl & 1) * 16 : nullptr;
-          const i32x8 a3 = mine ? cat8_ld(p, p + 64) : i32x8{0, 0, 0, 0, 0, 0, 0, 0};
-          const int s3 = mine ? (int)row[(long long)nsc * 512 + c * 16 + 4 * q + gl] : 127;
-#pragma unroll
-          for (int cg = 0; cg < 4; ++cg) acc[tt][cg] = mfma_f8f4<0, 0>(a3, b[cg], acc[tt][cg], s3, (int)sb[cg]);
-        }
-      }
-    }
-  }
-  wait_vm0();
-#pragma unroll
-  for (int tt = 0; tt < T; ++tt)
-    if (tt < ntl && w[tt].active) epilogue_direct<MODE>(a, w[tt], lane, acc[tt], tw[tt]);
-}
-
-// Resident grid over the items (group, block of eight column tiles), feature blocks outermost,
-// dealt over the XCDs in contiguous runs: the work-groups on one XCD at a time take neighbouring
-// groups (mostly of one expert) at the same columns, so they share the weights through its L2.
-template <int MODE, bool FL>
-__global__ __launch_bounds__(64 * kGmWaves, 1) void fwd_gemm_kernel(FwdArgs a)
-{
-  __shared__ GemmLds lds;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ng = *(cint_ptr)a.n_groups;
-  const int nfb = (a.n_ct + kGmWaves - 1) / kGmWaves;
-  const int total = ng * nfb;
-  const int per_xcd = (total + 7) >> 3;
-  for (int it = 0;; ++it) {
-    const int slot = (int)(blockIdx.x >> 3) + it * (int)(gridDim.x >> 3);
-    const int item = (int)(blockIdx.x & 7) * per_xcd + slot;
-    if (slot >= per_xcd || item >= total) break;
-    const int fb = item / ng, gi = item - fb * ng;
-    const cint_ptr gg = (cint_ptr)(a.groups + gi);
-    if (it > 0) __syncthreads();  // every wave is done with the previous item's LDS
-    int l = lane;
-    asm volatile("" : "+v"(l));
-    fwd_gemm_item<MODE, FL>(a, gg[0], gg[1], gg[2], fb, wave, l, lds);
-  }
-}
-
-// ---------------------------------------------------------------- large buckets, forward layout
-// With a forward layout the large buckets take wider items: one wide group (up to
-// kWideGroupTiles = 8 row tiles, 128 rows) x eight column tiles (512 weight rows, 64 per wave of
-// an eight-wave work-group that holds the CU alone). Each wave loads its own weight operands
-// straight into registers, one contiguous KiB per MFMA operand block of the forward layout
-// (two quarters in flight); only the activations go through LDS, one quarter (8 tiles x 4 KiB,
-// copied from the AT layout as it lies) at a time, double-buffered. Per quarter a wave issues
-// 8 tiles x 4 column groups x 2 terms = 64 MFMAs, for 64 KiB the CU reads (32 KiB of
-// activations, 32 KiB of weights): half the bytes per MFMA of the four-tile items, whose rate
-// the CU's reads in flight bound. Block order and lane layouts are the one-tile kernels' (MFMA q
-// takes blocks 4g + q), so both operands are copied as they lie. Each super-chunk's activation
-// scales (8 tiles x 512 B) go through LDS; the weight scales of four super-chunks at a time
-// (64 B per row) through a per-wave LDS window.
+// Forward layout: MFMA q takes blocks 4g + q, the order of the one-tile kernels, so both operands
+// are read as they lie, a weight operand as one contiguous KiB. Checkpoint layout: MFMA q takes
+// blocks 4q + g instead, so that a load instruction covers 64 contiguous bytes (one request) of
+// each of its 16 rows rather than 16-byte pieces of four requests; the activation copies gather
+// that order from the AT layout in 256-byte runs. With it 16,000 pairs over 128 experts (3584 /
+// 3072) take 1.17 ms for gate/up and 0.42 for down, where a four-tile shape with both operands
+// through LDS took 1.27 and 0.49.
+//
+// What bounds it: at full groups the matrix cores at the clock the card's power allows (8192 rows,
+// 32 experts, 7168 / 2048: 0.44 ms for gate/up, of which 0.30 with the same MFMAs on zero weights
+// and no memory traffic; a ring of four quarters of weights and three of activations, operands
+// read ahead of the barrier, requests spread between the MFMAs and an XCD-contiguous deal of the
+// items each measured the same within 2%). A quarter costs about 0.7 us + 0.24 us per tile.
 //
 // Per quarter s (super-chunk s / 4, MFMA q = s % 4): wait until only the weight loads of quarter
 // s + 1 are outstanding, barrier, request the activation copy of quarter s + 1 (and, when due,
-// the next super-chunk's activation scales and the next scale window), 64 MFMAs, then the weight
+// the next super-chunk's activation scales and the next scale window), the MFMAs, then the weight
 // loads of quarter s + 2 into the registers quarter s has just read. The copies are issued from
 // inline assembly, so the compiler counts only the weight loads, and its own wait for quarter s's
 // weights (vmcnt 4: quarter s + 1's four loads) is the one above.
@@ -1025,7 +780,7 @@ struct WideLds {
   uint8_t sw[kWgWaves][64 * 16 * kWgWin];  // weight-scale windows: [wave][row 0..63][super-chunk 0..3][16 B]
 };
 
-template <int MODE>
+template <int MODE, bool FL>
 __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int t0, int ntl, int fb, int wave,
                                               int lane, WideLds& lds)
 {
@@ -1043,31 +798,56 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
   auto s_base = [&](int cg) {
     return (MODE == kFwdGateUp && cg >= 2 ? a.ws1 : a.ws0) + (long long)expert * a.ws_estride;
   };
-  // weight operands: column group cg is row group rg = row0 / 16 of the forward layout, whose
-  // quarter s is the KiB at s * 1024 (lane l's 16 B at l * 16); past the last quarter an empty
-  // resource returns zeros without memory traffic and keeps the load count
+  // Weight operands, one 16-byte MX block per lane and column group cg. Forward layout: cg is row
+  // group rg = row0 / 16, whose quarter s is the KiB at s * 1024 (lane l's 16 B at l * 16).
+  // Checkpoint layout: lane (j, g) reads block 4q + g of row row0 + j, so that an instruction
+  // takes 64 contiguous bytes (one request) of each of 16 rows. Past the last quarter an empty
+  // resource returns zeros without memory traffic and keeps the load count.
   rsrc_t wr[4];
+  uint32_t woff[4];
 #pragma unroll
   for (int cg = 0; cg < 4; ++cg) {
-    const int rg = min(grp_row(cg), a.R - 1) / 16;
-    const uint8_t* base = (MODE == kFwdGateUp && cg >= 2 ? a.fl1 : a.fl0) + (long long)expert * a.fl_estride +
-                          (long long)rg * nsc * 4096;
-    wr[cg] = make_rsrc(base, (uint32_t)((a.R + 15) / 16 - rg) * (uint32_t)nsc * 4096u);
+    if constexpr (FL) {
+      const int rg = min(grp_row(cg), a.R - 1) / 16;
+      const uint8_t* base = (MODE == kFwdGateUp && cg >= 2 ? a.fl1 : a.fl0) + (long long)expert * a.fl_estride +
+                            (long long)rg * nsc * 4096;
+      wr[cg] = make_rsrc(base, (uint32_t)((a.R + 15) / 16 - rg) * (uint32_t)nsc * 4096u);
+      woff[cg] = (uint32_t)lane * 16u;
+    } else {
+      wr[cg] = make_rsrc((MODE == kFwdGateUp && cg >= 2 ? a.wp1 : a.wp0) + (long long)expert * a.wp_estride,
+                         (uint32_t)a.R * (uint32_t)(a.K / 2));
+      woff[cg] = (uint32_t)min(grp_row(cg) + (lane & 15), a.R - 1) * (uint32_t)(a.K / 2) + (uint32_t)g * 16u;
+    }
   }
-  const rsrc_t wr_none = make_rsrc(a.fl0, 0);
+  const rsrc_t wr_none = make_rsrc(FL ? a.fl0 : a.wp0, 0);
   auto load_b = [&](int s, i32x4 (&b)[4]) {
     const bool live = s < ns;  // uniform
 #pragma unroll
-    for (int cg = 0; cg < 4; ++cg) b[cg] = buf16_nt(live ? wr[cg] : wr_none, (uint32_t)lane * 16u, (uint32_t)s * 1024u);
+    for (int cg = 0; cg < 4; ++cg) {
+      if constexpr (FL) b[cg] = buf16_nt(live ? wr[cg] : wr_none, woff[cg], (uint32_t)s * 1024u);
+      else b[cg] = buf16(live ? wr[cg] : wr_none, woff[cg], (uint32_t)s * 64u);
+    }
   };
-  // activation copies: wave w takes tile w (the group's last tile past its end)
+  // activation copies: wave w takes tile w (past the group's end nothing: those slots are never
+  // multiplied, and a wave with fewer copies in flight only finds its waits met earlier)
+  const bool my_copy = wave < ntl;  // uniform
   const uint8_t* my_tile = a.a_tiles + (long long)(t0 + min(wave, ntl - 1)) * at_tile_bytes(a.K);
+  // (unit u = 2 plane + piece). Checkpoint layout: lane (i, g) of piece k takes block 4q + 2k + g / 2,
+  // elements 16 (g % 2) .. + 15, which the AT layout keeps as logical block q of its MFMA 2k + g / 2
   auto issue_a = [&](int s) {
-    const uint8_t* src = my_tile + (long long)(s >> 2) * kAtChunkBytes + (s & 3) * 4096;
+    if (!my_copy) return;
+    const uint8_t* src = my_tile + (long long)(s >> 2) * kAtChunkBytes;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) dma16_async_s(src, (uint32_t)(lane * 16 + u * 1024), &lds.a[s & 1][wave * 4096 + u * 1024]);
+    for (int u = 0; u < 4; ++u) {
+      const int q = s & 3;
+      const uint32_t off = FL ? (uint32_t)(q * 4096 + lane * 16 + u * 1024)
+                              : (uint32_t)((g >> 1) * 4096 + (g & 1) * 256 + (lane & 15) * 16 + (u & 1) * 8192 +
+                                           (u >> 1) * 2048 + (q >> 1) * 1024 + (q & 1) * 512);
+      dma16_async_s(src, off, &lds.a[s & 1][wave * 4096 + u * 1024]);
+    }
   };
   auto issue_sa = [&](int c) {  // lanes 32..63 repeat lanes 0..31 into the spare half
+    if (!my_copy) return;
     dma16_async_s(my_tile + (long long)c * kAtChunkBytes + kAtCodeBytes, (uint32_t)((lane & 31) * 16),
                   &lds.sa[c & 1][wave][0]);
   };
@@ -1112,10 +892,20 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
         const cint_ptr tl = (cint_ptr)(a.tiles + t0 + tt);
         const uint8_t* row = x3_slot_row(a, tl[1], tl[2], lane & 15);
         const bool mine = x3_row_flag(a, row, c);
-        const uint32_t s3 = mine ? *reinterpret_cast<const uint32_t*>(row + (long long)nsc * 512 + c * 16 + 4 * g) : 0x7F7F7F7Fu;
-        const i32x8 a3 = mine ? x3_operand(row, c, q, g) : i32x8{0, 0, 0, 0, 0, 0, 0, 0};
+        if constexpr (FL) {
+          const uint32_t s3 = mine ? *reinterpret_cast<const uint32_t*>(row + (long long)nsc * 512 + c * 16 + 4 * g) : 0x7F7F7F7Fu;
+          const i32x8 a3 = mine ? x3_operand(row, c, q, g) : i32x8{0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-        for (int cg = 0; cg < 4; ++cg) acc[tt][cg] = mfma_f8f4<q, q>(a3, b[cg], acc[tt][cg], (int)s3, (int)sb[cg]);
+          for (int cg = 0; cg < 4; ++cg) acc[tt][cg] = mfma_f8f4<q, q>(a3, b[cg], acc[tt][cg], (int)s3, (int)sb[cg]);
+        } else {
+          // MFMA q's logical block lb is block 4q + lb: lane (i, g) takes blocks 4q + g / 2 and
+          // 4q + 2 + g / 2, elements 16 (g % 2) .., and the scale of block 4q + g
+          const uint8_t* p = mine ? row + c * 512 + q * 128 + (g >> 1) * 32 + (g & 1) * 16 : nullptr;
+          const i32x8 a3 = mine ? cat8_ld(p, p + 64) : i32x8{0, 0, 0, 0, 0, 0, 0, 0};
+          const int s3 = mine ? (int)row[(long long)nsc * 512 + c * 16 + 4 * q + g] : 127;
+#pragma unroll
+          for (int cg = 0; cg < 4; ++cg) acc[tt][cg] = mfma_f8f4<0, q>(a3, b[cg], acc[tt][cg], s3, (int)sb[cg]);
+        }
       }
     }
   };
@@ -1124,11 +914,12 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
   issue_sa(0);
   issue_a(0);
   i32x4 b0[4], b1[4];
-  uint32_t rw[4];  // this super-chunk's weight scale dwords (byte q: block 4g + q)
+  uint32_t rw[4];  // this super-chunk's weight scale dwords (byte q: block 4g + q; checkpoint layout 4q + g)
   bool damaged = false;
 
   auto step = [&](int c, auto Q, i32x4 (&b)[4], bool tail) {
     constexpr int q = decltype(Q)::value;
+    constexpr int qa = FL ? q : 0;  // byte of the activation scale dwords
     const int s = 4 * c + q;
     wait_vm<4>();
     __syncthreads();
@@ -1141,7 +932,15 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
       uint32_t d = 0;
 #pragma unroll
       for (int cg = 0; cg < 4; ++cg) {
-        rw[cg] = *reinterpret_cast<const uint32_t*>(&lds.sw[wave][(cg * 16 + j) * 64 + (c % kWgWin) * 16 + (l >> 4) * 4]);
+        const uint8_t* sw = &lds.sw[wave][(cg * 16 + j) * 64 + (c % kWgWin) * 16];
+        if constexpr (FL) {
+          rw[cg] = *reinterpret_cast<const uint32_t*>(sw + (l >> 4) * 4);
+        } else {  // byte g of the four dwords: two byte permutes (selector 12 gives zero) and an or
+          const uint32_t gl = (uint32_t)(l >> 4);
+          const uint32_t lo = 0x0C0C0000u | ((4u + gl) << 8) | gl, hi = (lo << 16) | 0x0C0Cu;
+          const uint4 v = *reinterpret_cast<const uint4*>(sw);
+          rw[cg] = __builtin_amdgcn_perm(v.y, v.x, lo) | __builtin_amdgcn_perm(v.w, v.z, hi);
+        }
         d |= damaged_scale_bits(rw[cg]);
       }
       wait_lgkm0();  // before any copy may overwrite the window read here
@@ -1169,12 +968,14 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
     }
     // tile tt's operands are read from LDS while tile tt - 1's MFMAs run (one tile ahead)
     const uint8_t* la = &lds.a[q & 1][l * 16];
-    const uint8_t* ls = &lds.sa[c & 1][0][l * 8];
+    // checkpoint layout: the dwords of the AT lane (i, q), whose byte g is block 4q + g's scale
+    const uint8_t* ls = &lds.sa[c & 1][0][(FL ? l : 16 * q + (l & 15)) * 8];
     auto read_a = [&](int tt, i32x8& ah, i32x8& al, uint2& sc) {
       const uint8_t* pa = la + tt * 4096;
       ah = cat8(*reinterpret_cast<const i32x4*>(pa), *reinterpret_cast<const i32x4*>(pa + 1024));
       al = cat8(*reinterpret_cast<const i32x4*>(pa + 2048), *reinterpret_cast<const i32x4*>(pa + 3072));
       sc = *reinterpret_cast<const uint2*>(ls + tt * 1024);
+      if constexpr (!FL) sc = uint2{sc.x >> (8 * (l >> 4)), sc.y >> (8 * (l >> 4))};
     };
     i32x8 ah, al, nh, nl;
     uint2 sc, nsc2;
@@ -1190,9 +991,9 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
         // its hi MFMA wrote three instructions earlier rather than right before it
         f32x4 t4[4];
 #pragma unroll
-        for (int cg = 0; cg < 4; ++cg) t4[cg] = mfma_f8f4<q, q>(ah, b[cg], acc[tt][cg], (int)sc.x, (int)sb[cg]);
+        for (int cg = 0; cg < 4; ++cg) t4[cg] = mfma_f8f4<qa, q>(ah, b[cg], acc[tt][cg], (int)sc.x, (int)sb[cg]);
 #pragma unroll
-        for (int cg = 0; cg < 4; ++cg) acc[tt][cg] = mfma_f8f4<q, q>(al, b[cg], t4[cg], (int)sc.y, (int)sb[cg]);
+        for (int cg = 0; cg < 4; ++cg) acc[tt][cg] = mfma_f8f4<qa, q>(al, b[cg], t4[cg], (int)sc.y, (int)sb[cg]);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -1239,7 +1040,7 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
 // the full groups' items first, then the partial groups', which fill in behind them. Consecutive
 // items are the eight column blocks of one group, which run at about the same time and share its
 // activations.
-template <int MODE>
+template <int MODE, bool FL>
 __global__ __launch_bounds__(64 * kWgWaves, 1) void fwd_wide_kernel(FwdArgs a)
 {
   __shared__ WideLds lds;
@@ -1257,7 +1058,7 @@ __global__ __launch_bounds__(64 * kWgWaves, 1) void fwd_wide_kernel(FwdArgs a)
     const cint_ptr gg = (cint_ptr)(a.wgroups + gi);
     int l = lane;
     asm volatile("" : "+v"(l));
-    fwd_wide_item<MODE>(a, gg[0], gg[1], gg[2], fb, wave, l, lds);
+    fwd_wide_item<MODE, FL>(a, gg[0], gg[1], gg[2], fb, wave, l, lds);
   }
   queue_leave(a.wcounter);
 }
@@ -1299,7 +1100,7 @@ __global__ __launch_bounds__(64 * kWgWaves, 1) void fwd_fused_kernel(FwdArgs a)
     const cint_ptr gg = (cint_ptr)(a.wgroups + gi);
     int l = lane;
     asm volatile("" : "+v"(l));
-    fwd_wide_item<MODE>(a, gg[0], gg[1], gg[2], fb, wave, l, lds.w);
+    fwd_wide_item<MODE, true>(a, gg[0], gg[1], gg[2], fb, wave, l, lds.w);
   }
   queue_leave(a.wcounter);
 }
@@ -1334,7 +1135,7 @@ hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s)
   const long long blocks8 = std::min<long long>(((long long)max_tiles * n_cg8 + 7) / 8 * 8, resident_groups() / 16 * 8);
   const bool fast = fast_path(a.R, a.K);
   // the bucket split needs the tile list and the fast path; otherwise every tile takes fwd_kernel
-  const bool split = fwd_bucket_split(a.R, a.K) && a.tiles && a.small_tiles && a.groups;
+  const bool split = mode != kFwdPlain && fwd_bucket_split(a.R, a.K) && a.tiles && a.small_tiles && a.wgroups && a.wcounter;
   FwdArgs b = a;
   if (!split) {
     b.small_tiles = nullptr;
@@ -1346,7 +1147,7 @@ hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s)
   const bool fl = fast && mode != kFwdPlain && a.fl0 && (mode != kFwdGateUp || a.fl1) &&
                   forward_layout_bytes(a.R, a.K) < (1LL << 32);
   // both bucket kinds in one launch: eight-wave one-tile items and wide large-bucket items
-  const bool fused = fl && a.n_ct % 8 == 0 && split && b.wgroups && b.wcounter;
+  const bool fused = fl && a.n_ct % 8 == 0 && split;
   dim3 grid((unsigned)blocks), block(64 * kWavesPerGroup);
 #define MX_LAUNCH(M, F, L) hipLaunchKernelGGL((fwd_kernel<M, F, L>), grid, block, 0, s, b)
   if (mode == kFwdPlain) {
@@ -1371,21 +1172,14 @@ hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s)
 #undef MX_LAUNCH
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !split) return e;
-  dim3 mgrid((unsigned)(resident_groups() / 16 * 8)), mblock(64 * kGmWaves);  // one per CU, a multiple of 8
-  if (fl && b.wgroups && b.wcounter && mode != kFwdPlain) {  // wide groups, weights straight from the forward layout
-    dim3 wblock(64 * kWgWaves);
-    if (mode == kFwdGateUp) hipLaunchKernelGGL((fwd_wide_kernel<kFwdGateUp>), mgrid, wblock, 0, s, b);
-    else hipLaunchKernelGGL((fwd_wide_kernel<kFwdDown>), mgrid, wblock, 0, s, b);
-    return hipGetLastError();
-  }
+  dim3 mgrid((unsigned)(resident_groups() / 16 * 8));  // one per CU, a multiple of 8
+  dim3 wblock(64 * kWgWaves);
   if (mode == kFwdGateUp) {
-    if (fl) hipLaunchKernelGGL((fwd_gemm_kernel<kFwdGateUp, true>), mgrid, mblock, 0, s, b);
-    else hipLaunchKernelGGL((fwd_gemm_kernel<kFwdGateUp, false>), mgrid, mblock, 0, s, b);
-  } else if (mode == kFwdDown) {
-    if (fl) hipLaunchKernelGGL((fwd_gemm_kernel<kFwdDown, true>), mgrid, mblock, 0, s, b);
-    else hipLaunchKernelGGL((fwd_gemm_kernel<kFwdDown, false>), mgrid, mblock, 0, s, b);
+    if (fl) hipLaunchKernelGGL((fwd_wide_kernel<kFwdGateUp, true>), mgrid, wblock, 0, s, b);
+    else hipLaunchKernelGGL((fwd_wide_kernel<kFwdGateUp, false>), mgrid, wblock, 0, s, b);
   } else {
-    hipLaunchKernelGGL((fwd_gemm_kernel<kFwdPlain, false>), mgrid, mblock, 0, s, b);
+    if (fl) hipLaunchKernelGGL((fwd_wide_kernel<kFwdDown, true>), mgrid, wblock, 0, s, b);
+    else hipLaunchKernelGGL((fwd_wide_kernel<kFwdDown, false>), mgrid, wblock, 0, s, b);
   }
   return hipGetLastError();
 }

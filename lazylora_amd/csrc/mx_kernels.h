@@ -53,15 +53,15 @@ struct FwdArgs {
   long long x3_row_bytes;
   const int* x3_any;
   // Bucket split (with a tile list and K a multiple of 512): the tiles of small buckets
-  // (indices into `tiles`) take the one-row-tile work-groups; large-bucket groups of up to
-  // kGroupTiles tiles ({expert, first tile, tiles, 0}) take work-groups that share each column
-  // tile's weights over the group's row tiles. Null small_tiles: every tile takes the first shape.
+  // (indices into `tiles`) take the one-row-tile work-groups; the large buckets' tiles, in groups
+  // ({expert, first tile, tiles, 0}), work-groups that share each column tile's weights over the
+  // group's row tiles. Null small_tiles: every tile takes the first shape.
   const int* small_tiles;
   const int* n_small;
   const int4* groups;
   const int* n_groups;
   // The same large-bucket tiles as wide groups of up to kWideGroupTiles tiles, taken instead of
-  // `groups` by the large-bucket work-groups that read a forward layout (null: use `groups`).
+  // `groups` by the forward's large-bucket work-groups.
   const int4* wgroups;
   const int* n_wgroups;
   int* wcounter;  // the wide-group launch's work queue: 2 ints, zero before the first launch (queue_next)
@@ -138,7 +138,7 @@ struct BwdArgs {
 
 constexpr int kFwdRowsPerTile = 16;
 constexpr int kGroupTiles = 4;     // row tiles of one large-bucket group
-constexpr int kWideGroupTiles = 8;  // row tiles of one wide group (the forward-layout large-bucket forward)
+constexpr int kWideGroupTiles = 8;  // row tiles of one wide group (the large-bucket forward)
 constexpr int kGroupMinTiles = 4;  // experts with at least this many tiles take the large-bucket path
 constexpr int kFwdColsPerTile = 64;  // kFwdPlain / kFwdDown; kFwdGateUp covers 32 features
 constexpr int kBwdColsPerTile = 256;  // output columns of one transposed-product wave
