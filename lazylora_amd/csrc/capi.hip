@@ -830,7 +830,7 @@ int mxfp4_moe_backward_fl(float* grad_h, float* grad_w, const float* grad_out, c
   b.nseg = 1; b.R = D; b.C = F;
   b.a_hi = at<uint16_t>(workspace, L.g_hi); b.a_lo = at<uint16_t>(workspace, L.g_lo); b.lda = D;
   b.a_row_map = at<int>(workspace, L.pair_token);
-  b.tiles = at<int4>(workspace, L.tiles); b.n_tiles = at<int>(workspace, L.meta);
+  b.tiles = at<int4>(workspace, L.tiles); b.n_tiles = at<int>(workspace, L.meta); b.M = (int)P;
   b.n_ct = L.n_ct_bwd;
   b.row_w = at<float>(workspace, L.pair_w);
   b.saved = at<float>(workspace, L.saved);
@@ -872,7 +872,7 @@ int mxfp4_moe_backward_fl(float* grad_h, float* grad_w, const float* grad_out, c
   c.ws_estride = (long long)F * D / 32;
   c.nseg = 2; c.R = F; c.C = D;
   c.a_hi = at<uint16_t>(workspace, L.d_hi); c.a_lo = at<uint16_t>(workspace, L.d_lo); c.lda = 2LL * F;
-  c.tiles = at<int4>(workspace, L.tiles); c.n_tiles = at<int>(workspace, L.meta);
+  c.tiles = at<int4>(workspace, L.tiles); c.n_tiles = at<int>(workspace, L.meta); c.M = (int)P;
   c.n_ct = (D + mx::kBwdColsPerTile - 1) / mx::kBwdColsPerTile;
   c.y = at<float>(workspace, L.ypair); c.ldy = D;
   set_buckets(c, workspace, L);

@@ -69,22 +69,21 @@ __device__ __forceinline__ int one_tile_count(const BwdArgs& a)
                            : a.tiles ? *(cint_ptr)a.n_tiles : (a.M + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
 }
 
-// Work item `it` of this work-group among items of NW stripes (items are dealt round-robin over
-// the XCDs, blockIdx % 8, each XCD taking one contiguous run, in strides of the grid, so the stripe
-// blocks of one tile, which read the same A rows, run on one XCD). Returns 0 when there is none
-// left, 1 for an item.
+// The work item of one-tile work-group `bid` among items of NW stripes (items are dealt round-robin
+// over the XCDs, bid % 8, each XCD taking one contiguous run, so the stripe blocks of one tile,
+// which read the same A rows, run on one XCD). Returns whether there is one.
 template <int T, int NW>
-__device__ __forceinline__ int decode_work(const BwdArgs& a, int it, WorkItem<T>& w)
+__device__ __forceinline__ bool decode_work(const BwdArgs& a, int bid, WorkItem<T>& w)
 {
-  static_assert(T == 1, "large buckets take bwd_group_kernel");
+  static_assert(T == 1, "large buckets take bwd_group_item");
   const bool use_small = use_small_list(a);
   const int count = one_tile_count(a);
   const int n_ct4 = (a.n_ct + NW - 1) / NW;
   const int total = count * n_ct4;
   const int per_xcd = (total + 7) >> 3;
-  const int slot = (int)(blockIdx.x >> 3) + it * (int)(gridDim.x >> 3);
-  const int item = (int)(blockIdx.x & 7) * per_xcd + slot;
-  if (slot >= per_xcd || item >= total) return 0;
+  const int slot = bid >> 3;
+  const int item = (bid & 7) * per_xcd + slot;
+  if (slot >= per_xcd || item >= total) return false;
   const int i = item / n_ct4;
   w.ct4 = item - i * n_ct4;
   const int t0 = use_small ? ((cint_ptr)a.small_tiles)[i] : i;
@@ -103,7 +102,7 @@ __device__ __forceinline__ int decode_work(const BwdArgs& a, int it, WorkItem<T>
       w.nrows[tt] = min(kFwdRowsPerTile, a.M - w.row0[tt]);
     }
   }
-  return 1;
+  return true;
 }
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -458,30 +457,6 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, const WorkItem<T>& w,
   });
 }
 
-// One work-group of kWaves waves per item (one row tile x kWaves stripes); the grid covers
-// every item. With `wide` the launch has an eight-stripe companion (bwd_wide_kernel) and each
-// kernel runs only when its item count suits it: this one when there are fewer than
-// kWideMinItems eight-stripe items. BL: the weights come from the backward layout.
-template <int MODE, bool BL>
-__global__ __launch_bounds__(64 * kWaves, 2) void bwd_kernel(BwdArgs a, int wide)
-{
-  __shared__ __attribute__((aligned(16))) uint8_t abuf[2 * Cfg<1>::kChunkBytes];
-  if (wide && one_tile_count(a) * ((a.n_ct + kWideWaves - 1) / kWideWaves) >= kWideMinItems) return;
-  WorkItem<1> w;
-  if (decode_work<1, kWaves>(a, 0, w) == 1) bwd_item<MODE, 1, BL, kWaves>(a, w, abuf);
-}
-
-// The same items with eight stripes (one work-group per CU; the grid covers every item); it runs
-// only when there are at least kWideMinItems of them (else bwd_kernel takes the launch's items).
-template <int MODE, bool BL>
-__global__ __launch_bounds__(64 * kWideWaves, 1) void bwd_wide_kernel(BwdArgs a)
-{
-  __shared__ __attribute__((aligned(16))) uint8_t abuf[2 * Cfg<1>::kChunkBytes];
-  if (one_tile_count(a) * ((a.n_ct + kWideWaves - 1) / kWideWaves) < kWideMinItems) return;
-  WorkItem<1> w;
-  if (decode_work<1, kWideWaves>(a, 0, w) == 1) bwd_item<MODE, 1, BL, kWideWaves>(a, w, abuf);
-}
-
 // ---------------------------------------------------------------- large buckets
 // An expert with many rows would stream (and decode) its weights once per row tile. Its tiles
 // come in groups of up to kGroupTiles (4) consecutive tiles; a work item is GT of them (a part of
@@ -814,31 +789,58 @@ __device__ __forceinline__ void bwd_group_item(const BwdArgs& a, int expert, int
   }
 }
 
-// Resident grid over the large-bucket items (group, part, column block), dealt round-robin over
-// the XCDs like the one-tile items, so launches with few or no groups cost almost nothing.
+// Both bucket kinds in one launch. The first `gblocks` work-groups (a multiple of 8; 0 without a
+// bucket split) are a resident grid over the large-bucket items (group, part, column block), dealt
+// round-robin over the XCDs like the one-tile items: the longer items start first and the one-tile
+// items fill the slots beside and behind them (128 tokens, top-16 of 64 experts, 3584 / 3072: the
+// two transposed products 0.32 and 0.46 ms in two launches each, 0.20 and 0.38 in one), and a routing without large buckets
+// pays for no second launch. Every further work-group takes one one-tile item (one row tile x
+// kWaves stripes), the grid covering them all; with `wide` these have an eight-stripe companion
+// (bwd_wide_kernel) and run only when there are fewer than kWideMinItems eight-stripe items. BL:
+// the weights come from the backward layout.
 template <int MODE, bool BL>
-__global__ __launch_bounds__(64 * kWaves, MX_BWD_GPER_CU) void bwd_group_kernel(BwdArgs a)
+__global__ __launch_bounds__(64 * kWaves, MX_BWD_GPER_CU) void bwd_kernel(BwdArgs a, int wide, int gblocks)
 {
-  __shared__ __attribute__((aligned(16))) uint8_t abuf[2 * kGChunkBytes];
-  __shared__ float red[kWaves * kGT * 16];
-  const int ng = *(cint_ptr)a.n_groups;
-  const int ncb = (a.C + kGCols - 1) / kGCols;
-  const int total = ng * kGParts * ncb;
-  const int per_xcd = (total + 7) >> 3;
-  bool busy = false;
-  for (int it = 0;; ++it) {
-    const int slot = (int)(blockIdx.x >> 3) + it * (int)(gridDim.x >> 3);
-    const int item = (int)(blockIdx.x & 7) * per_xcd + slot;
-    if (slot >= per_xcd || item >= total) break;
-    const int gp = item / ncb, cb = item - gp * ncb;
-    const int gi = gp / kGParts, part = gp - gi * kGParts;
-    const cint_ptr gg = (cint_ptr)(a.groups + gi);
-    const int ntl = gg[2] - part * kGT;
-    if (ntl <= 0) continue;  // the empty part of a short group
-    if (busy) __syncthreads();  // every wave has finished reading the previous item's LDS
-    bwd_group_item<MODE, BL>(a, gg[0], gg[1] + part * kGT, min(ntl, kGT), cb, abuf, red);
-    busy = true;
+  static_assert(2 * kGChunkBytes <= 2 * Cfg<1>::kChunkBytes, "the A buffers serve both kinds");
+  __shared__ __attribute__((aligned(16))) uint8_t abuf[2 * Cfg<1>::kChunkBytes];
+  if constexpr (MODE != kBwdPlain) {
+    if ((int)blockIdx.x < gblocks) {
+      __shared__ float red[kWaves * kGT * 16];
+      const int ng = *(cint_ptr)a.n_groups;
+      const int ncb = (a.C + kGCols - 1) / kGCols;
+      const int total = ng * kGParts * ncb;
+      const int per_xcd = (total + 7) >> 3;
+      bool busy = false;
+      for (int it = 0;; ++it) {
+        const int slot = (int)(blockIdx.x >> 3) + it * (gblocks >> 3);
+        const int item = (int)(blockIdx.x & 7) * per_xcd + slot;
+        if (slot >= per_xcd || item >= total) break;
+        const int gp = item / ncb, cb = item - gp * ncb;
+        const int gi = gp / kGParts, part = gp - gi * kGParts;
+        const cint_ptr gg = (cint_ptr)(a.groups + gi);
+        const int ntl = gg[2] - part * kGT;
+        if (ntl <= 0) continue;  // the empty part of a short group
+        if (busy) __syncthreads();  // every wave has finished reading the previous item's LDS
+        bwd_group_item<MODE, BL>(a, gg[0], gg[1] + part * kGT, min(ntl, kGT), cb, abuf, red);
+        busy = true;
+      }
+      return;
+    }
   }
+  if (wide && one_tile_count(a) * ((a.n_ct + kWideWaves - 1) / kWideWaves) >= kWideMinItems) return;
+  WorkItem<1> w;
+  if (decode_work<1, kWaves>(a, (int)blockIdx.x - gblocks, w)) bwd_item<MODE, 1, BL, kWaves>(a, w, abuf);
+}
+
+// The one-tile items with eight stripes (one work-group per CU; the grid covers every item); it runs
+// only when there are at least kWideMinItems of them (else bwd_kernel takes the launch's items).
+template <int MODE, bool BL>
+__global__ __launch_bounds__(64 * kWideWaves, 1) void bwd_wide_kernel(BwdArgs a)
+{
+  __shared__ __attribute__((aligned(16))) uint8_t abuf[2 * Cfg<1>::kChunkBytes];
+  if (one_tile_count(a) * ((a.n_ct + kWideWaves - 1) / kWideWaves) < kWideMinItems) return;
+  WorkItem<1> w;
+  if (decode_work<1, kWideWaves>(a, (int)blockIdx.x, w)) bwd_item<MODE, 1, BL, kWideWaves>(a, w, abuf);
 }
 
 int resident_groups(int per_cu)
@@ -862,8 +864,8 @@ hipError_t launch_bwd(const BwdArgs& a, int mode, int max_tiles, hipStream_t s)
   // the epilogue's 16-byte accesses of rows assume these (true for every caller: C is a multiple
   // of 32 and the row strides are multiples of 16 elements)
   if (a.C % 32 || (a.y && a.ldy % 4) || a.lda % 8) return hipErrorInvalidValue;
-  // large buckets take the grouped kernel when their scale rows are whole dwords
-  const bool split = a.tiles && a.small_tiles && a.groups && a.C % 128 == 0;
+  // large buckets take the grouped items when their scale rows are whole dwords
+  const bool split = mode != kBwdPlain && a.tiles && a.small_tiles && a.groups && a.C % 128 == 0;
   BwdArgs b = a;
   if (!split) {
     b.small_tiles = nullptr;
@@ -878,28 +880,24 @@ hipError_t launch_bwd(const BwdArgs& a, int mode, int max_tiles, hipStream_t s)
   long long blocks = (total + 7) / 8 * 8;
   if (wide)  // bwd_kernel then runs only with fewer than kWideMinItems wide items: twice as many of its own
     blocks = (std::min<long long>(total, 2LL * kWideMinItems) + 7) / 8 * 8;
-  dim3 grid((unsigned)blocks), block(64 * kWaves);
-  if (mode == kBwdPlain) hipLaunchKernelGGL((bwd_kernel<kBwdPlain, false>), grid, block, 0, s, b, 0);
-  else if (mode == kBwdDownT && bl) hipLaunchKernelGGL((bwd_kernel<kBwdDownT, true>), grid, block, 0, s, b, wide);
-  else if (mode == kBwdDownT) hipLaunchKernelGGL((bwd_kernel<kBwdDownT, false>), grid, block, 0, s, b, wide);
-  else if (bl) hipLaunchKernelGGL((bwd_kernel<kBwdGateUpT, true>), grid, block, 0, s, b, 0);
-  else hipLaunchKernelGGL((bwd_kernel<kBwdGateUpT, false>), grid, block, 0, s, b, 0);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if (wide) {
-    dim3 wgrid((unsigned)((witems + 7) / 8 * 8)), wblock(64 * kWideWaves);
-    hipLaunchKernelGGL((bwd_wide_kernel<kBwdDownT, true>), wgrid, wblock, 0, s, b);
-    e = hipGetLastError();
+  // groups come from experts with at least kGroupMinTiles tiles: at most one per 32 rows (two from 65)
+  long long gblocks = 0;
+  if (split) {
+    const long long gtotal = (long long)(a.M / 32) * kGParts * ((a.C + kGCols - 1) / kGCols);
+    gblocks = std::min<long long>((gtotal + 7) / 8 * 8, resident_groups(MX_BWD_GPER_CU));
   }
-  if (e != hipSuccess || !split) return e;
-  // groups come from experts of at least kGroupMinTiles tiles: at most max_tiles / kGroupMinTiles + 1
-  const long long gtotal = ((long long)max_tiles / kGroupMinTiles + 1) * kGParts * ((a.C + kGCols - 1) / kGCols);
-  dim3 ggrid((unsigned)std::min<long long>((gtotal + 7) / 8 * 8, resident_groups(MX_BWD_GPER_CU)));
-  if (mode == kBwdPlain) hipLaunchKernelGGL((bwd_group_kernel<kBwdPlain, false>), ggrid, block, 0, s, b);
-  else if (mode == kBwdDownT && bl) hipLaunchKernelGGL((bwd_group_kernel<kBwdDownT, true>), ggrid, block, 0, s, b);
-  else if (mode == kBwdDownT) hipLaunchKernelGGL((bwd_group_kernel<kBwdDownT, false>), ggrid, block, 0, s, b);
-  else if (bl) hipLaunchKernelGGL((bwd_group_kernel<kBwdGateUpT, true>), ggrid, block, 0, s, b);
-  else hipLaunchKernelGGL((bwd_group_kernel<kBwdGateUpT, false>), ggrid, block, 0, s, b);
+  dim3 grid((unsigned)(gblocks + blocks)), block(64 * kWaves);
+#define MX_LAUNCH(M, L) hipLaunchKernelGGL((bwd_kernel<M, L>), grid, block, 0, s, b, wide, (int)gblocks)
+  if (mode == kBwdPlain) MX_LAUNCH(kBwdPlain, false);
+  else if (mode == kBwdDownT && bl) MX_LAUNCH(kBwdDownT, true);
+  else if (mode == kBwdDownT) MX_LAUNCH(kBwdDownT, false);
+  else if (bl) MX_LAUNCH(kBwdGateUpT, true);
+  else MX_LAUNCH(kBwdGateUpT, false);
+#undef MX_LAUNCH
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !wide) return e;
+  dim3 wgrid((unsigned)((witems + 7) / 8 * 8)), wblock(64 * kWideWaves);
+  hipLaunchKernelGGL((bwd_wide_kernel<kBwdDownT, true>), wgrid, wblock, 0, s, b);
   return hipGetLastError();
 }
 

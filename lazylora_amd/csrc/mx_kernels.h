@@ -107,7 +107,7 @@ struct BwdArgs {
   const int* a_row_map;
   const int4* tiles;
   const int* n_tiles;
-  int M;
+  int M;  // rows: all of them, or with a tile list at most
   int n_ct;  // column tiles of kBwdColsPerTile
   float* y;
   long long ldy;
