@@ -1105,6 +1105,210 @@ __global__ __launch_bounds__(64 * kWgWaves, 1) void fwd_fused_kernel(FwdArgs a)
   queue_leave(a.wcounter);
 }
 
+// ---------------------------------------------------------------- few work items
+// With few row tiles the shapes above leave most of the chip idle: one row against W [2048, 7168]
+// is 8 work-groups of fwd_kernel, each wave 14 super-chunks in series (30 us for 7.8 MB), and one
+// token's 8 experts 64 eight-wave items of gate/up. Here the waves of a work-group share one
+// output tile and split K instead: wave w takes column sub-tile w / KS and the super-chunks
+// ks, ks + KS, .. (ks = w % KS), everything it needs of a chunk requested at once straight from
+// memory, and the partial sums meet in LDS, where they are added in the order of ks (fixed, so the
+// results do not depend on timing). An item is T row tiles x (8 / KS) sub-tiles of 16 G columns;
+// gate/up needs G = 4 (32 gate and 32 up features, whole MX blocks of act). Column blocks are the
+// fast index, padded to the 8 XCDs, so the row groups that share weights run on one XCD.
+constexpr int kSplitWaves = 8;
+
+__host__ __device__ inline long long forward_layout_size(int R, int K)
+{
+  return (long long)((R + 15) / 16) * (K / kChunk) * (4096 + 256);
+}
+
+template <int MODE, bool FL, int G, int T, int KS>
+__global__ __launch_bounds__(64 * kSplitWaves) void fwd_split_kernel(FwdArgs a)
+{
+  static_assert(kSplitWaves % KS == 0 && (MODE == kFwdPlain || (G == 4 && T == 1)), "routed items are one-tile, 64 columns");
+  constexpr int kSub = kSplitWaves / KS;  // column sub-tiles per work-group
+  constexpr bool kXt = MODE == kFwdGateUp;
+  __shared__ float part[kSplitWaves][T * 16][16 * G + 4];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = lane & 15, g = lane >> 4;
+  const int ks = wave % KS, sub = wave / KS;
+  const int n_sub = (MODE == kFwdGateUp ? 2 * a.R : a.R) / (16 * G) + ((MODE == kFwdGateUp ? 2 * a.R : a.R) % (16 * G) ? 1 : 0);
+  const int ncb = (n_sub + kSub - 1) / kSub, ncb8 = (ncb + 7) / 8 * 8;
+  const int cb = (int)(blockIdx.x % (unsigned)ncb8), rgrp = (int)(blockIdx.x / (unsigned)ncb8);
+  if (cb >= ncb) return;
+  const int nb = a.K / kGroup, nsc = at_nchunks(a.K);
+  WorkItem w[T];
+  const int ntiles = a.tiles ? *(cint_ptr)a.n_tiles : (a.M + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
+  if (rgrp * T >= ntiles) return;  // the whole work-group
+#pragma unroll
+  for (int tt = 0; tt < T; ++tt) {
+    w[tt].tile = min(rgrp * T + tt, ntiles - 1);
+    if (a.tiles) {
+      const cint_ptr tl = (cint_ptr)(a.tiles + w[tt].tile);
+      w[tt].expert = tl[0];
+      w[tt].row0 = tl[1];
+      w[tt].nrows = tl[2];
+    } else {
+      w[tt].expert = 0;
+      w[tt].row0 = w[tt].tile * kFwdRowsPerTile;
+      w[tt].nrows = min(kFwdRowsPerTile, a.M - w[tt].row0);
+    }
+    w[tt].ct0 = w[tt].ct = cb * kSub + sub;
+    w[tt].active = w[tt].ct < n_sub;
+  }
+  const int ct = min(cb * kSub + sub, n_sub - 1), expert = w[0].expert;
+  auto grp_row = [&](int grp) { return MODE == kFwdGateUp ? ct * 32 + (grp & 1) * 16 : ct * 16 * G + grp * 16; };
+
+  // weights as in fwd_item (block 4g + q of row j's super-chunk), codes and scales through buffer
+  // resources: past the matrix's end they read as zeros, and a block past a row's end (K not a
+  // multiple of 512) meets zero activations
+  rsrc_t wr[2], sr[2];
+#pragma unroll
+  for (int h = 0; h < (MODE == kFwdGateUp ? 2 : 1); ++h) {
+    if constexpr (FL) {
+      const uint8_t* base = (h ? a.fl1 : a.fl0) + (long long)expert * a.fl_estride;
+      wr[h] = make_rsrc(base, (uint32_t)forward_layout_size(a.R, a.K));
+      sr[h] = wr[h];
+    } else {
+      wr[h] = make_rsrc((h ? a.wp1 : a.wp0) + (long long)expert * a.wp_estride, (uint32_t)a.R * (uint32_t)(a.K / 2));
+      sr[h] = make_rsrc((h ? a.ws1 : a.ws0) + (long long)expert * a.ws_estride, (uint32_t)a.R * (uint32_t)nb);
+    }
+  }
+  f32x4 acc[T][G];
+#pragma unroll
+  for (int tt = 0; tt < T; ++tt)
+#pragma unroll
+    for (int grp = 0; grp < G; ++grp) acc[tt][grp] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const bool use3 = MODE == kFwdGateUp && a.x3 != nullptr && *(cint_ptr)a.x3_any != 0;
+  for (int c = ks; c < nsc; c += KS) {
+    i32x4 b[G][4];
+    uint32_t sb[G];
+#pragma unroll
+    for (int grp = 0; grp < G; ++grp) {
+      const int h = MODE == kFwdGateUp ? grp >> 1 : 0;
+      if constexpr (FL) {
+        const uint32_t rg = (uint32_t)(min(grp_row(grp), a.R - 1) / 16), nrg = (uint32_t)((a.R + 15) / 16);
+        const uint32_t blk = rg * (uint32_t)nsc + (uint32_t)c;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) b[grp][q] = buf16_nt(wr[h], (uint32_t)lane * 16u + 1024u * q, blk * 4096u);
+        sb[grp] = buf4_nt(sr[h], (uint32_t)lane * 4u, nrg * (uint32_t)nsc * 4096u + blk * 256u);
+      } else {
+        const uint32_t n = (uint32_t)min(grp_row(grp) + j, a.R - 1);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) b[grp][q] = buf16(wr[h], n * (uint32_t)(a.K / 2) + (uint32_t)(c * 256 + g * 64 + 16 * q), 0u);
+        const uint32_t so = n * (uint32_t)nb + (uint32_t)(c * 16 + 4 * g);
+        if ((nb & 3) == 0) {  // uniform: whole dwords of scales
+          sb[grp] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(sr[h], (int)so, 0, 0);
+        } else {
+          sb[grp] = (uint32_t)buf8(sr[h], so) | (uint32_t)buf8(sr[h], so + 1) << 8 | (uint32_t)buf8(sr[h], so + 2) << 16 |
+                    (uint32_t)buf8(sr[h], so + 3) << 24;
+        }
+      }
+    }
+    i32x8 ah[T][4], al[T][4];
+    uint2 s2[T];
+#pragma unroll
+    for (int tt = 0; tt < T; ++tt) {
+      const ASrc<kXt> as(a, w[tt], lane);
+      s2[tt] = uint2{0u, 0u};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) ah[tt][q] = al[tt][q] = i32x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (j < w[tt].nrows) {  // the rows there are
+        s2[tt] = as.scales(c);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          ah[tt][q] = cat8(ldg16(as.unit(c, 4 * q)), ldg16(as.unit(c, 4 * q + 1)));
+          al[tt][q] = cat8(ldg16(as.unit(c, 4 * q + 2)), ldg16(as.unit(c, 4 * q + 3)));
+        }
+      }
+    }
+    uint32_t d = 0;
+#pragma unroll
+    for (int grp = 0; grp < G; ++grp) d |= damaged_scale_bits(sb[grp]);
+    if (__builtin_amdgcn_ballot_w64(d != 0u) != 0) {  // scale bytes >= 253: zero block, scale 2^0 (rare)
+#pragma unroll
+      for (int grp = 0; grp < G; ++grp)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const bool dead = ((sb[grp] >> (8 * q)) & 0xFFu) >= 253u;
+          b[grp][q] = dead ? i32x4{0, 0, 0, 0} : b[grp][q];
+          sb[grp] = dead ? (sb[grp] & ~(0xFFu << (8 * q))) | (127u << (8 * q)) : sb[grp];
+        }
+    }
+    static_for<4>([&](auto qc) {
+      constexpr int q = decltype(qc)::value;
+#pragma unroll
+      for (int tt = 0; tt < T; ++tt)
+#pragma unroll
+        for (int grp = 0; grp < G; ++grp) {
+          acc[tt][grp] = mfma_f8f4<q, q>(ah[tt][q], b[grp][q], acc[tt][grp], (int)s2[tt].x, (int)sb[grp]);
+          acc[tt][grp] = mfma_f8f4<q, q>(al[tt][q], b[grp][q], acc[tt][grp], (int)s2[tt].y, (int)sb[grp]);
+        }
+    });
+    if constexpr (MODE == kFwdGateUp) {
+      if (use3 && c < kX3Flags) {  // the third term of x, where a row has one in this super-chunk
+        const uint8_t* row = x3_slot_row(a, w[0].row0, w[0].nrows, j);
+        const bool mine = x3_row_flag(a, row, c);
+        if (__builtin_amdgcn_ballot_w64(mine) != 0) {
+          const uint32_t s3 = mine ? *reinterpret_cast<const uint32_t*>(row + (long long)nsc * 512 + c * 16 + 4 * g) : 0x7F7F7F7Fu;
+          static_for<4>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            const i32x8 a3 = mine ? x3_operand(row, c, q, g) : i32x8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+            for (int grp = 0; grp < G; ++grp) acc[0][grp] = mfma_f8f4<q, q>(a3, b[grp][q], acc[0][grp], (int)s3, (int)sb[grp]);
+          });
+        }
+      }
+    }
+  }
+
+#pragma unroll
+  for (int tt = 0; tt < T; ++tt)
+#pragma unroll
+    for (int grp = 0; grp < G; ++grp)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) part[wave][tt * 16 + 4 * g + v][grp * 16 + j] = acc[tt][grp][v];
+  __syncthreads();
+  if constexpr (MODE == kFwdGateUp) {
+    // one wave per column tile takes the sums back in the accumulators' layout for the epilogue
+    if (ks != 0 || !w[0].active) return;
+#pragma unroll
+    for (int grp = 0; grp < G; ++grp)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        float t = 0.f;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) t += part[wave + k][4 * g + v][grp * 16 + j];
+        acc[0][grp][v] = t;
+      }
+    const float tw[4] = {1.f, 1.f, 1.f, 1.f};
+    epilogue_direct<kFwdGateUp>(a, w[0], lane, acc[0], tw);
+  } else {
+    constexpr int kCols = kSub * 16 * G;  // of the work-group, a power of two
+    for (int o = threadIdx.x; o < T * 16 * kCols; o += 64 * kSplitWaves) {
+      const int r = o / kCols, cc = o % kCols, col = cb * kCols + cc;
+      const int tile = rgrp * T + r / 16, i = r % 16;
+      if (tile >= ntiles || col >= a.R) continue;
+      int row0, nrows;
+      if (T == 1) {
+        row0 = w[0].row0;
+        nrows = w[0].nrows;
+      } else {  // dense rows
+        row0 = tile * kFwdRowsPerTile;
+        nrows = a.M - row0;
+      }
+      if (i >= nrows) continue;
+      float t = 0.f;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) t += part[cc / (16 * G) * KS + k][r][cc % (16 * G)];
+      const int row = row0 + i;
+      a.y[(long long)(a.y_rows ? a.y_rows[row] : row) * a.ldy + col] = MODE == kFwdDown ? t * a.row_w[row] : t;
+    }
+  }
+}
+
 // Work-groups that fit on the device at once (two per CU: the LDS and register budgets of
 // fwd_kernel), rounded down to a multiple of the 8 XCDs.
 int resident_groups()
@@ -1124,11 +1328,38 @@ bool fast_path(int R, int K) { return K > 0 && (K % kChunk) == 0 && (long long)R
 
 bool fwd_bucket_split(int R, int K) { return fast_path(R, K); }
 
+// The split-K launch of a dense product: two row tiles (one when there is only one) and as many
+// columns per work-group as still leave at least kSplitMinGroups of them, since each item reads its
+// activations (2 bytes per element) and weights (0.53) from L2 again. Up to kSplitMaxTiles row
+// tiles: measured against fwd_kernel, quantisation included (us, M = 1 / 16 / 48 / 100 / 256):
+// [2048, 7168] 38 / 39 / 39 / 40 / 41 before, 13 / 13 / 16 / 20 / 27 here; [7168, 2048] 18 / 19 /
+// 19 / 21 / 30, 11 / 11 / 16 / 18 / 29; [7168, 7168] 38 / 39 / 40 / 43 / 76, 17 / 18 / 29 / 37 / 65;
+// the lines meet at about 400 rows.
+constexpr int kSplitMinGroups = 192;
+constexpr int kSplitMaxTiles = 16;
+static hipError_t launch_fwd_split_plain(const FwdArgs& a, hipStream_t s)
+{
+  const int tiles = (a.M + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
+  auto blocks = [&](int T, int cols) { return (long long)((tiles + T - 1) / T) * (((a.R + cols - 1) / cols + 7) / 8 * 8); };
+  const dim3 block(64 * kSplitWaves);
+#define MX_SPLIT(G, T, KS) \
+  hipLaunchKernelGGL((fwd_split_kernel<kFwdPlain, false, G, T, KS>), dim3((unsigned)blocks(T, 16 * G * (kSplitWaves / KS))), block, 0, s, a)
+  if (tiles > 1 && blocks(2, 128) >= kSplitMinGroups) MX_SPLIT(4, 2, 4);
+  else if (tiles > 1 && blocks(2, 64) >= kSplitMinGroups) MX_SPLIT(4, 2, 8);
+  else if (tiles > 1 && blocks(2, 32) >= kSplitMinGroups) MX_SPLIT(2, 2, 8);
+  else if (tiles > 1) MX_SPLIT(1, 2, 8);
+  else MX_SPLIT(1, 1, 8);
+#undef MX_SPLIT
+  return hipGetLastError();
+}
+
 hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s)
 {
   const long long n_cg = (a.n_ct + kWavesPerGroup - 1) / kWavesPerGroup;
   const long long total = (long long)max_tiles * n_cg;
   if (total <= 0) return hipSuccess;
+  if (mode == kFwdPlain && max_tiles <= kSplitMaxTiles && (long long)a.R * (a.K / 2) < (1LL << 32))
+    return launch_fwd_split_plain(a, s);
   const long long blocks = std::min<long long>((total + 7) / 8 * 8, resident_groups());
   // the down product from the forward layout: eight column tiles per work-group, one per CU
   const long long n_cg8 = (a.n_ct + 7) / 8;
@@ -1184,10 +1415,7 @@ hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s)
   return hipGetLastError();
 }
 
-long long forward_layout_bytes(int R, int K)
-{
-  return (long long)((R + 15) / 16) * (K / kChunk) * (4096 + 256);
-}
+long long forward_layout_bytes(int R, int K) { return forward_layout_size(R, K); }
 
 namespace {
 
