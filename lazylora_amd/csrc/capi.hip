@@ -401,7 +401,7 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
   // large buckets also in the AT layout, which the grouped work-groups re-read for every column
   // tile, and the XT rows are skipped when no bucket is small (the routing's meta says so on
   // the device). Without the split every tile reads the XT rows, so they are always written.
-  const bool gu_split = mx::fwd_bucket_split(F, D);
+  const bool gu_split = mx::fwd_bucket_split(F, D) && !mx::fwd_few_rows((int)P, F / 32, F, D);
   MX_TRY(mx::launch_quant_rows(h, h_dtype == MXFP4_BF16, D, N, D, gu_split ? at<int>(ws, L.meta) : nullptr,
                                at<uint8_t>(ws, L.xt_x), at<uint8_t>(ws, L.x3_x), at<int>(ws, L.meta) + 6, s),
          "quantise h");
@@ -429,7 +429,7 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
   a.x3_row_bytes = mx::x3_row_bytes(D);
   a.x3_any = at<int>(ws, L.meta) + 6;
   a.row_token = at<int>(ws, L.pair_token);
-  a.tiles = at<int4>(ws, L.tiles); a.n_tiles = at<int>(ws, L.meta);
+  a.tiles = at<int4>(ws, L.tiles); a.n_tiles = at<int>(ws, L.meta); a.M = (int)P;
   a.n_ct = F / 32;
   a.q_tiles = at<uint8_t>(ws, L.at_act);
   set_buckets(a, ws, L);
@@ -713,7 +713,7 @@ int mxfp4_moe_forward_fl(float* out, const void* h, int h_dtype, const void* top
   a.ws_estride = (long long)F * D / 32;
   a.R = D; a.K = F;
   a.a_tiles = at<uint8_t>(workspace, L.at_act);
-  a.tiles = at<int4>(workspace, L.tiles); a.n_tiles = at<int>(workspace, L.meta);
+  a.tiles = at<int4>(workspace, L.tiles); a.n_tiles = at<int>(workspace, L.meta); a.M = N * k;
   a.n_ct = (D + mx::kFwdColsPerTile - 1) / mx::kFwdColsPerTile;
   a.y = at<float>(workspace, L.ypair); a.ldy = D;
   // top-1 routing without LoRA: each token has at most one row, which the down product writes

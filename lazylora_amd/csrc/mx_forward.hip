@@ -1123,7 +1123,7 @@ __host__ __device__ inline long long forward_layout_size(int R, int K)
 }
 
 template <int MODE, bool FL, int G, int T, int KS>
-__global__ __launch_bounds__(64 * kSplitWaves) void fwd_split_kernel(FwdArgs a)
+__global__ __launch_bounds__(64 * kSplitWaves, 2) void fwd_split_kernel(FwdArgs a)
 {
   static_assert(kSplitWaves % KS == 0 && (MODE == kFwdPlain || (G == 4 && T == 1)), "routed items are one-tile, 64 columns");
   constexpr int kSub = kSplitWaves / KS;  // column sub-tiles per work-group
@@ -1207,6 +1207,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void fwd_split_kernel(FwdArgs a)
         }
       }
     }
+    __builtin_amdgcn_sched_barrier(0);  // the weights, which come from farthest, first
     i32x8 ah[T][4], al[T][4];
     uint2 s2[T];
 #pragma unroll
@@ -1328,6 +1329,31 @@ bool fast_path(int R, int K) { return K > 0 && (K % kChunk) == 0 && (long long)R
 
 bool fwd_bucket_split(int R, int K) { return fast_path(R, K); }
 
+bool fwd_few_rows(int rows, int n_ct, int R, int K)
+{
+  return (long long)rows * ((n_ct + 7) / 8) <= 128 && (long long)R * (K / 2) < (1LL << 32);
+}
+
+// The split-K launch of a routed product: one tile (at most one per row) x 64 weight rows per item
+static hipError_t launch_fwd_split_routed(const FwdArgs& a, int mode, int max_tiles, bool fl, hipStream_t s)
+{
+  const long long tiles = std::min(a.M, max_tiles);
+  auto blocks = [&](int sub) { return dim3((unsigned)(tiles * (((a.n_ct + sub - 1) / sub + 7) / 8 * 8))); };
+  const dim3 block(64 * kSplitWaves);
+#define MX_SPLIT(M, KS) \
+  do { \
+    if (fl) hipLaunchKernelGGL((fwd_split_kernel<M, true, 4, 1, KS>), blocks(kSplitWaves / KS), block, 0, s, a); \
+    else hipLaunchKernelGGL((fwd_split_kernel<M, false, 4, 1, KS>), blocks(kSplitWaves / KS), block, 0, s, a); \
+  } while (0)
+  // up to four super-chunks: half the waves take another column tile
+  if (mode == kFwdGateUp && at_nchunks(a.K) <= 4) MX_SPLIT(kFwdGateUp, 4);
+  else if (mode == kFwdGateUp) MX_SPLIT(kFwdGateUp, 8);
+  else if (at_nchunks(a.K) <= 4) MX_SPLIT(kFwdDown, 4);
+  else MX_SPLIT(kFwdDown, 8);
+#undef MX_SPLIT
+  return hipGetLastError();
+}
+
 // The split-K launch of a dense product: two row tiles (one when there is only one) and as many
 // columns per work-group as still leave at least kSplitMinGroups of them, since each item reads its
 // activations (2 bytes per element) and weights (0.53) from L2 again. Up to kSplitMaxTiles row
@@ -1379,6 +1405,7 @@ hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s)
                   forward_layout_bytes(a.R, a.K) < (1LL << 32);
   // both bucket kinds in one launch: eight-wave one-tile items and wide large-bucket items
   const bool fused = fl && a.n_ct % 8 == 0 && split;
+  if (a.tiles && fwd_few_rows(a.M, a.n_ct, a.R, a.K)) return launch_fwd_split_routed(a, mode, max_tiles, fl, s);
   dim3 grid((unsigned)blocks), block(64 * kWavesPerGroup);
 #define MX_LAUNCH(M, F, L) hipLaunchKernelGGL((fwd_kernel<M, F, L>), grid, block, 0, s, b)
   if (mode == kFwdPlain) {

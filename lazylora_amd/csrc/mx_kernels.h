@@ -33,7 +33,7 @@ struct FwdArgs {
   // work: tiles[t] = {expert, first row, row count <= 16, 1 in a large bucket}; null = dense, rows 16t.. of M
   const int4* tiles;
   const int* n_tiles;
-  int M;
+  int M;  // rows: all of them, or with a tile list at most
   int n_ct;  // column tiles per row tile
   // outputs
   float* y;
@@ -148,6 +148,14 @@ constexpr int kBwdColsPerTile = 256;  // output columns of one transposed-produc
 // resource addressing the whole matrix). Without the split every tile takes the one-tile
 // work-groups, whose gate/up product reads the token-major (XT) rows of x for every tile.
 bool fwd_bucket_split(int R, int K);
+// Whether a routed product of at most `rows` pair rows (so at most as many tiles) over W [R, K] runs
+// as split-K items of one tile x 64 weight rows, whatever its buckets: while its eight-column-tile
+// items (rows * ceil(n_ct / 8) of them at most) would leave half of the 256 CUs without one. Its
+// gate/up product then reads the token-major (XT) rows of x for every tile. Measured (us, gate/up
+// and down of 7168 / 2048 experts, one token's 8 experts, then two tokens' 16): forward layout 51 +
+// 20 -> 30 + 15, 57 + 26 -> 56 + 28; checkpoint layout 43 + 19 -> 32 + 18, 53 + 32 -> 65 + 34: the
+// line lies between one and two tokens.
+bool fwd_few_rows(int rows, int n_ct, int R, int K);
 hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s);
 hipError_t launch_bwd(const BwdArgs& a, int mode, int max_tiles, hipStream_t s);
 
