@@ -200,7 +200,7 @@ struct MoeLayout {
   int max_tiles, n_ct_bwd;
 };
 
-MoeLayout moe_layout(int N, int k, int E, int D, int F)
+MoeLayout make_moe_layout(int N, int k, int E, int D, int F)
 {
   MoeLayout L;
   const long long P = (long long)N * k;
@@ -239,6 +239,21 @@ MoeLayout moe_layout(int N, int k, int E, int D, int F)
   L.l_part = o; o = align_up(o + sizeof(float) * lora_part_floats(N, P, D, F));
   L.end = o;
   return L;
+}
+
+// The layout of a call. A pure function of the five sizes that plans the LoRA passes of every rank
+// (7 us), and a step asks for it five times (the size for its caller, twice, and both directions):
+// the calling thread's last one is kept.
+const MoeLayout& moe_layout(int N, int k, int E, int D, int F)
+{
+  thread_local int key[5] = {-1, -1, -1, -1, -1};
+  thread_local MoeLayout last;
+  const int want[5] = {N, k, E, D, F};
+  if (memcmp(key, want, sizeof(key)) != 0) {
+    last = make_moe_layout(N, k, E, D, F);
+    memcpy(key, want, sizeof(key));
+  }
+  return last;
 }
 
 template <typename T>
