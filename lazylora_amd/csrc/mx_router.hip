@@ -13,15 +13,37 @@ namespace mx {
 
 namespace {
 
-// (value, index) pair order for the selection: NaN first (torch.topk ranks NaN above every
-// number), then the larger value, then the lower index.
-__device__ __forceinline__ bool beats(float v, int i, float bv, int bi)
+// The choice values as whole numbers in selection order: NaN first (torch.topk ranks NaN above every
+// number), then the larger value; 0 stands for "not selectable" (below every float's key). A choice
+// is never -0 (a score is at least +0), so equal values have equal keys.
+__device__ __forceinline__ uint32_t order_key(float v)
 {
-  const bool vn = v != v, bn = bv != bv;
-  if (vn != bn) return vn;
-  return (vn || v == bv) ? i < bi : v > bv;
+  const uint32_t u = f_bits(v);
+  return v != v ? 0xFFFFFFFFu : u & 0x80000000u ? ~u : u | 0x80000000u;
+}
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_umax(uint32_t v)
+{
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false));
+}
+// Largest key of the wave: a DPP butterfly within each row of 16 lanes, then the four rows' lanes.
+__device__ __forceinline__ uint32_t wave_max_key(uint32_t v)
+{
+  v = dpp_umax<kDppXor1>(v);
+  v = dpp_umax<kDppXor2>(v);
+  v = dpp_umax<kDppHalfMirror>(v);
+  v = dpp_umax<kDppMirror>(v);
+  const uint32_t a = __builtin_amdgcn_readlane((int)v, 0), b = __builtin_amdgcn_readlane((int)v, 16);
+  const uint32_t c = __builtin_amdgcn_readlane((int)v, 32), d = __builtin_amdgcn_readlane((int)v, 48);
+  return max(max(a, b), max(c, d));
 }
 
+// One wave per token, lane l holding experts l + 64 m. A selection round is bound by its serial
+// chain, not by data (1024 x 896 logits are 3.7 MB): the lanes' largest open keys meet in four DPP
+// steps and four lane reads, one ballot names the owner (a second one only if several lanes tie),
+// which retires the expert and hands over its score from a register. Rounds of twelve cross-lane
+// shuffles and a dependent load of the winner's logit took 49 us for 1024 tokens, top-16 of 896;
+// this form 14.
 template <int PER_LANE>
 __global__ __launch_bounds__(256) void router_topk_kernel(long long* __restrict__ topk_idx, float* __restrict__ topk_w,
                                                           const float* __restrict__ logits,
@@ -33,53 +55,63 @@ __global__ __launch_bounds__(256) void router_topk_kernel(long long* __restrict_
   if (token >= N) return;  // whole waves leave together
   const float* row = logits + (long long)token * E;
 
-  // this lane's experts e = lane + 64 m; `open` marks the ones still selectable (present and
-  // not yet chosen), so every round's winner is a real expert id whatever the scores hold
-  // (NaN, infinities) as long as top_k <= E, which the host checks
-  float choice[PER_LANE];
-  uint64_t open = 0;
+  float score[PER_LANE];
+  uint32_t key[PER_LANE];  // 0: absent or already chosen
+  uint32_t best = 0;
 #pragma unroll
   for (int m = 0; m < PER_LANE; ++m) {
     const int e = lane + 64 * m;
-    choice[m] = 0.f;
+    score[m] = e < E ? row[e] : 0.f;
+  }
+#pragma unroll
+  for (int m = 0; m < PER_LANE; ++m) {
+    const int e = lane + 64 * m;
+    key[m] = 0;
     if (e < E) {
-      const float s = 1.0f / (1.0f + expf(-row[e]));
-      choice[m] = bias ? s + bias[e] : s;
-      open |= 1ull << m;
+      score[m] = 1.0f / (1.0f + expf(-score[m]));
+      key[m] = order_key(bias ? score[m] + bias[e] : score[m]);
     }
+    best = max(best, key[m]);
   }
 
   float sum = 0.f;
   float mine = 0.f;  // lane t keeps the t-th chosen score
   int mine_idx = 0;
   for (int t = 0; t < top_k; ++t) {
-    float bv = -__builtin_inff();
-    int bi = 0x7fffffff;  // "none": loses to every open entry
+    const uint32_t win = wave_max_key(best);
+    // the lowest expert id among the open entries with this key: every lane's lowest m, then, if
+    // several lanes hold one, the lowest id
+    int mm = PER_LANE;
+    float s_mm = 0.f;
+#pragma unroll
+    for (int m = PER_LANE - 1; m >= 0; --m) {
+      const bool hit = key[m] == win;
+      mm = hit ? m : mm;
+      s_mm = hit ? score[m] : s_mm;
+    }
+    const uint64_t holders = __builtin_amdgcn_ballot_w64(best == win);
+    int owner = __builtin_ctzll(holders);
+    if (holders & (holders - 1)) {  // uniform, rare
+      int id = best == win ? lane + 64 * mm : 0x7fffffff;
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) id = min(id, __shfl_xor(id, off, 64));
+      owner = id & 63;
+    }
+    owner = __builtin_amdgcn_readfirstlane(owner);
+    const int e = owner + 64 * __builtin_amdgcn_readlane(mm, owner);
+    const float s = bits_f((uint32_t)__builtin_amdgcn_readlane((int)f_bits(s_mm), owner));  // the unbiased score
+    // the owner retires it
+    uint32_t nb = 0;
 #pragma unroll
     for (int m = 0; m < PER_LANE; ++m) {
-      const int e = lane + 64 * m;
-      if (((open >> m) & 1) && (bi == 0x7fffffff || beats(choice[m], e, bv, bi))) {
-        bv = choice[m];
-        bi = e;
-      }
+      key[m] = lane == owner && m == mm ? 0u : key[m];
+      nb = max(nb, key[m]);
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      const float ov = __shfl_xor(bv, off, 64);
-      const int oi = __shfl_xor(bi, off, 64);
-      if (oi != 0x7fffffff && (bi == 0x7fffffff || beats(ov, oi, bv, bi))) {
-        bv = ov;
-        bi = oi;
-      }
-    }
-    if (bi >= E) bi = 0;  // unreachable while top_k <= E; keeps the read below in bounds
-    // every lane now holds the winner; its owner retires it
-    if ((bi & 63) == lane) open &= ~(1ull << (bi >> 6));
-    const float s = 1.0f / (1.0f + expf(-row[bi]));  // the unbiased score
+    best = nb;
     sum += s;
     if (lane == t) {
       mine = s;
-      mine_idx = bi;
+      mine_idx = e;
     }
   }
   if (lane < top_k) {
@@ -140,13 +172,12 @@ __global__ __launch_bounds__(256) void router_topk_bwd_kernel(float* __restrict_
 #pragma unroll
   for (int m = 0; m < PER_LANE; ++m) out[m] = 0.f;
   for (int j = 0; j < top_k; ++j) {
-    const int ej = __shfl(e, j, 64);
-    const float vj = __shfl(val, j, 64);
-    if (ej >= 0 && (ej & 63) == lane) {
+    const int ej = __builtin_amdgcn_readlane(e, j);
+    const float vj = bits_f((uint32_t)__builtin_amdgcn_readlane((int)f_bits(val), j));
+    if (ej < 0) continue;  // uniform
 #pragma unroll
-      for (int m = 0; m < PER_LANE; ++m)
-        if (lane + 64 * m == ej) out[m] += vj;
-    }
+    for (int m = 0; m < PER_LANE; ++m)
+      if (lane + 64 * m == ej) out[m] += vj;
   }
   float* orow = grad_logits + (long long)token * E;
 #pragma unroll
