@@ -226,6 +226,49 @@ __global__ __launch_bounds__(256) void dequant_kernel(void* out, const uint8_t* 
   }
 }
 
+// The same values where out is 16-byte and packed 4-byte aligned: bound by the output's bytes, so the
+// lanes of a wave write neighbouring 16-byte pieces (8 bf16 or 4 fp32 elements each, whole lines per
+// store instruction; the kernel above writes 64 or 128 bytes per lane in 4- and 8-byte stores that
+// far apart). Codes and scales are flat in memory (K is a multiple of 32), so the row plays no part.
+// kDequantPieces pieces per thread, a block apart, with all their loads in flight. [7168, 2048] to
+// bf16: 13.4 -> 7.2 us.
+constexpr int kDequantPieces = 4;
+template <bool BF16>
+__global__ __launch_bounds__(256) void dequant_flat_kernel(i32x4* out, const uint8_t* packed, const uint8_t* scales,
+                                                           long long pieces)
+{
+  constexpr int kPer = BF16 ? 8 : 4;  // elements per piece
+  const long long p0 = (long long)blockIdx.x * (256 * kDequantPieces) + threadIdx.x;
+  uint32_t code[kDequantPieces], sc[kDequantPieces];
+#pragma unroll
+  for (int u = 0; u < kDequantPieces; ++u) {
+    const long long p = min(p0 + u * 256, pieces - 1);
+    code[u] = BF16 ? reinterpret_cast<const uint32_t*>(packed)[p] : reinterpret_cast<const uint16_t*>(packed)[p];
+    sc[u] = scales[p * kPer / kGroup];
+  }
+#pragma unroll
+  for (int u = 0; u < kDequantPieces; ++u) {
+    const long long p = p0 + u * 256;
+    if (p >= pieces) return;
+    uint32_t pr[kPer / 2];  // bf16 pairs, the even element in the low half
+    if (sc[u] >= 253u) {  // +-0 with the code's sign (bit 3 of each code)
+#pragma unroll
+      for (int n = 0; n < kPer / 2; ++n)
+        pr[n] = (((code[u] >> (8 * n)) & 8u) << 12) | (((code[u] >> (8 * n + 4)) & 8u) << 28);
+    } else {
+      const float scale = bits_f(sc[u] << 23);
+      static_for<kPer / 2>([&](auto nc) {
+        constexpr int n = decltype(nc)::value;
+        pr[n] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(code[u], scale, n));
+      });
+    }
+    if constexpr (BF16)
+      out[p] = i32x4{(int)pr[0], (int)pr[1], (int)pr[2], (int)pr[3]};
+    else
+      out[p] = i32x4{(int)(pr[0] << 16), (int)(pr[0] & 0xFFFF0000u), (int)(pr[1] << 16), (int)(pr[1] & 0xFFFF0000u)};
+  }
+}
+
 constexpr int kQuantResidentBlocks = 1536;  // resident grid of quant_tiles over the large buckets: six per CU
 
 // ---------------------------------------------------------------- routing
@@ -685,6 +728,15 @@ hipError_t launch_dequant(void* out, int out_bf16, const uint8_t* packed, const 
 {
   const long long blocks = (long long)R * (K / kGroup);
   if (blocks == 0) return hipSuccess;
+  if ((reinterpret_cast<uintptr_t>(out) & 15) == 0 && (reinterpret_cast<uintptr_t>(packed) & 3) == 0) {
+    const long long pieces = blocks * kGroup / (out_bf16 ? 8 : 4), per = 256 * kDequantPieces;
+    const dim3 fgrid((unsigned)((pieces + per - 1) / per)), fblock(256);
+    if (out_bf16)
+      hipLaunchKernelGGL(dequant_flat_kernel<true>, fgrid, fblock, 0, s, static_cast<i32x4*>(out), packed, scales, pieces);
+    else
+      hipLaunchKernelGGL(dequant_flat_kernel<false>, fgrid, fblock, 0, s, static_cast<i32x4*>(out), packed, scales, pieces);
+    return hipGetLastError();
+  }
   dim3 grid((unsigned)((blocks + 255) / 256)), block(256);
   if (out_bf16) hipLaunchKernelGGL(dequant_kernel<true>, grid, block, 0, s, out, packed, scales, K, R);
   else hipLaunchKernelGGL(dequant_kernel<false>, grid, block, 0, s, out, packed, scales, K, R);
