@@ -628,7 +628,6 @@ int mxfp4_gemm_t(float* y, const float* dy, const uint8_t* packed, const uint8_t
   const long long rp = pad32(R);
   uint16_t* hi = at<uint16_t>(workspace, 0);
   uint16_t* lo = at<uint16_t>(workspace, need / 2);
-  MX_TRY(mx::launch_split_bf16(dy, R, M, R, (int)rp, hi, lo, stream), "gemm_t: split dy");
   mx::BwdArgs a = {};
   a.wp0 = packed; a.ws0 = scales;
   a.nseg = 1; a.R = R; a.C = K;
@@ -636,6 +635,11 @@ int mxfp4_gemm_t(float* y, const float* dy, const uint8_t* packed, const uint8_t
   a.M = M;
   a.n_ct = (K + mx::kBwdColsPerTile - 1) / mx::kBwdColsPerTile;
   a.y = y; a.ldy = K; a.accumulate = 1;
+  if (M <= mx::kBwdFewRows) {
+    MX_TRY(mx::launch_bwd_few(a, dy, stream), "gemm_t: product");
+    return MXFP4_OK;
+  }
+  MX_TRY(mx::launch_split_bf16(dy, R, M, R, (int)rp, hi, lo, stream), "gemm_t: split dy");
   const int tiles = (M + mx::kFwdRowsPerTile - 1) / mx::kFwdRowsPerTile;
   MX_TRY(mx::launch_bwd(a, mx::kBwdPlain, tiles, stream), "gemm_t: product");
   return MXFP4_OK;

@@ -843,6 +843,142 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void bwd_wide_kernel(BwdArgs a)
   if (decode_work<1, kWideWaves>(a, (int)blockIdx.x, w)) bwd_item<MODE, 1, BL, kWideWaves>(a, w, abuf);
 }
 
+// ---------------------------------------------------------------- few rows
+// A dense product of few rows leaves the shapes above idle: 22 rows against W [3072, 3584] are 8
+// work-groups, each wave 96 steps in series (68 us for 6 MB). Here the eight waves of a work-group
+// share one item (T row tiles x 128 columns) and split the contraction: wave w takes the 32-row
+// steps w, w + 8, .. with the next one's loads in flight, and the partial sums meet in LDS, added in
+// wave order (fixed, so the results do not depend on timing). The gradient rows are read as they
+// are, fp32, and split into the bf16 hi and lo terms in registers (32 operations per step beside
+// 64 of decoding), which saves the launch and the pass that would write the terms. Lane (n, g)
+// holds columns 8n .. 8n + 7, its own dword of each of the rows 8g .. 8g + 7 (as bwd_group_item).
+constexpr int kFewWaves = 8;
+constexpr int kFewCols = 128;
+
+template <int T>
+__global__ __launch_bounds__(64 * kFewWaves, 2) void bwd_few_kernel(BwdArgs a, const float* x, int n_cb8)
+{
+  __shared__ f32x4 part[kFewWaves][16 * 32];  // one tile's partial rows per wave, pieces swizzled as in bwd_group_item
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  // column blocks are the fast index, padded to the 8 XCDs: the row groups of one run on one XCD
+  const int cb = (int)(blockIdx.x % (unsigned)n_cb8), t0 = (int)(blockIdx.x / (unsigned)n_cb8) * T;
+  if (cb * kFewCols >= a.C) return;  // the whole work-group
+  const int col = cb * kFewCols + 8 * n, colc = col < a.C ? col : 0;  // past C: never stored
+  const uint32_t wpitch = (uint32_t)a.C / 2, cbs = (uint32_t)a.C / kGroup;
+  // rows past R lie past the resources: zero weights
+  const rsrc_t W = make_rsrc(a.wp0, (uint32_t)a.R * wpitch), S = make_rsrc(a.ws0, (uint32_t)a.R * cbs);
+  const float* px[T];
+#pragma unroll
+  for (int tt = 0; tt < T; ++tt) px[tt] = x + (long long)min((t0 + tt) * 16 + n, a.M - 1) * a.R;
+
+  struct Step {
+    uint32_t w[8], s[8];
+    float v[T][8];
+  };
+  auto load = [&](int step, Step& r) {
+    const uint32_t row = (uint32_t)step * kStepRows + 8u * (uint32_t)g;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      r.w[q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(W, (int)((row + q) * wpitch + (uint32_t)colc / 2), 0, 2);
+      r.s[q] = buf8(S, (row + q) * cbs + (uint32_t)colc / kGroup);
+    }
+    const int k0 = step * kStepRows + 8 * g;
+    if ((step + 1) * kStepRows <= a.R) {  // uniform
+#pragma unroll
+      for (int tt = 0; tt < T; ++tt) __builtin_memcpy(r.v[tt], px[tt] + k0, 32);
+    } else {
+#pragma unroll
+      for (int tt = 0; tt < T; ++tt)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r.v[tt][e] = k0 + e < a.R ? px[tt][k0 + e] : 0.f;
+    }
+  };
+
+  f32x4 acc[T][8];
+#pragma unroll
+  for (int tt = 0; tt < T; ++tt)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[tt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](const Step& r) {
+    uint32_t wl[8];
+    float sf[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const bool dead = r.s[q] >= 253u;  // the row's block contributes zero
+      wl[q] = dead ? 0u : r.w[q];
+      sf[q] = bits_f((dead ? 127u : r.s[q]) << 23);
+    }
+    bf16x8 ah[T], al[T];
+#pragma unroll
+    for (int tt = 0; tt < T; ++tt) {
+      uint32_t h[4], l[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v0 = r.v[tt][2 * e], v1 = r.v[tt][2 * e + 1];
+        h[e] = pack_bf16(v0, v1);
+        l[e] = pack_bf16(v0 - bf16_lo(h[e]), v1 - bf16_hi(h[e]));
+      }
+      ah[tt] = __builtin_bit_cast(bf16x8, i32x4{(int)h[0], (int)h[1], (int)h[2], (int)h[3]});
+      al[tt] = __builtin_bit_cast(bf16x8, i32x4{(int)l[0], (int)l[1], (int)l[2], (int)l[3]});
+    }
+    static_for<4>([&](auto pc) {
+      constexpr int P = decltype(pc)::value;
+      bf16x8 b0, b1;
+      gdecode_pair<P>(wl, sf, b0, b1);
+#pragma unroll
+      for (int tt = 0; tt < T; ++tt) {
+        acc[tt][2 * P] = mfma_bf16(ah[tt], b0, acc[tt][2 * P]);
+        acc[tt][2 * P + 1] = mfma_bf16(ah[tt], b1, acc[tt][2 * P + 1]);
+      }
+#pragma unroll
+      for (int tt = 0; tt < T; ++tt) {
+        acc[tt][2 * P] = mfma_bf16(al[tt], b0, acc[tt][2 * P]);
+        acc[tt][2 * P + 1] = mfma_bf16(al[tt], b1, acc[tt][2 * P + 1]);
+      }
+    });
+  };
+
+  const int nsteps = (a.R + kStepRows - 1) / kStepRows;
+  if (wave < nsteps) {
+    Step r0, r1;
+    load(wave, r0);
+    for (int s = wave;; s += 2 * kFewWaves) {
+      const bool second = s + kFewWaves < nsteps, third = s + 2 * kFewWaves < nsteps;
+      if (second) load(s + kFewWaves, r1);
+      compute(r0);
+      if (!second) break;
+      if (third) load(s + 2 * kFewWaves, r0);
+      compute(r1);
+      if (!third) break;
+    }
+  }
+
+  const int orow = (int)threadIdx.x >> 5, oq = (int)threadIdx.x & 31;
+  static_assert(64 * kFewWaves == 16 * 32, "one 16-byte piece of a tile per thread");
+  static_for<T>([&](auto ttc) {
+    constexpr int tt = decltype(ttc)::value;
+    if (tt > 0) __syncthreads();  // the previous tile's pieces are read
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int c4 = 0; c4 < 2; ++c4)
+        part[wave][(4 * g + v) * 32 + 2 * n + (c4 ^ ((n >> 2) & 1))] =
+            f32x4{acc[tt][4 * c4][v], acc[tt][4 * c4 + 1][v], acc[tt][4 * c4 + 2][v], acc[tt][4 * c4 + 3][v]};
+    __syncthreads();
+    const int row = (t0 + tt) * 16 + orow, oc = cb * kFewCols + 4 * oq;
+    if (row < a.M && oc < a.C) {
+      f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < kFewWaves; ++w) o += part[w][orow * 32 + (oq ^ ((oq >> 3) & 1))];
+      f32x4* const dst = reinterpret_cast<f32x4*>(a.y + (long long)row * a.ldy + oc);
+      if (a.accumulate) o += *dst;
+      *dst = o;
+    }
+  });
+}
+
 int resident_groups(int per_cu)
 {
   int dev = 0, cus = 0;
@@ -898,6 +1034,26 @@ hipError_t launch_bwd(const BwdArgs& a, int mode, int max_tiles, hipStream_t s)
   if (e != hipSuccess || !wide) return e;
   dim3 wgrid((unsigned)((witems + 7) / 8 * 8)), wblock(64 * kWideWaves);
   hipLaunchKernelGGL((bwd_wide_kernel<kBwdDownT, true>), wgrid, wblock, 0, s, b);
+  return hipGetLastError();
+}
+
+// Two row tiles per item (each decoded operand used twice) as long as kFewMinGroups work-groups are
+// left; four spill. Measured against the split pass + bwd_kernel (us, M = 1 / 22 / 100 / 256):
+// W [2048, 7168] 46 / 50 / 52 / 54 -> 15 / 15 / 28 / 43, [3072, 3584] 66 / 71 / 72 / 74 -> 18 / 20 /
+// 20 / 38, [7168, 2048] 146 / 150 / 153 / 157 -> 39 / 41 / 39 / 42, [7168, 7168] 147 / 150 / 155 /
+// 159 -> 43 / 47 / 91 / 137; the lines meet between 256 and 512 rows.
+constexpr int kFewMinGroups = 256;
+hipError_t launch_bwd_few(const BwdArgs& a, const float* x, hipStream_t s)
+{
+  if (a.M <= 0 || a.C <= 0) return hipSuccess;
+  if (a.nseg != 1 || a.tiles || a.C % 32 || a.ldy % 4 || (long long)a.R * (a.C / 2) >= (1LL << 32)) return hipErrorInvalidValue;
+  const int tiles = (a.M + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
+  const int n_cb = (a.C + kFewCols - 1) / kFewCols, n_cb8 = (n_cb + 7) / 8 * 8;
+  auto groups = [&](int T) { return (long long)((tiles + T - 1) / T); };
+  const int T = groups(2) * n_cb >= kFewMinGroups ? 2 : 1;
+  const dim3 grid((unsigned)(groups(T) * n_cb8)), block(64 * kFewWaves);
+  if (T == 2) hipLaunchKernelGGL(bwd_few_kernel<2>, grid, block, 0, s, a, x, n_cb8);
+  else hipLaunchKernelGGL(bwd_few_kernel<1>, grid, block, 0, s, a, x, n_cb8);
   return hipGetLastError();
 }
 

@@ -158,6 +158,11 @@ bool fwd_bucket_split(int R, int K);
 bool fwd_few_rows(int rows, int n_ct, int R, int K);
 hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s);
 hipError_t launch_bwd(const BwdArgs& a, int mode, int max_tiles, hipStream_t s);
+// The dense transposed product (kBwdPlain) straight from the fp32 rows x [M, R] (4-byte aligned),
+// the contraction split over the waves of a work-group: for up to kBwdFewRows rows. a_hi, a_lo and
+// lda are not used.
+constexpr int kBwdFewRows = 256;
+hipError_t launch_bwd_few(const BwdArgs& a, const float* x, hipStream_t s);
 
 // Backward layout: a load-time copy of E stacked MXFP4 matrices [R, C] (codes [R, C/2], E8M0
 // scales [R, C/32]) for the one-tile transposed products. Per expert, blocks (32-row step st,
