@@ -192,7 +192,7 @@ size_t lora_part_floats(int N, long long P, int D, int F)
 // Routed-layer workspace: one layout for forward and backward so the backward can reuse
 // what the forward left behind.
 struct MoeLayout {
-  size_t meta, counts, offsets, cursor, tiles, small_tiles, groups, wgroups, pair_token, pair_w, pair_of;
+  size_t meta, counts, offsets, cursor, tiles, small_tiles, bsmall_tiles, groups, wgroups, pair_token, pair_w, pair_of;
   size_t at_x, xt_x, x3_x, at_act;
   size_t saved, ypair, g_hi, g_lo, d_hi, d_lo, gw_part;
   size_t l_u, l_delta, l_vsum, l_q, l_rq, l_dsum, l_part;  // LoRA (rank <= kLoraMaxRank)
@@ -213,6 +213,7 @@ MoeLayout make_moe_layout(int N, int k, int E, int D, int F)
   L.cursor = o; o = align_up(o + sizeof(int) * (size_t)E);
   L.tiles = o; o = align_up(o + sizeof(int4) * (size_t)L.max_tiles);
   L.small_tiles = o; o = align_up(o + sizeof(int) * (size_t)L.max_tiles);
+  L.bsmall_tiles = o; o = align_up(o + sizeof(int) * (size_t)L.max_tiles);
   L.groups = o; o = align_up(o + sizeof(int4) * (size_t)L.max_tiles);
   L.wgroups = o; o = align_up(o + sizeof(int4) * (size_t)L.max_tiles);
   L.pair_token = o; o = align_up(o + sizeof(int) * (size_t)P);
@@ -283,13 +284,16 @@ int check_moe_args(const void* h, int h_dtype, const void* idx, int idx_dtype, c
 template <typename Args>
 void set_buckets(Args& a, void* ws, const MoeLayout& L)
 {
-  a.small_tiles = at<int>(ws, L.small_tiles);
-  a.n_small = at<int>(ws, L.meta) + 2;
-  a.groups = at<int4>(ws, L.groups);
-  a.n_groups = at<int>(ws, L.meta) + 3;
   if constexpr (std::is_same<Args, mx::FwdArgs>::value) {
+    a.small_tiles = at<int>(ws, L.small_tiles);
+    a.n_small = at<int>(ws, L.meta) + 2;
     a.wgroups = at<int4>(ws, L.wgroups);
     a.n_wgroups = at<int>(ws, L.meta) + 4;
+  } else {
+    a.small_tiles = at<int>(ws, L.bsmall_tiles);
+    a.n_small = at<int>(ws, L.meta) + 7;
+    a.groups = at<int4>(ws, L.groups);
+    a.n_groups = at<int>(ws, L.meta) + 3;
   }
 }
 
@@ -405,9 +409,12 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
               const Lora& lo, void* ws, const MoeLayout& L, hipStream_t s)
 {
   const long long P = (long long)N * k;
+  const bool fewer = P >= (long long)mx::kFewerMinRows * E && (long long)D * F >= mx::kFewerMinWeights;
   MX_TRY(mx::launch_route(idx, idx_dtype == MXFP4_I64, w, N, k, E, at<int>(ws, L.counts), at<int>(ws, L.offsets),
                           at<int>(ws, L.cursor), at<int4>(ws, L.tiles), at<int>(ws, L.small_tiles),
-                          at<int4>(ws, L.groups), at<int4>(ws, L.wgroups), at<int>(ws, L.meta), at<int>(ws, L.pair_token),
+                          at<int>(ws, L.bsmall_tiles), at<int4>(ws, L.groups), at<int4>(ws, L.wgroups),
+                          at<int>(ws, L.meta), fewer ? mx::kWideMinTiles : mx::kLargeMinTiles,
+                          fewer ? mx::kGroupMinTiles : mx::kLargeMinTiles, at<int>(ws, L.pair_token),
                           at<float>(ws, L.pair_w), at<int>(ws, L.pair_of), s),
          "route");
   MX_PHASE("route", s);
@@ -422,9 +429,9 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
          "quantise h");
   if (gu_split) {
     MX_TRY(mx::launch_quant_tiles(h, h_dtype == MXFP4_BF16, D, N, D, at<int4>(ws, L.tiles), at<int>(ws, L.meta),
-                                  L.max_tiles, at<int>(ws, L.pair_token), 1, at<uint8_t>(ws, L.xt_x),
+                                  L.max_tiles, at<int>(ws, L.pair_token), at<uint8_t>(ws, L.xt_x),
                                   at<int>(ws, L.meta), at<uint8_t>(ws, L.at_x), at<uint8_t>(ws, L.x3_x),
-                                  at<int>(ws, L.meta) + 6, s, at<int4>(ws, L.groups), at<int>(ws, L.meta) + 3),
+                                  at<int>(ws, L.meta) + 6, s, at<int4>(ws, L.wgroups), at<int>(ws, L.meta) + 4),
            "quantise h tiles");
   }
   MX_PHASE("quant_h", s);
@@ -501,7 +508,7 @@ int gemm_into(float* y, const float* x, const uint8_t* packed, const uint8_t* sc
               uint8_t* tiles_dev, hipStream_t stream)
 {
   const int tiles = (M + mx::kFwdRowsPerTile - 1) / mx::kFwdRowsPerTile;
-  MX_TRY(mx::launch_quant_tiles(x, 0, K, M, K, nullptr, nullptr, tiles, nullptr, 0, nullptr, nullptr, tiles_dev,
+  MX_TRY(mx::launch_quant_tiles(x, 0, K, M, K, nullptr, nullptr, tiles, nullptr, nullptr, nullptr, tiles_dev,
                                 nullptr, nullptr, stream),
          "gemm: quantise x");
   mx::FwdArgs a = {};

@@ -1016,7 +1016,7 @@ hipError_t launch_bwd(const BwdArgs& a, int mode, int max_tiles, hipStream_t s)
   long long blocks = (total + 7) / 8 * 8;
   if (wide)  // bwd_kernel then runs only with fewer than kWideMinItems wide items: twice as many of its own
     blocks = (std::min<long long>(total, 2LL * kWideMinItems) + 7) / 8 * 8;
-  // groups come from experts with at least kGroupMinTiles tiles: at most one per 32 rows (two from 65)
+  // groups come from experts with more than two tiles: at most one per 32 rows (one from 33, two from 65)
   long long gblocks = 0;
   if (split) {
     const long long gtotal = (long long)(a.M / 32) * kGParts * ((a.C + kGCols - 1) / kGCols);

@@ -60,13 +60,13 @@ struct WorkItem {
 typedef const __attribute__((address_space(4))) int* cint_ptr;
 
 __device__ __forceinline__ bool decode_work(const int4* tiles, const int* n_tiles, const int* small_tiles,
-                                            const int* n_small, const int* n_groups, int M, int n_ct, int wave,
+                                            const int* n_small, const int* n_wgroups, int M, int n_ct, int wave,
                                             int it, WorkItem& w, int nw = kWavesPerGroup)
 {
   // The tile lists are written before this kernel and only read here: scalar loads through the
   // constant address space, which do not wait for this work-group's outstanding stores.
   // with no large-bucket groups the small-bucket list is every tile in order: skip it
-  const bool use_small = small_tiles && *(cint_ptr)n_groups > 0;
+  const bool use_small = small_tiles && *(cint_ptr)n_wgroups > 0;
   const int ntiles = use_small ? *(cint_ptr)n_small
                                : tiles ? *(cint_ptr)n_tiles : (M + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
   const int n_cg = (n_ct + nw - 1) / nw;
@@ -728,7 +728,7 @@ __global__ __launch_bounds__(64 * NW, NW == kWavesPerGroup ? 2 : 1) void fwd_ker
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: keeps control flow scalar
   WorkItem w;
-  for (int it = 0; decode_work(a.tiles, a.n_tiles, a.small_tiles, a.n_small, a.n_groups, a.M, a.n_ct, wave, it, w, NW); ++it) {
+  for (int it = 0; decode_work(a.tiles, a.n_tiles, a.small_tiles, a.n_small, a.n_wgroups, a.M, a.n_ct, wave, it, w, NW); ++it) {
     // the previous item's reads of LDS are complete before this item's copies land there;
     // its output stores drain while this item's first loads are in flight
     if (FAST && it > 0) __syncthreads();
@@ -1083,7 +1083,7 @@ __global__ __launch_bounds__(64 * kWgWaves, 1) void fwd_fused_kernel(FwdArgs a)
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   WorkItem w;
-  for (int it = 0; decode_work(a.tiles, a.n_tiles, a.small_tiles, a.n_small, a.n_groups, a.M, a.n_ct, wave, it, w, 8); ++it) {
+  for (int it = 0; decode_work(a.tiles, a.n_tiles, a.small_tiles, a.n_small, a.n_wgroups, a.M, a.n_ct, wave, it, w, 8); ++it) {
     if (it > 0) __syncthreads();
     int l = lane;
     asm volatile("" : "+v"(l));
@@ -1396,7 +1396,6 @@ hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s)
   FwdArgs b = a;
   if (!split) {
     b.small_tiles = nullptr;
-    b.groups = nullptr;
     b.wgroups = nullptr;
   }
   // both work-group shapes read the forward layout when every matrix of the product has one

@@ -58,10 +58,6 @@ struct FwdArgs {
   // group's row tiles. Null small_tiles: every tile takes the first shape.
   const int* small_tiles;
   const int* n_small;
-  const int4* groups;
-  const int* n_groups;
-  // The same large-bucket tiles as wide groups of up to kWideGroupTiles tiles, taken instead of
-  // `groups` by the forward's large-bucket work-groups.
   const int4* wgroups;
   const int* n_wgroups;
   int* wcounter;  // the wide-group launch's work queue: 2 ints, zero before the first launch (queue_next)
@@ -139,7 +135,16 @@ struct BwdArgs {
 constexpr int kFwdRowsPerTile = 16;
 constexpr int kGroupTiles = 4;     // row tiles of one large-bucket group
 constexpr int kWideGroupTiles = 8;  // row tiles of one wide group (the large-bucket forward)
-constexpr int kGroupMinTiles = 4;  // experts with at least this many tiles take the large-bucket path
+// Experts with at least this many tiles take the large-bucket path: usually four; where the
+// buckets average kFewerMinRows rows, two in the forward (a wide item of two tiles reads the weights
+// once and takes little longer than a one-tile item; with few such experts, as under uniform
+// routing of small batches, the extra items would only lengthen the launch's tail) and three in
+// the transposed products (whose items always compute four tiles). 128 tokens, top-16 of 64 experts
+// (32 rows on average, 3584 / 3072, checkpoint layout), four everywhere, then this: gate/up 0.33 ->
+// 0.24 ms, down 0.18 -> 0.13, W1 | W3 transposed 0.38 -> 0.29, W2 0.20 -> 0.20.
+constexpr int kLargeMinTiles = 4, kWideMinTiles = 2, kGroupMinTiles = 3;
+constexpr int kFewerMinRows = 12;
+constexpr long long kFewerMinWeights = 1 << 20;  // elements per matrix: below, both shapes are a launch's latency
 constexpr int kFwdColsPerTile = 64;  // kFwdPlain / kFwdDown; kFwdGateUp covers 32 features
 constexpr int kBwdColsPerTile = 256;  // output columns of one transposed-product wave
 
@@ -180,16 +185,15 @@ hipError_t launch_backward_layout(const uint8_t* packed, const uint8_t* scales, 
 // holds row tiles[t].y + i (through row_map when given: the token of a (token, slot) pair);
 // with tiles == null the tiles are dense: tile t holds rows 16t.. of `rows`. Unused slots get
 // zeros. max_tiles bounds the grid; the live tile count is read from n_tiles on the device.
-// large_only: only the tiles of large buckets (tiles[t].w != 0); the others are left untouched.
 // xt (with meta and row_map): the XT rows of x written by launch_quant_rows on the same stream;
 // when that call wrote them (meta says some bucket is small) the tiles are copied from them
 // instead of quantising x again (the same bytes). x3 (with row_map): where the tiles are quantised
 // from x, also the X3 rows of their tokens (launch_quant_rows writes them otherwise). x3_any
 // (with x3): set to non-zero when some block has a third term (it must be zero before the call).
-// groups (with large_only; n_groups on the device): the large buckets' tiles are found through
-// the routing's group list by a resident grid, instead of one work-group per tile and chunk.
+// groups (the routing's wide groups; n_groups on the device): only their tiles, found through the
+// list by a resident grid instead of one work-group per tile and chunk; the others are left untouched.
 hipError_t launch_quant_tiles(const void* x, int x_bf16, long long ldx, int rows, int K, const int4* tiles,
-                              const int* n_tiles, int max_tiles, const int* row_map, int large_only, const uint8_t* xt,
+                              const int* n_tiles, int max_tiles, const int* row_map, const uint8_t* xt,
                               const int* meta, uint8_t* out, uint8_t* x3, int* x3_any, hipStream_t s,
                               const int4* groups = nullptr, const int* n_groups = nullptr);
 // Rows 0 .. rows - 1 of x into the XT layout (xt_row_bytes(K) per row), followed by zero rows
@@ -203,16 +207,19 @@ hipError_t launch_split_bf16(const float* x, long long ldx, int rows, int K, int
                              uint16_t* lo, hipStream_t s);
 hipError_t launch_dequant(void* out, int out_bf16, const uint8_t* packed, const uint8_t* scales, int K, int R,
                           hipStream_t s);
-// Routing: per-expert counts, scan, the tile list (tiles[t] = {expert, first pair row, rows, large}),
-// the small-bucket tile indices, the large-bucket groups ({expert, first tile, tiles, 0}) of up to
-// kGroupTiles tiles and the same tiles again as wide groups of up to kWideGroupTiles (the full
-// ones first), meta = {tiles, flags (bit 0: an id outside [0, E)), small tiles, groups, wide
-// groups, full wide groups, third term present (set by the quantisers), -, then the work queues
-// (2 ints each) of the wide-group launches of the forward gate/up and down products, ...} (16
-// ints, all zeroed here), and the pair maps.
-hipError_t launch_route(const void* topk_idx, int idx64, const float* topk_w, int N, int k, int E,
-                        int* counts, int* offsets, int* cursor, int4* tiles, int* small_tiles, int4* groups,
-                        int4* wgroups, int* meta, int* pair_token, float* pair_w, int* pair_of, hipStream_t s);
+// Routing: per-expert counts, scan, the tile list (tiles[t] = {expert, first pair row, rows, 0}),
+// the forward's large buckets (experts with at least wide_min tiles) as wide groups of up to
+// kWideGroupTiles tiles ({expert, first tile, tiles, 0}, the full ones first) and its other tiles'
+// indices (small_tiles), the transposed products' large buckets (at least group_min tiles) as groups
+// of up to kGroupTiles and their other tiles' indices (bsmall_tiles), meta = {tiles, flags (bit 0:
+// an id outside [0, E)), small tiles (forward), groups, wide groups, full wide groups, third term
+// present (set by the quantisers), small tiles (transposed), then the work queues (2 ints each) of
+// the wide-group launches of the forward gate/up and down products, ...} (16 ints, all zeroed
+// here), and the pair maps.
+hipError_t launch_route(const void* topk_idx, int idx64, const float* topk_w, int N, int k, int E, int* counts,
+                        int* offsets, int* cursor, int4* tiles, int* small_tiles, int* bsmall_tiles, int4* groups,
+                        int4* wgroups, int* meta, int wide_min, int group_min, int* pair_token, float* pair_w,
+                        int* pair_of, hipStream_t s);
 hipError_t launch_combine(float* out, const float* ypair, long long ldy, const int* pair_of, int N, int k,
                           int D, hipStream_t s);
 // Top-1 routing (the down product writes token rows itself): zeros into the rows of tokens with no

@@ -41,7 +41,7 @@ MX_DEV void quant_tile_chunk(const void* x, long long ldx, int rows, int K, int 
   const int nsc = at_nchunks(K);
   const int i = threadIdx.x >> 4, l16 = threadIdx.x & 15;
   const long long cbase = (long long)c * kAtChunkBytes;  // at_*_off are tile-relative
-  if (xt && !(meta[2] == 0 && meta[3] > 0)) {
+  if (xt && !(meta[2] == 0 && meta[4] > 0)) {
     // The token-major rows are written (quant_rows_kernel runs before this kernel and quantises
     // each token's row with the same blocks, so they hold the same codes): tile unit u, lane
     // 16g + i is piece (u, g) of the row of slot i's token (the zero row `rows` for unused
@@ -111,7 +111,7 @@ MX_DEV void quant_tile_chunk(const void* x, long long ldx, int rows, int K, int 
 template <bool BF16>
 __global__ __launch_bounds__(256) void quant_tiles_kernel(const void* x, long long ldx, int rows, int K,
                                                           const int4* tiles, const int* n_tiles, const int* row_map,
-                                                          int large_only, const int4* groups, const int* n_groups,
+                                                          const int4* groups, const int* n_groups,
                                                           const uint8_t* xt, const int* meta, uint8_t* out,
                                                           uint8_t* x3, int* x3_any)
 {
@@ -120,9 +120,9 @@ __global__ __launch_bounds__(256) void quant_tiles_kernel(const void* x, long lo
   if (groups) {
     // the large buckets' tiles, by groups: a resident grid loops over (group, tile, super-chunk),
     // so a routing without large buckets costs one read of the group count per work-group
-    const int total = *n_groups * kGroupTiles * nsc;
+    const int total = *n_groups * kWideGroupTiles * nsc;
     for (int wi = blockIdx.x; wi < total; wi += gridDim.x) {
-      const int g = wi / (kGroupTiles * nsc), r = wi - g * (kGroupTiles * nsc);
+      const int g = wi / (kWideGroupTiles * nsc), r = wi - g * (kWideGroupTiles * nsc);
       const int ti = r / nsc, c = r - ti * nsc;
       const int4 gr = groups[g];
       if (ti >= gr.z) continue;  // uniform
@@ -139,7 +139,6 @@ __global__ __launch_bounds__(256) void quant_tiles_kernel(const void* x, long lo
   int row0, nrows;
   if (tiles) {
     const int4 tt = tiles[t];
-    if (large_only && tt.w == 0) return;  // the whole work-group: a small bucket's tile
     row0 = tt.y;
     nrows = tt.z;
   } else {
@@ -338,94 +337,118 @@ __global__ __launch_bounds__(256) void route_count_kernel(const void* idx, int i
   wave_bucket_add(counts, valid ? (int)raw : 0, valid);
 }
 
-// Single work-group: exclusive scan of counts and of per-expert tile counts, tile list. An
-// expert with at least kGroupMinTiles tiles (a large bucket) also gets its tiles listed as
-// groups of up to kGroupTiles consecutive tiles, and again as wide groups of up to
-// kWideGroupTiles: every full wide group first (expert order), then the experts' last, partial
-// ones, so that a work queue taking them in order hands out the largest items first. The other
-// experts' tile indices go to the small-bucket list. meta = {tiles, flags, small tiles, groups,
-// wide groups, full wide groups}. cursor[e] gets offsets[e] (cursor may be counts itself: each
-// expert's count is read before its cursor is written, by the same thread).
-__device__ __forceinline__ void route_scan(const int* counts, int E, int* offsets, int* cursor, int4* tiles,
-                                           int* small_tiles, int4* groups, int4* wgroups, int* meta, int* s_rows,
-                                           int* s_tiles, int* s_small, int* s_groups, int* s_wgroups, int* s_wpart)
+// Sum over the 16 lanes of a lane group, on DPP lane moves (as group16_sum).
+template <int CTRL>
+MX_DEV int dpp_add(int v)
 {
-  const int t = threadIdx.x;
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+}
+MX_DEV int group16_isum(int v)
+{
+  return dpp_add<kDppMirror>(dpp_add<kDppHalfMirror>(dpp_add<kDppXor2>(dpp_add<kDppXor1>(v))));
+}
+
+// Single work-group of 1024: exclusive scan of counts and of per-expert tile counts, tile list. An
+// expert with at least group_min tiles (a large bucket of the transposed products) also gets its
+// tiles listed as groups of up to kGroupTiles consecutive tiles, the others' tile indices go to
+// bsmall_tiles; an expert with at least wide_min tiles (a large bucket of the forward products)
+// gets wide groups of up to kWideGroupTiles: every full wide group first (expert order), then the
+// experts' last, partial ones, so that a work queue taking them in order hands out the largest
+// items first; the other experts' tile indices go to small_tiles. meta = {tiles, flags, small tiles
+// (forward), groups, wide groups, full wide groups, -, small tiles (transposed)}. cursor[e] gets
+// offsets[e] (cursor may be counts itself: each expert's count is read before its cursor is written,
+// by the same thread). The scan is within each wave by lane moves and across the 16 waves through
+// their totals: two barriers (one for 20 in LDS took 4 us of this latency-bound kernel's 20).
+// Returns the number of rows (pairs with an expert).
+constexpr int kScan = 7;  // rows, tiles, small (forward), groups, full wide groups, partial ones, small (transposed)
+struct RouteOut {
+  int* offsets;
+  int4* tiles;
+  int* small_tiles;
+  int* bsmall_tiles;
+  int4* groups;
+  int4* wgroups;
+  int* meta;
+  int wide_min, group_min;
+};
+__device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor, const RouteOut& o, int (*s_tot)[16])
+{
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int per = (E + 1023) / 1024;
   const int e0 = min(t * per, E), e1 = min(e0 + per, E);
-  int rows = 0, nt = 0, ns = 0, ng = 0, nw = 0, np = 0;  // nw: full wide groups, np: partial ones
+  int v[kScan] = {};
   for (int e = e0; e < e1; ++e) {
     const int et = (counts[e] + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
-    rows += counts[e];
-    nt += et;
-    if (et >= kGroupMinTiles) {
-      ng += (et + kGroupTiles - 1) / kGroupTiles;
-      nw += et / kWideGroupTiles;
-      np += et % kWideGroupTiles ? 1 : 0;
+    v[0] += counts[e];
+    v[1] += et;
+    if (et >= o.wide_min) {
+      v[4] += et / kWideGroupTiles;
+      v[5] += et % kWideGroupTiles ? 1 : 0;
     } else {
-      ns += et;
+      v[2] += et;
     }
+    if (et >= o.group_min) v[3] += (et + kGroupTiles - 1) / kGroupTiles;
+    else v[6] += et;
   }
-  s_rows[t] = rows;
-  s_tiles[t] = nt;
-  s_small[t] = ns;
-  s_groups[t] = ng;
-  s_wgroups[t] = nw;
-  s_wpart[t] = np;
+  int inc[kScan];  // inclusive sums
+#pragma unroll
+  for (int i = 0; i < kScan; ++i) inc[i] = v[i];
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1)
+#pragma unroll
+    for (int i = 0; i < kScan; ++i) {
+      const int u = __shfl_up(inc[i], d, 64);
+      inc[i] += lane >= d ? u : 0;
+    }
+  if (lane == 63)
+#pragma unroll
+    for (int i = 0; i < kScan; ++i) s_tot[i][wave] = inc[i];
   __syncthreads();
-  for (int d = 1; d < 1024; d <<= 1) {  // Hillis-Steele inclusive scans
-    const int a = t >= d ? s_rows[t - d] : 0;
-    const int b = t >= d ? s_tiles[t - d] : 0;
-    const int c = t >= d ? s_small[t - d] : 0;
-    const int g = t >= d ? s_groups[t - d] : 0;
-    const int w = t >= d ? s_wgroups[t - d] : 0;
-    const int v = t >= d ? s_wpart[t - d] : 0;
-    __syncthreads();
-    s_rows[t] += a;
-    s_tiles[t] += b;
-    s_small[t] += c;
-    s_groups[t] += g;
-    s_wgroups[t] += w;
-    s_wpart[t] += v;
-    __syncthreads();
+  int off[kScan], total[kScan];  // exclusive offsets and totals
+#pragma unroll
+  for (int i = 0; i < kScan; ++i) {
+    const int w = s_tot[i][lane & 15];
+    total[i] = group16_isum(w);
+    off[i] = group16_isum((lane & 15) < wave ? w : 0) + inc[i] - v[i];
   }
-  const int n_full = s_wgroups[1023];
-  int row_off = s_rows[t] - rows, tile_off = s_tiles[t] - nt, small_off = s_small[t] - ns, group_off = s_groups[t] - ng,
-      wgroup_off = s_wgroups[t] - nw, wpart_off = n_full + s_wpart[t] - np;
+  int row_off = off[0], tile_off = off[1], small_off = off[2], group_off = off[3], wgroup_off = off[4],
+      wpart_off = total[4] + off[5], bsmall_off = off[6];
   for (int e = e0; e < e1; ++e) {
     const int c = counts[e];
     const int et = (c + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
-    offsets[e] = row_off;
+    o.offsets[e] = row_off;
     cursor[e] = row_off;
-    if (et >= kGroupMinTiles) {
-      for (int g = 0; g < et; g += kGroupTiles) groups[group_off++] = make_int4(e, tile_off + g, min(kGroupTiles, et - g), 0);
+    if (et >= o.group_min)
+      for (int g = 0; g < et; g += kGroupTiles) o.groups[group_off++] = make_int4(e, tile_off + g, min(kGroupTiles, et - g), 0);
+    else
+      for (int m = 0; m < et; ++m) o.bsmall_tiles[bsmall_off++] = tile_off + m;
+    if (et >= o.wide_min) {
       for (int g = 0; g + kWideGroupTiles <= et; g += kWideGroupTiles)
-        wgroups[wgroup_off++] = make_int4(e, tile_off + g, kWideGroupTiles, 0);
+        o.wgroups[wgroup_off++] = make_int4(e, tile_off + g, kWideGroupTiles, 0);
       if (et % kWideGroupTiles)
-        wgroups[wpart_off++] = make_int4(e, tile_off + et / kWideGroupTiles * kWideGroupTiles, et % kWideGroupTiles, 0);
+        o.wgroups[wpart_off++] = make_int4(e, tile_off + et / kWideGroupTiles * kWideGroupTiles, et % kWideGroupTiles, 0);
     } else {
-      for (int m = 0; m < et; ++m) small_tiles[small_off++] = tile_off + m;
+      for (int m = 0; m < et; ++m) o.small_tiles[small_off++] = tile_off + m;
     }
-    for (int m = 0; m < c; m += kFwdRowsPerTile)
-      tiles[tile_off++] = make_int4(e, row_off + m, min(kFwdRowsPerTile, c - m), et >= kGroupMinTiles ? 1 : 0);
+    for (int m = 0; m < c; m += kFwdRowsPerTile) o.tiles[tile_off++] = make_int4(e, row_off + m, min(kFwdRowsPerTile, c - m), 0);
     row_off += c;
   }
   if (t == 1023) {
-    offsets[E] = s_rows[1023];
-    meta[0] = s_tiles[1023];
-    meta[2] = s_small[1023];
-    meta[3] = s_groups[1023];
-    meta[4] = s_wgroups[1023] + s_wpart[1023];
-    meta[5] = s_wgroups[1023];
+    o.offsets[E] = total[0];
+    o.meta[0] = total[1];
+    o.meta[2] = total[2];
+    o.meta[3] = total[3];
+    o.meta[4] = total[4] + total[5];
+    o.meta[5] = total[4];
+    o.meta[7] = total[6];
   }
+  return total[0];
 }
 
-__global__ __launch_bounds__(1024) void route_scan_kernel(const int* counts, int E, int* offsets, int* cursor,
-                                                          int4* tiles, int* small_tiles, int4* groups, int4* wgroups,
-                                                          int* meta)
+__global__ __launch_bounds__(1024) void route_scan_kernel(const int* counts, int E, int* cursor, RouteOut o)
 {
-  __shared__ int s[6][1024];
-  route_scan(counts, E, offsets, cursor, tiles, small_tiles, groups, wgroups, meta, s[0], s[1], s[2], s[3], s[4], s[5]);
+  __shared__ int s_tot[kScan][16];
+  route_scan(counts, E, cursor, o, s_tot);
 }
 
 // The whole routing in one work-group (P <= kRouteOneP pairs, E <= kRouteOneE experts): counts
@@ -440,11 +463,10 @@ constexpr int kRouteOneE = 8192;
 constexpr int kRouteStageP = 8192;
 
 __global__ __launch_bounds__(1024) void route_one_kernel(const void* idx, int idx64, const float* w, int P, int k,
-                                                         int E, int* counts, int* offsets, int4* tiles,
-                                                         int* small_tiles, int4* groups, int4* wgroups, int* meta,
-                                                         int* pair_token, float* pair_w, int* pair_of)
+                                                         int E, int* counts, RouteOut o, int* pair_token,
+                                                         float* pair_w, int* pair_of)
 {
-  __shared__ int s[6][1024];
+  __shared__ int s_tot[kScan][16];
   __shared__ int s_cnt[kRouteOneE];
   __shared__ int s_tok[kRouteStageP];
   __shared__ float s_w[kRouteStageP];
@@ -472,11 +494,11 @@ __global__ __launch_bounds__(1024) void route_one_kernel(const void* idx, int id
   }
   __syncthreads();
   for (int e = t; e < E; e += 1024) counts[e] = s_cnt[e];
-  // meta: the scan writes words 0 and 2..5; the flags word and words 6..15 (the products' flags
-  // and work-queue counters, which start at zero) are written here
-  if (t == 1) meta[1] = s_bad;
-  if (t >= 6 && t < 16) meta[t] = 0;
-  route_scan(s_cnt, E, offsets, s_cnt, tiles, small_tiles, groups, wgroups, meta, s[0], s[1], s[2], s[3], s[4], s[5]);
+  // meta: the scan writes words 0, 2..5 and 7; the flags word, word 6 and words 8..15 (the products'
+  // flags and work-queue counters, which start at zero) are written here
+  if (t == 1) o.meta[1] = s_bad;
+  if (t == 6 || (t >= 8 && t < 16)) o.meta[t] = 0;
+  const int placed = route_scan(s_cnt, E, s_cnt, o, s_tot);  // pairs with a valid expert id
   __syncthreads();
   for (int p0 = 0; p0 < P; p0 += 8 * 1024) {
     int raw[8];
@@ -509,7 +531,6 @@ __global__ __launch_bounds__(1024) void route_one_kernel(const void* idx, int id
   }
   if (stage) {
     __syncthreads();
-    const int placed = s[0][1023];  // the scan's total: pairs with a valid expert id
     for (int i = t; i < placed; i += 1024) {
       pair_token[i] = s_tok[i];
       pair_w[i] = s_w[i];
@@ -619,7 +640,7 @@ template <bool BF16>
 __global__ __launch_bounds__(256) void quant_rows_kernel(const void* x, long long ldx, int rows, int K,
                                                          const int* meta, uint8_t* out, uint8_t* x3, int* x3_any)
 {
-  if (meta && meta[2] == 0 && meta[3] > 0) return;  // the whole grid (quant_tiles writes X3 then)
+  if (meta && meta[2] == 0 && meta[4] > 0) return;  // the whole grid (quant_tiles writes X3 then)
   __shared__ __attribute__((aligned(16))) uint8_t chunk[16 * kXtChunkBytes];
   const int nsc = at_nchunks(K);
   const int rg = (int)(blockIdx.x / nsc), c = (int)(blockIdx.x - (long long)rg * nsc);
@@ -681,7 +702,7 @@ __global__ __launch_bounds__(256) void zero_kernel(uint32_t* p, long long n_word
 }  // namespace
 
 hipError_t launch_quant_tiles(const void* x, int x_bf16, long long ldx, int rows, int K, const int4* tiles,
-                              const int* n_tiles, int max_tiles, const int* row_map, int large_only, const uint8_t* xt,
+                              const int* n_tiles, int max_tiles, const int* row_map, const uint8_t* xt,
                               const int* meta, uint8_t* out, uint8_t* x3, int* x3_any, hipStream_t s,
                               const int4* groups, const int* n_groups)
 {
@@ -689,15 +710,15 @@ hipError_t launch_quant_tiles(const void* x, int x_bf16, long long ldx, int rows
   if (blocks == 0) return hipSuccess;
   if (xt && (!meta || !row_map || !tiles)) return hipErrorInvalidValue;
   if (x3 && (!row_map || !x3_any)) return hipErrorInvalidValue;
-  if (groups && (!large_only || !tiles || !n_groups)) return hipErrorInvalidValue;
+  if (groups && (!tiles || !n_groups)) return hipErrorInvalidValue;
   if (groups) blocks = std::min(blocks, (long long)kQuantResidentBlocks);  // a resident grid over the groups
   dim3 grid((unsigned)blocks), block(256);
   if (x_bf16)
     hipLaunchKernelGGL(quant_tiles_kernel<true>, grid, block, 0, s, x, ldx, rows, K, tiles, n_tiles, row_map,
-                       large_only, groups, n_groups, xt, meta, out, x3, x3_any);
+                       groups, n_groups, xt, meta, out, x3, x3_any);
   else
     hipLaunchKernelGGL(quant_tiles_kernel<false>, grid, block, 0, s, x, ldx, rows, K, tiles, n_tiles, row_map,
-                       large_only, groups, n_groups, xt, meta, out, x3, x3_any);
+                       groups, n_groups, xt, meta, out, x3, x3_any);
   return hipGetLastError();
 }
 
@@ -754,13 +775,15 @@ hipError_t launch_zero(void* p, size_t bytes, hipStream_t s)
 }
 
 hipError_t launch_route(const void* topk_idx, int idx64, const float* topk_w, int N, int k, int E, int* counts,
-                        int* offsets, int* cursor, int4* tiles, int* small_tiles, int4* groups, int4* wgroups,
-                        int* meta, int* pair_token, float* pair_w, int* pair_of, hipStream_t s)
+                        int* offsets, int* cursor, int4* tiles, int* small_tiles, int* bsmall_tiles, int4* groups,
+                        int4* wgroups, int* meta, int wide_min, int group_min, int* pair_token, float* pair_w,
+                        int* pair_of, hipStream_t s)
 {
   const int P = N * k;
+  const RouteOut o{offsets, tiles, small_tiles, bsmall_tiles, groups, wgroups, meta, wide_min, group_min};
   if (P <= kRouteOneP && E <= kRouteOneE) {
-    hipLaunchKernelGGL(route_one_kernel, dim3(1), dim3(1024), 0, s, topk_idx, idx64, topk_w, P, k, E, counts, offsets,
-                       tiles, small_tiles, groups, wgroups, meta, pair_token, pair_w, pair_of);
+    hipLaunchKernelGGL(route_one_kernel, dim3(1), dim3(1024), 0, s, topk_idx, idx64, topk_w, P, k, E, counts, o,
+                       pair_token, pair_w, pair_of);
     return hipGetLastError();
   }
   hipError_t e = launch_zero(counts, sizeof(int) * (size_t)E, s);
@@ -768,8 +791,7 @@ hipError_t launch_route(const void* topk_idx, int idx64, const float* topk_w, in
   e = launch_zero(meta, sizeof(int) * 16, s);
   if (e != hipSuccess) return e;
   if (P > 0) hipLaunchKernelGGL(route_count_kernel, dim3((P + 255) / 256), dim3(256), 0, s, topk_idx, idx64, P, E, counts, meta);
-  hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(1024), 0, s, counts, E, offsets, cursor, tiles, small_tiles,
-                     groups, wgroups, meta);
+  hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(1024), 0, s, counts, E, cursor, o);
   if (P > 0)
     hipLaunchKernelGGL(route_place_kernel, dim3((P + 255) / 256), dim3(256), 0, s, topk_idx, idx64, topk_w, P, k, E,
                        cursor, pair_token, pair_w, pair_of);
