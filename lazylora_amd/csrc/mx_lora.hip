@@ -707,46 +707,40 @@ MX_DEV void finish_coef(const FinishJob& J, int tb)
       scale[n] = J.scale[min(j[n] / J.r, 1)];
     }
     float val[4] = {0.f, 0.f, 0.f, 0.f};
-    if (J.pair_of && J.k <= 8) {
+    if (J.pair_of) {
 #pragma unroll 1
-      for (int n = 0; n < 4; ++n) {  // one value at a time, its slots' loads together
+      for (int n = 0; n < 4; ++n) {  // one value at a time, the loads of 8 of its slots together
         if (base + 256 * n + (int)threadIdx.x >= nv) break;
-        int p[8];
-        float wv[8], sum[8];
+#pragma unroll 1
+        for (int k0 = 0; k0 < J.k; k0 += 8) {
+          int p[8];
+          float wv[8], sum[8];
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-          p[s] = J.pair_of[t[n] * J.k + min(s, J.k - 1)];
-          wv[s] = J.topk_w ? J.topk_w[t[n] * J.k + min(s, J.k - 1)] : 1.0f;
-          sum[s] = 0.f;
+          for (int s = 0; s < 8; ++s) {
+            const long long ts = t[n] * J.k + min(k0 + s, J.k - 1);
+            p[s] = J.pair_of[ts];
+            wv[s] = J.topk_w ? J.topk_w[ts] : 1.0f;
+            sum[s] = 0.f;
+          }
+          for (int sl0 = 0; sl0 < J.count; sl0 += 4) {  // 4 slices of 8 slots per round of loads
+            float v[4][8];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+              for (int s = 0; s < 8; ++s)
+                if ((k0 + s < J.k) & (sl0 + u < J.count))  // uniform
+                  v[u][s] = J.partial[((long long)(sl0 + u) * J.prow + max(p[s], 0)) * J.m + j[n]];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+              for (int s = 0; s < 8; ++s)
+                if ((k0 + s < J.k) & (sl0 + u < J.count)) sum[s] += v[u][s];
+          }
+#pragma unroll
+          for (int s = 0; s < 8; ++s)  // a skipped slot adds +0, which leaves val (never -0) unchanged
+            val[n] += ((k0 + s < J.k) & (p[s] >= 0)) ? wv[s] * (scale[n] * sum[s]) : 0.f;
         }
-        for (int sl0 = 0; sl0 < J.count; sl0 += 4) {  // 4 slices of 8 slots per round of loads
-          float v[4][8];
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int s = 0; s < 8; ++s)
-              if ((s < J.k) & (sl0 + u < J.count))  // uniform
-                v[u][s] = J.partial[((long long)(sl0 + u) * J.prow + max(p[s], 0)) * J.m + j[n]];
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int s = 0; s < 8; ++s)
-              if ((s < J.k) & (sl0 + u < J.count)) sum[s] += v[u][s];
-        }
-#pragma unroll
-        for (int s = 0; s < 8; ++s)  // a skipped slot adds +0, which leaves val (never -0) unchanged
-          val[n] += ((s < J.k) & (p[s] >= 0)) ? wv[s] * (scale[n] * sum[s]) : 0.f;
       }
-    } else if (J.pair_of) {
-#pragma unroll
-      for (int n = 0; n < 4; ++n)
-        for (int s = 0; s < J.k; ++s) {
-          const int p = J.pair_of[t[n] * J.k + s];
-          float sum = 0.f;
-          for (int sl = 0; sl < J.count; ++sl) sum += J.partial[((long long)sl * J.prow + max(p, 0)) * J.m + j[n]];
-          const float wv = J.topk_w ? J.topk_w[t[n] * J.k + s] : 1.0f;
-          if (p >= 0) val[n] += wv * (scale[n] * sum);
-        }
     } else {
       float sum[4] = {0.f, 0.f, 0.f, 0.f};
       for (int s0 = 0; s0 < J.count; s0 += 8) {
@@ -970,9 +964,19 @@ MX_DEV void combine_store(const CombineArgs& a, const int p[2][8], const f32x4 v
 #pragma unroll
     for (int s = 0; s < 8; ++s)
       if (s < a.k && p[u][s] >= 0) acc += v[u][s];  // slots in order; a skipped slot adds nothing
-    for (int s = 8; s < a.k; ++s) {                 // more than 8 slots
-      const int pp = a.pair_of[(long long)(tb + min(tt, nt - 1)) * a.k + s];
-      if (pp >= 0) acc += *reinterpret_cast<const f32x4*>(a.rows + (long long)pp * a.ldy + cc);
+#pragma unroll 1
+    for (int s0 = 8; s0 < a.k; s0 += 8) {  // more than 8 slots: the loads of 8 at a time together
+      int pm[8];
+      f32x4 vm[8];
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        pm[s] = s0 + s < a.k ? a.pair_of[(long long)(tb + min(tt, nt - 1)) * a.k + s0 + s] : -1;
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        if (s0 + s < a.k) vm[s] = ldnt(reinterpret_cast<const f32x4*>(a.rows + (long long)max(pm[s], 0) * a.ldy + cc));
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        if (s0 + s < a.k && pm[s] >= 0) acc += vm[s];
     }
     acc += *reinterpret_cast<const f32x4*>(&term[min(tt, nt - 1) * kTermLd + 4 * lane]);
     if (tt < nt && c < a.D) *reinterpret_cast<f32x4*>(a.out + (long long)(tb + tt) * a.D + c) = acc;
