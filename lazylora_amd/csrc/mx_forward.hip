@@ -413,6 +413,112 @@ __device__ __forceinline__ void epilogue_direct(const FwdArgs& a, const WorkItem
 }
 
 
+// Orders this wave's LDS writes before its later LDS reads (and the other way round): the lanes of
+// one wave exchange data through LDS without a work-group barrier.
+__device__ __forceinline__ void wave_lds_fence()
+{
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Epilogue of one wave's tile through 8 KiB of LDS of its own (st; no work-group barrier): the same
+// results as epilogue_direct, written as 16-byte pieces that cover 128- or 256-byte runs instead of
+// single bytes and dwords (16 and 16 store instructions for a tile's act codes and gate | up, 16 for
+// its down rows; here 1, 4 and 4).
+constexpr int kWavePitch = 64 + 4;  // floats per staged row
+template <int MODE>
+__device__ __forceinline__ void epilogue_wave(const FwdArgs& a, const WorkItem& w, int lane, const f32x4 (&acc)[4],
+                                              const float (&tw)[4], uint8_t* st)
+{
+  const int j = lane & 15, g = lane >> 4;
+  float* const sf = reinterpret_cast<float*>(st);  // [16 rows][kWavePitch]
+  if (MODE == kFwdGateUp) {
+    const int F = a.R, f0 = w.ct * 32;
+    uint8_t* const sq = st + 16 * kWavePitch * 4;  // codes [plane][half][row][16 B], then scales [plane][row]
+    float dl[4][4] = {};  // LoRA gate/up delta of each row's token
+    if (a.lora_delta) {
+      int tok[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) tok[v] = a.row_token[w.row0 + min(4 * g + v, w.nrows - 1)];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float* d = a.lora_delta + (long long)tok[v] * 2 * F + f0 + j;
+        const bool row = 4 * g + v < w.nrows;  // unused slots keep their zeros
+        dl[v][0] = row ? d[0] : 0.f;
+        dl[v][1] = row ? d[16] : 0.f;
+        dl[v][2] = row ? d[F] : 0.f;
+        dl[v][3] = row ? d[F + 16] : 0.f;
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = 4 * g + v;
+      const float ga = acc[0][v] + dl[v][0], gb = acc[1][v] + dl[v][1], ua = acc[2][v] + dl[v][2], ub = acc[3][v] + dl[v][3];
+      const Quant2 q = quant2_block16(glu_fwd(ga, ua, a.act_kind), glu_fwd(gb, ub, a.act_kind));
+      sq[(0 * 2 + 0) * 256 + i * 16 + j] = (uint8_t)q.hi;
+      sq[(0 * 2 + 1) * 256 + i * 16 + j] = (uint8_t)(q.hi >> 8);
+      sq[(1 * 2 + 0) * 256 + i * 16 + j] = (uint8_t)q.lo;
+      sq[(1 * 2 + 1) * 256 + i * 16 + j] = (uint8_t)(q.lo >> 8);
+      if (j == 0) {
+        sq[1024 + i] = (uint8_t)q.s_hi;
+        sq[1024 + 16 + i] = (uint8_t)q.s_lo;
+      }
+      if (a.save) {
+        float* r = sf + i * kWavePitch + j;
+        r[0] = ga;
+        r[16] = gb;
+        r[32] = ua;
+        r[48] = ub;
+      }
+    }
+    wave_lds_fence();
+    uint8_t* const qt = a.q_tiles + (long long)w.tile * at_tile_bytes(F);
+    {
+      const int plane = lane >> 5, half = (lane >> 4) & 1;
+      __builtin_nontemporal_store(*reinterpret_cast<const i32x4*>(sq + lane * 16),
+                                  reinterpret_cast<i32x4*>(qt + at_code_off(lane & 15, f0 + 16 * half, plane)));
+      if (lane < 32) qt[at_scale_off(lane & 15, f0, lane >> 4)] = sq[1024 + lane];
+    }
+    if (a.save) {
+      const int quad = lane & 15;
+      const long long at = quad < 8 ? f0 + 4 * quad : F + f0 + 4 * (quad - 8);
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int r = it * 4 + (lane >> 4);
+        if (r < w.nrows)
+          __builtin_nontemporal_store(*reinterpret_cast<const f32x4*>(sf + r * kWavePitch + 4 * quad),
+                                      reinterpret_cast<f32x4*>(a.save + (long long)(w.row0 + r) * 2 * F + at));
+      }
+    }
+    wave_lds_fence();  // read before the next tile is staged over it
+    return;
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const float wv = MODE == kFwdDown ? tw[v] : 1.0f;
+#pragma unroll
+    for (int grp = 0; grp < 4; ++grp) sf[(4 * g + v) * kWavePitch + grp * 16 + j] = acc[grp][v] * wv;
+  }
+  wave_lds_fence();
+  const bool vec = ((a.ldy & 3) == 0) && ((reinterpret_cast<uintptr_t>(a.y) & 15) == 0);
+  const int col = w.ct * kFwdColsPerTile + 4 * j;
+#pragma unroll
+  for (int it = 0; it < 4; ++it) {
+    const int r = it * 4 + g;
+    if (r >= w.nrows) continue;
+    const f32x4 val = *reinterpret_cast<const f32x4*>(sf + r * kWavePitch + 4 * j);
+    float* yr = a.y + (long long)(a.y_rows ? a.y_rows[w.row0 + r] : w.row0 + r) * a.ldy;
+    if (vec && col + 4 <= a.R) {
+      __builtin_nontemporal_store(val, reinterpret_cast<f32x4*>(yr + col));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (col + e < a.R) yr[col + e] = val[e];
+    }
+  }
+  wave_lds_fence();
+}
+
 // One work item: the 16 x 64 tile (w.tile, w.ct) over all of K, then its epilogue.
 // FL: the weights come from the forward layout (fl0 / fl1), one 1 KiB block per load instruction
 // NW waves per work-group (column tiles per item): 4, or 8 for the routed products from the
@@ -1013,6 +1119,7 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
     step(c, std::integral_constant<int, 3>{}, b1, false);
   }
   wait_vm0();
+  __syncthreads();  // every wave is done with the activations: their LDS stages the epilogues
   if (!active) return;
 #pragma unroll
   for (int tt = 0; tt < T; ++tt) {
@@ -1030,7 +1137,7 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
     if (MODE == kFwdDown)
 #pragma unroll
       for (int v = 0; v < 4; ++v) tw[v] = a.row_w[w.row0 + min(4 * g + v, w.nrows - 1)];
-    epilogue_direct<MODE>(a, w, lane, acc[tt], tw);
+    epilogue_wave<MODE>(a, w, lane, acc[tt], tw, &lds.a[0][0] + wave * 8192);
   }
 }
 
