@@ -185,9 +185,9 @@ hipError_t launch_backward_layout(const uint8_t* packed, const uint8_t* scales, 
 // holds row tiles[t].y + i (through row_map when given: the token of a (token, slot) pair);
 // with tiles == null the tiles are dense: tile t holds rows 16t.. of `rows`. Unused slots get
 // zeros. max_tiles bounds the grid; the live tile count is read from n_tiles on the device.
-// xt (with meta and row_map): the XT rows of x written by launch_quant_rows on the same stream;
-// when that call wrote them (meta says some bucket is small) the tiles are copied from them
-// instead of quantising x again (the same bytes). x3 (with row_map): where the tiles are quantised
+// xt (with row_map): the XT rows of x written by launch_quant_rows on the same stream; when that
+// call wrote them (it got no meta, or meta says some bucket is small) the tiles are copied from
+// them instead of quantising x again (the same bytes). x3 (with row_map): where the tiles are quantised
 // from x, also the X3 rows of their tokens (launch_quant_rows writes them otherwise). x3_any
 // (with x3): set to non-zero when some block has a third term (it must be zero before the call).
 // groups (the routing's wide groups; n_groups on the device): only their tiles, found through the

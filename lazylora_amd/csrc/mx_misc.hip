@@ -41,7 +41,7 @@ MX_DEV void quant_tile_chunk(const void* x, long long ldx, int rows, int K, int 
   const int nsc = at_nchunks(K);
   const int i = threadIdx.x >> 4, l16 = threadIdx.x & 15;
   const long long cbase = (long long)c * kAtChunkBytes;  // at_*_off are tile-relative
-  if (xt && !(meta[2] == 0 && meta[4] > 0)) {
+  if (xt && !(meta && meta[2] == 0 && meta[4] > 0)) {
     // The token-major rows are written (quant_rows_kernel runs before this kernel and quantises
     // each token's row with the same blocks, so they hold the same codes): tile unit u, lane
     // 16g + i is piece (u, g) of the row of slot i's token (the zero row `rows` for unused
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(const int* counts, int
 // order (contiguous stores) rather than scattered from the one CU.
 constexpr int kRouteOneP = 65536;
 constexpr int kRouteOneE = 8192;
-constexpr int kRouteStageP = 8192;
+constexpr int kRouteStageP = 16384;
 
 __global__ __launch_bounds__(1024) void route_one_kernel(const void* idx, int idx64, const float* w, int P, int k,
                                                          int E, int* counts, RouteOut o, int* pair_token,
@@ -468,7 +468,7 @@ __global__ __launch_bounds__(1024) void route_one_kernel(const void* idx, int id
 {
   __shared__ int s_tot[kScan][16];
   __shared__ int s_cnt[kRouteOneE];
-  __shared__ int s_tok[kRouteStageP];
+  __shared__ uint16_t s_tok[kRouteStageP];  // tokens fit: no more of them than pairs, at most 2^16
   __shared__ float s_w[kRouteStageP];
   __shared__ int s_bad;
   const int t = threadIdx.x;
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(1024) void route_one_kernel(const void* idx, int id
         continue;
       }
       if (stage) {
-        s_tok[pos] = p / k;
+        s_tok[pos] = (uint16_t)(p / k);
         s_w[pos] = wv[u];
       } else {
         pair_token[pos] = p / k;
@@ -704,7 +704,7 @@ hipError_t launch_quant_tiles(const void* x, int x_bf16, long long ldx, int rows
 {
   long long blocks = (long long)max_tiles * at_nchunks(K);  // (tile, super-chunk) work-groups
   if (blocks == 0) return hipSuccess;
-  if (xt && (!meta || !row_map || !tiles)) return hipErrorInvalidValue;
+  if (xt && (!row_map || !tiles)) return hipErrorInvalidValue;
   if (x3 && (!row_map || !x3_any)) return hipErrorInvalidValue;
   if (groups && (!tiles || !n_groups)) return hipErrorInvalidValue;
   if (groups) blocks = std::min(blocks, (long long)kQuantResidentBlocks);  // a resident grid over the groups
