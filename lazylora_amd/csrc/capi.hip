@@ -400,6 +400,17 @@ int check_forward_layout(const uint8_t* const* fl, int D, int F, int flags)
   return MXFP4_OK;
 }
 
+// Whether the buckets of a routed call are large from fewer tiles on (kFewerMinRows), and whether every
+// bucket of its forward is one.
+bool moe_fewer(long long P, int E, int D, int F)
+{
+  return P >= (long long)mx::kFewerMinRows * E && (long long)D * F >= mx::kFewerMinWeights;
+}
+bool moe_all_wide(long long P, int E, int D, int F, const uint8_t* const* fl)
+{
+  return moe_fewer(P, E, D, F) && !(fl && (fl[0] || fl[2]));
+}
+
 // Routing + quantised x + gate/up (+GLU) into the workspace. With LoRA also the per-token
 // adapter inputs U = [A_gate x | A_up x], their gate/up deltas (added in the product's
 // epilogue) and V = sum over a token's slots of w * A_down act; gate|up are then always saved,
@@ -409,11 +420,12 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
               const Lora& lo, void* ws, const MoeLayout& L, hipStream_t s)
 {
   const long long P = (long long)N * k;
-  const bool fewer = P >= (long long)mx::kFewerMinRows * E && (long long)D * F >= mx::kFewerMinWeights;
+  const bool fewer = moe_fewer(P, E, D, F);
+  const bool all_wide = moe_all_wide(P, E, D, F, fl);
   MX_TRY(mx::launch_route(idx, idx_dtype == MXFP4_I64, w, N, k, E, at<int>(ws, L.counts), at<int>(ws, L.offsets),
                           at<int>(ws, L.cursor), at<int4>(ws, L.tiles), at<int>(ws, L.small_tiles),
                           at<int>(ws, L.bsmall_tiles), at<int4>(ws, L.groups), at<int4>(ws, L.wgroups),
-                          at<int>(ws, L.meta), fewer ? mx::kWideMinTiles : mx::kLargeMinTiles,
+                          at<int>(ws, L.meta), all_wide ? 1 : fewer ? mx::kWideMinTiles : mx::kLargeMinTiles,
                           fewer ? mx::kGroupMinTiles : mx::kLargeMinTiles, at<int>(ws, L.pair_token),
                           at<float>(ws, L.pair_w), at<int>(ws, L.pair_of), s),
          "route");
@@ -455,6 +467,7 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
   a.x3_any = at<int>(ws, L.meta) + 6;
   a.row_token = at<int>(ws, L.pair_token);
   a.tiles = at<int4>(ws, L.tiles); a.n_tiles = at<int>(ws, L.meta); a.M = (int)P;
+  a.all_wide = all_wide;
   a.n_ct = F / 32;
   a.q_tiles = at<uint8_t>(ws, L.at_act);
   set_buckets(a, ws, L);
@@ -743,6 +756,7 @@ int mxfp4_moe_forward_fl(float* out, const void* h, int h_dtype, const void* top
   a.R = D; a.K = F;
   a.a_tiles = at<uint8_t>(workspace, L.at_act);
   a.tiles = at<int4>(workspace, L.tiles); a.n_tiles = at<int>(workspace, L.meta); a.M = N * k;
+  a.all_wide = moe_all_wide((long long)N * k, E, D, F, fwd_layout);
   a.n_ct = (D + mx::kFwdColsPerTile - 1) / mx::kFwdColsPerTile;
   a.y = at<float>(workspace, L.ypair); a.ldy = D;
   // top-1 routing without LoRA: each token has at most one row, which the down product writes

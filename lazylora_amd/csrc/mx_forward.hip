@@ -1512,10 +1512,13 @@ hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s)
   // both bucket kinds in one launch: eight-wave one-tile items and wide large-bucket items
   const bool fused = fl && a.n_ct % 8 == 0 && split;
   if (a.tiles && fwd_few_rows(a.M, a.n_ct, a.R, a.K)) return launch_fwd_split_routed(a, mode, max_tiles, fl, s);
+  const bool only_wide = split && a.all_wide;
   dim3 grid((unsigned)blocks), block(64 * kWavesPerGroup);
 #define MX_LAUNCH(M, F, L) hipLaunchKernelGGL((fwd_kernel<M, F, L>), grid, block, 0, s, b)
   if (mode == kFwdPlain) {
     if (fast) MX_LAUNCH(kFwdPlain, true, false); else MX_LAUNCH(kFwdPlain, false, false);
+  } else if (only_wide) {
+    // every tile is in a wide group: only the launch below
   } else if (fused) {
     if (mode == kFwdGateUp) hipLaunchKernelGGL((fwd_fused_kernel<kFwdGateUp>), dim3((unsigned)blocks8), dim3(512), 0, s, b);
     else hipLaunchKernelGGL((fwd_fused_kernel<kFwdDown>), dim3((unsigned)blocks8), dim3(512), 0, s, b);

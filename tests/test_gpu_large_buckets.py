@@ -49,3 +49,40 @@ def test_bucket_sizes(k, D, F, inputs, forward_layout):
     for e, n in enumerate(ROWS):  # no bucket hides in the others
         rows = idx[:, 0] == e
         assert_close(got[rows], want[rows], f"expert with {n} rows")
+
+
+@pytest.mark.parametrize("pairs_over_line", (0, -3))
+@pytest.mark.parametrize("D,F", ((1024, 1056), (1056, 1024), (1536, 1024)))
+@pytest.mark.parametrize("rank", (0, 8))
+def test_no_one_tile_items(k, D, F, rank, pairs_over_line):
+    """Top-3, on both sides of the 12 rows per expert from which a forward from the checkpoint layout
+    gives every bucket wide items (some of one row, one of none), and where only one of the two products
+    has them (the other's K is no multiple of 512)."""
+    import types
+
+    from lazylora_amd.experts import ExpertLayer
+    print(f"\n[case] D {D} F {F} rank {rank} pairs over the line {pairs_over_line}", flush=True)
+    rng = np.random.default_rng(D + F + rank)
+    E, topk = 7, 3
+    N = (12 * E + pairs_over_line) // topk
+    ex = oracle.random_experts(rng, E, D, F, 117, 121)
+    h, g = (rng.standard_normal((N, D)).astype(np.float32) for _ in range(2))
+    idx = np.stack([np.array([0, 1 + t % 2, 3]) for t in range(N)])  # two buckets of N rows, two of N / 2
+    idx[0], idx[1, 1] = [4, 5, 1], 5                                  # one row, two rows; expert 6 has none
+    w = rng.uniform(0.2, 1.0, (N, topk)).astype(np.float32)
+    lo = adapters = None
+    if rank:
+        A = lambda n_in, n_out: (0.05 * rng.standard_normal((rank, n_in)).astype(np.float32),
+                                 0.05 * rng.standard_normal((n_out, rank)).astype(np.float32))
+        parts = A(D, F), A(D, F), A(F, D)
+        lo = oracle.LoRA(*[v for p in parts for v in p])
+        adapters = tuple(types.SimpleNamespace(lora_A=torch.from_numpy(a).cuda(), lora_B=torch.from_numpy(b).cuda(),
+                                               scaling=2.0, dropout_rate=0.0) for a, b in parts)
+    L = ExpertLayer(*[torch.from_numpy(a).cuda() for a in (ex.w1p, ex.w1s, ex.w3p, ex.w3s, ex.w2p, ex.w2s)])
+    c = lambda a: torch.from_numpy(a).cuda()
+    out = k.routed_forward(c(h), c(idx), c(w), L, lora=adapters)
+    got = k.routed_backward(c(h), c(idx), c(w), L, c(g), lora=adapters)
+    assert_close(out.cpu().numpy(), oracle.routed_forward(h, idx, w, ex, lora=lo), "out")
+    want = oracle.routed_backward(h, idx, w, ex, g, lora=lo)
+    for name, a, b in zip(("grad_h", "grad_w"), got, want):
+        assert_close(a.cpu().numpy(), b, name)
