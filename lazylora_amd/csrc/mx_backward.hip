@@ -105,8 +105,6 @@ __device__ __forceinline__ bool decode_work(const BwdArgs& a, int bid, WorkItem<
   return true;
 }
 
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
 // 8 bytes, streaming (non-temporal): weight bytes are read exactly once per wave, and the 16
 // lanes of a row group consume whole 128-byte lines
 MX_DEV u32x2 buf8B_nt(rsrc_t r, uint32_t off)

@@ -27,6 +27,7 @@
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -159,7 +160,6 @@ MX_DEV float group16_sum(float v)
 struct Quant2 {
   uint32_t hi, lo;
   uint32_t s_hi, s_lo;
-  float amax;  // the block's max |x|
 };
 MX_DEV Quant2 quant2_block16(float v0, float v1)
 {
@@ -186,7 +186,70 @@ MX_DEV Quant2 quant2_block16(float v0, float v1)
   r.lo = ql;
   r.s_hi = (uint32_t)sb;
   r.s_lo = (uint32_t)sl;
-  r.amax = amax;
+  return r;
+}
+
+// The same quantisation of a block held 8 consecutive values per lane over the 4 lanes of a quad
+// (the quantisers of x, which are bound by these instructions more than by their bytes: the maxima
+// and scales cost each lane about the same whatever it holds, so 8 values share what 2 would pay).
+// The same codes and scales as quant2_block16. Codes as 8 bytes, the first element lowest.
+struct Quant2x8 {
+  uint32_t hi[2], lo[2];
+  uint32_t s_hi, s_lo;
+  float amax;
+};
+MX_DEV float quad_max(float v)
+{
+  v = fmaxf(v, dpp_lane<kDppXor1>(v));
+  return fmaxf(v, dpp_lane<kDppXor2>(v));
+}
+MX_DEV float abs_max8(const float (&v)[8])
+{
+  const float a = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fabsf(v[2])), b = fmaxf(fmaxf(fabsf(v[3]), fabsf(v[4])), fabsf(v[5]));
+  return fmaxf(fmaxf(a, b), fmaxf(fabsf(v[6]), fabsf(v[7])));
+}
+// 8 values times m as e4m3 bytes
+MX_DEV void fp8x8(const float (&v)[8], float m, uint32_t (&q)[2])
+{
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    int w = __builtin_amdgcn_cvt_pk_fp8_f32(v[4 * h] * m, v[4 * h + 1] * m, 0, false);
+    q[h] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(v[4 * h + 2] * m, v[4 * h + 3] * m, w, true);
+  }
+}
+// d -= s times the values of 8 e4m3 bytes
+MX_DEV void sub_fp8x8(float (&d)[8], const uint32_t (&q)[2], float s)
+{
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    d[4 * h] -= __builtin_amdgcn_cvt_f32_fp8((int)q[h], 0) * s;
+    d[4 * h + 1] -= __builtin_amdgcn_cvt_f32_fp8((int)q[h], 1) * s;
+    d[4 * h + 2] -= __builtin_amdgcn_cvt_f32_fp8((int)q[h], 2) * s;
+    d[4 * h + 3] -= __builtin_amdgcn_cvt_f32_fp8((int)q[h], 3) * s;
+  }
+}
+MX_DEV Quant2x8 quant2_block4(const float (&v)[8])
+{
+  Quant2x8 r;
+  r.amax = quad_max(abs_max8(v));
+  const int eb = (int)((f_bits(r.amax) >> 23) & 0xFF);
+  const int sb = eb > 7 ? eb - 7 : 0;
+  const float inv = bits_f((uint32_t)(254 - sb) << 23);  // 2^(127 - sb)
+  fp8x8(v, inv, r.hi);
+  float d[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) d[e] = v[e] * inv;
+  sub_fp8x8(d, r.hi, 1.0f);
+  const int ed = (int)((f_bits(quad_max(abs_max8(d))) >> 23) & 0xFF);
+  int sl = 127;
+  r.lo[0] = r.lo[1] = 0u;
+  if (ed >= 27) {  // residual above 2^-100 of the hi scale: worth a second term
+    const int t = sb + ed - 134;
+    sl = t > 0 ? t : 0;
+    fp8x8(d, bits_f((uint32_t)(127 + sb - sl) << 23), r.lo);  // 2^(sb - sl)
+  }
+  r.s_hi = (uint32_t)sb;
+  r.s_lo = (uint32_t)sl;
   return r;
 }
 
@@ -196,36 +259,37 @@ MX_DEV Quant2 quant2_block16(float v0, float v1)
 // (up to 2^-8 relative) then shows undiluted in that token's outputs. Such blocks are flagged and
 // get a third term: the residual after hi + lo, quantised again with its own scale (~12 bits for
 // the maximum). For every other block the third term is zero and its flag is clear.
-// Returns the third term's bytes (element 2n | 2n+1 << 8 of the lane), its scale byte and the flag
-// (the same on all 16 lanes of the block). q2 is the block's two-term result.
-struct Quant3 {
-  uint32_t th, s_th;
+// Returns the third term's bytes, its scale byte and the flag (the same on the block's 4 lanes).
+// q2 is the block's two-term result.
+struct Quant3x8 {
+  uint32_t th[2], s_th;
   bool flag;
 };
-MX_DEV Quant3 quant3_block16(float v0, float v1, const Quant2& q2)
+MX_DEV Quant3x8 quant3_block4(const float (&v)[8], const Quant2x8& q2)
 {
-  Quant3 r{0u, 127u, false};
+  Quant3x8 r{{0u, 0u}, 127u, false};
   // in the hi term's scaled domain (|y| < 256): the flag and the residual after hi + lo
   const float inv = bits_f((uint32_t)(254 - (int)q2.s_hi) << 23);  // 2^(127 - s_hi)
-  const float y0 = v0 * inv, y1 = v1 * inv;
+  float d[8], ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    d[e] = v[e] * inv;
+    ss = fmaf(d[e], d[e], ss);
+  }
+  ss += dpp_lane<kDppXor1>(ss);
+  ss += dpp_lane<kDppXor2>(ss);
   const float m = q2.amax * inv;
-  const float ss = group16_sum(y0 * y0 + y1 * y1);
   // max > 16 rms(rest) <=> 31 m^2 > 256 (ss - m^2) <=> 287 m^2 > 256 ss
   r.flag = 287.0f * m * m > 256.0f * ss;
   if (!r.flag) return r;
-  const float hi0 = __builtin_amdgcn_cvt_f32_fp8((int)q2.hi, 0), hi1 = __builtin_amdgcn_cvt_f32_fp8((int)q2.hi, 1);
-  // lo's codes scaled by 2^(s_hi - s_lo) in the hi domain
-  const float lsc = bits_f((uint32_t)(127 + (int)q2.s_lo - (int)q2.s_hi) << 23);
-  const float lo0 = __builtin_amdgcn_cvt_f32_fp8((int)q2.lo, 0) * lsc, lo1 = __builtin_amdgcn_cvt_f32_fp8((int)q2.lo, 1) * lsc;
-  const float d0 = (y0 - hi0) - lo0, d1 = (y1 - hi1) - lo1;
-  const float dmax = group16_max(fmaxf(fabsf(d0), fabsf(d1)));
-  const int ed = (int)((f_bits(dmax) >> 23) & 0xFF);
+  sub_fp8x8(d, q2.hi, 1.0f);
+  sub_fp8x8(d, q2.lo, bits_f((uint32_t)(127 + (int)q2.s_lo - (int)q2.s_hi) << 23));  // lo's codes in the hi domain
+  const int ed = (int)((f_bits(quad_max(abs_max8(d))) >> 23) & 0xFF);
   if (ed < 27) return r;  // nothing left worth a term (the block is exact in two terms)
   // scale 2^(t - 127) relative to x: the residual's maximum maps into [128, 256)
   const int t = (int)q2.s_hi + ed - 134;
   const int st = t > 0 ? t : 0;
-  const float mm = bits_f((uint32_t)(127 + (int)q2.s_hi - st) << 23);  // 2^(s_hi - st)
-  r.th = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(d0 * mm, d1 * mm, 0, false) & 0xFFFFu;
+  fp8x8(d, bits_f((uint32_t)(127 + (int)q2.s_hi - st) << 23), r.th);  // 2^(s_hi - st)
   r.s_th = (uint32_t)st;
   return r;
 }

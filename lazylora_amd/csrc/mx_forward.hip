@@ -115,7 +115,7 @@ __device__ __forceinline__ uint2 x3_flags(const FwdArgs& a, const uint8_t* row, 
   return uint2{*reinterpret_cast<const uint32_t*>(f + 4 * g), *reinterpret_cast<const uint32_t*>(f + 16 + 4 * g)};
 }
 // Bit c of the result (uniform): some row slot of the tile has a third term in super-chunk c
-// (quant3_block16); the lanes' flag bytes (x3_flags) OR-ed over the wave.
+// (quant3_block4); the lanes' flag bytes (x3_flags) OR-ed over the wave.
 __device__ __forceinline__ uint32_t x3_mask(uint2 d, int lane)
 {
   const int g = lane >> 4;
