@@ -1141,33 +1141,47 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
   }
 }
 
-// Resident grid (one eight-wave work-group per CU) over the items (wide group, block of eight
-// column tiles). Items vary in cost (a partial group has fewer tiles, and its MFMAs for the
+// The items (wide group, block of eight column tiles) of a resident grid of one eight-wave
+// work-group per CU. Items vary in cost (a partial group has fewer tiles, and its MFMAs for the
 // missing tiles are skipped), so the work-groups take them from a work counter in list order:
 // the full groups' items first, then the partial groups', which fill in behind them. Consecutive
 // items are the eight column blocks of one group, which run at about the same time and share its
-// activations.
+// activations. The items past the last whole round of the grid are cut into two or four runs of tiles
+// where that many work-groups per item would idle: a run of two of eight tiles reads the weights
+// again but takes about half the time (whole forward from the checkpoint layout, top-8, Zipf routing: 1024
+// pairs over 128 experts, 7168 / 2048, 535 -> 443 us; 512 over 64, 3584 / 3072, 312 -> 281; 256 rows to each
+// of 32 experts from the forward layout 701 -> 691).
+template <int MODE, bool FL>
+__device__ __forceinline__ void fwd_wide_items(const FwdArgs& a, int wave, int lane, WideLds& lds, int* s_item)
+{
+  const int ng = *(cint_ptr)a.n_wgroups;
+  if (ng == 0) return;  // no large buckets: the whole grid leaves without touching the queue
+  const int nfb = (a.n_ct + kWgWaves - 1) / kWgWaves;
+  const int total = ng * nfb, rem = total % (int)gridDim.x, whole = total - rem;
+  const int sh = rem * 4 <= (int)gridDim.x ? 2 : rem * 2 <= (int)gridDim.x ? 1 : 0;  // log2 of the runs
+  const int end = whole + (rem << sh);
+  for (;;) {
+    const int it = queue_next(a.wcounter, s_item);  // also: every wave is done with the LDS before
+    if (it >= end) break;
+    const int ish = it >= whole ? sh : 0, past = it - whole;
+    const int item = ish ? whole + (past >> ish) : it, part = ish ? past & ((1 << ish) - 1) : 0;
+    const int gi = item / nfb, fb = item - gi * nfb;
+    const cint_ptr gg = (cint_ptr)(a.wgroups + gi);
+    const int t0 = (gg[2] * part) >> ish, t1 = (gg[2] * (part + 1)) >> ish;
+    if (t0 == t1) continue;  // fewer tiles than runs
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    fwd_wide_item<MODE, FL>(a, gg[0], gg[1] + t0, t1 - t0, fb, wave, l, lds);
+  }
+  queue_leave(a.wcounter);
+}
+
 template <int MODE, bool FL>
 __global__ __launch_bounds__(64 * kWgWaves, 1) void fwd_wide_kernel(FwdArgs a)
 {
   __shared__ WideLds lds;
   __shared__ int s_item;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ng = *(cint_ptr)a.n_wgroups;
-  if (ng == 0) return;  // no large buckets: the whole grid leaves without touching the queue
-  const int nfb = (a.n_ct + kWgWaves - 1) / kWgWaves;
-  const int total = ng * nfb;
-  for (;;) {
-    const int item = queue_next(a.wcounter, &s_item);  // also: every wave is done with the previous item's LDS
-    if (item >= total) break;
-    const int gi = item / nfb, fb = item - gi * nfb;
-    const cint_ptr gg = (cint_ptr)(a.wgroups + gi);
-    int l = lane;
-    asm volatile("" : "+v"(l));
-    fwd_wide_item<MODE, FL>(a, gg[0], gg[1], gg[2], fb, wave, l, lds);
-  }
-  queue_leave(a.wcounter);
+  fwd_wide_items<MODE, FL>(a, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63, lds, &s_item);
 }
 
 // Both bucket kinds of a routed product from the forward layout in one launch of eight-wave
@@ -1196,20 +1210,7 @@ __global__ __launch_bounds__(64 * kWgWaves, 1) void fwd_fused_kernel(FwdArgs a)
     asm volatile("" : "+v"(l));
     fwd_item<MODE, true, true, 8>(a, w, wave, l, lds.f);
   }
-  const int ng = *(cint_ptr)a.n_wgroups;
-  if (ng == 0) return;  // no large buckets: the work queue is not touched
-  const int nfb = (a.n_ct + kWgWaves - 1) / kWgWaves;
-  const int total = ng * nfb;
-  for (;;) {
-    const int item = queue_next(a.wcounter, &s_item);  // also: every wave is done with the LDS before
-    if (item >= total) break;
-    const int gi = item / nfb, fb = item - gi * nfb;
-    const cint_ptr gg = (cint_ptr)(a.wgroups + gi);
-    int l = lane;
-    asm volatile("" : "+v"(l));
-    fwd_wide_item<MODE, true>(a, gg[0], gg[1], gg[2], fb, wave, l, lds.w);
-  }
-  queue_leave(a.wcounter);
+  fwd_wide_items<MODE, true>(a, wave, lane, lds.w, &s_item);
 }
 
 // ---------------------------------------------------------------- few work items
