@@ -1141,16 +1141,15 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
   }
 }
 
-// The items (wide group, block of eight column tiles) of a resident grid of one eight-wave
-// work-group per CU. Items vary in cost (a partial group has fewer tiles, and its MFMAs for the
-// missing tiles are skipped), so the work-groups take them from a work counter in list order:
-// the full groups' items first, then the partial groups', which fill in behind them. Consecutive
-// items are the eight column blocks of one group, which run at about the same time and share its
-// activations. The items past the last whole round of the grid are cut into two or four runs of tiles
-// where that many work-groups per item would idle: a run of two of eight tiles reads the weights
-// again but takes about half the time (whole forward from the checkpoint layout, top-8, Zipf routing: 1024
-// pairs over 128 experts, 7168 / 2048, 535 -> 443 us; 512 over 64, 3584 / 3072, 312 -> 281; 256 rows to each
-// of 32 experts from the forward layout 701 -> 691).
+// The items (wide group, block of eight column tiles) of a resident grid of one eight-wave work-group per
+// CU. Items vary in cost (a partial group has fewer tiles, and its MFMAs for the missing tiles are
+// skipped), so the work-groups take them from a work counter in list order: the full groups' items first,
+// then the partial groups', which fill in behind them. Consecutive items are the eight column blocks of one
+// group, which run at about the same time and share its activations. The items past the last whole round of
+// the grid are cut into two or four runs of tiles where that many work-groups per item would idle: a run of
+// two of eight tiles reads the weights again but takes about half the time (whole forward from the
+// checkpoint layout, top-8, Zipf routing: 1024 pairs over 128 experts, 7168 / 2048, 535 -> 443 us; 512 over
+// 64, 3584 / 3072, 312 -> 281; 256 rows to each of 32 experts from the forward layout 701 -> 691).
 template <int MODE, bool FL>
 __device__ __forceinline__ void fwd_wide_items(const FwdArgs& a, int wave, int lane, WideLds& lds, int* s_item)
 {

@@ -136,18 +136,18 @@ struct BwdArgs {
 constexpr int kFwdRowsPerTile = 16;
 constexpr int kGroupTiles = 4;     // row tiles of one large-bucket group
 constexpr int kWideGroupTiles = 8;  // row tiles of one wide group (the large-bucket forward)
-// Experts with at least this many tiles take the large-bucket path: usually four; where the
-// buckets average kFewerMinRows rows, two in the forward (a wide item of two tiles reads the weights
-// once and takes little longer than a one-tile item; with few such experts, as under uniform
-// routing of small batches, the extra items would only lengthen the launch's tail) and three in
-// the transposed products (whose items always compute four tiles). From the checkpoint layout the forward
-// then has no one-tile items at all: a launch of their own for the few short buckets costs more than
-// their wide items (3584 / 3072, 64 experts, top-8, whole forward, us, with them then without: 8 rows
-// per bucket 252 / 296, 12 rows 352 / 306, 20 rows 375 / 314, 64 rows 419 / 412; Zipf 20 rows 363 /
-// 349, 64 rows 538 / 506; 7168 / 2048, 128 experts, 16 rows 748 / 699). With a forward layout both kinds share
-// one launch, and the one-tile items stay (12 rows 233 / 239, Zipf 64 rows 430 / 440). 128 tokens, top-16 of 64 experts
-// (32 rows on average, 3584 / 3072, checkpoint layout), four everywhere, then this: gate/up 0.33 ->
-// 0.24 ms, down 0.18 -> 0.13, W1 | W3 transposed 0.38 -> 0.29, W2 0.20 -> 0.20.
+// Experts with at least this many tiles take the large-bucket path: usually four; where the buckets average
+// kFewerMinRows rows, two in the forward (a wide item of two tiles reads the weights once and takes little
+// longer than a one-tile item; with few such experts, as under uniform routing of small batches, the extra
+// items would only lengthen the launch's tail) and three in the transposed products (whose items always
+// compute four tiles). From the checkpoint layout the forward then has no one-tile items at all: a launch
+// of their own for the few short buckets costs more than their wide items (3584 / 3072, 64 experts, top-8,
+// whole forward, us, with them then without: 8 rows per bucket 252 / 296, 12 rows 352 / 306, 20 rows 375 /
+// 314, 64 rows 419 / 412; Zipf 20 rows 363 / 349, 64 rows 538 / 506; 7168 / 2048, 128 experts, 16 rows 748
+// / 699). With a forward layout both kinds share one launch, and the one-tile items stay (12 rows 233 /
+// 239, Zipf 64 rows 430 / 440). 128 tokens, top-16 of 64 experts (32 rows on average, 3584 / 3072,
+// checkpoint layout), four everywhere, then this: gate/up 0.33 -> 0.24 ms, down 0.18 -> 0.13, W1 | W3
+// transposed 0.38 -> 0.29, W2 0.20 -> 0.20.
 constexpr int kLargeMinTiles = 4, kWideMinTiles = 2, kGroupMinTiles = 3;
 constexpr int kFewerMinRows = 12;
 constexpr long long kFewerMinWeights = 1 << 20;  // elements per matrix: below, both shapes are a launch's latency

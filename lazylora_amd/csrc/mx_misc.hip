@@ -7,16 +7,15 @@ namespace mx {
 namespace {
 
 // ---------------------------------------------------------------- activation quantisation
-// One row's super-chunk c, quantised by the 16 lanes l16 of a lane group: quad l16 / 4 takes blocks
-// 4 it + l16 / 4 (it = 0..3), lane l16 % 4 of it 8 consecutive elements, so the loads of one step are
-// 512 contiguous bytes (fp32) per row. Rows that are not `valid` and positions past K give zeros.
-// put(plane, e, codes) stores 8 code bytes of the elements e .. e + 7 of the super-chunk, put_scale(plane,
-// e, byte) the scale of the block holding e. x3r (non-null): also the third term of the flagged blocks
-// (quant3_block4) into the row's X3 row: the codes and scales only when some block of the chunk is
-// flagged (readers use them only then), the chunk's flag byte always.
-// Eight values per lane share what the maxima and scales cost (2 per lane before): 256 rows to each of 32
-// experts (7168 fp32) 720 -> 702 us for the forward call, one token's 8 experts (bf16) 64.5 -> 60.1,
-// a product of 200 rows x 2048 27.9 -> 25.4.
+// One row's super-chunk c, quantised by the 16 lanes l16 of a lane group: quad l16 / 4 takes blocks 4 it +
+// l16 / 4 (it = 0..3), lane l16 % 4 of it 8 consecutive elements, so the loads of one step are 512
+// contiguous bytes (fp32) per row. Rows that are not `valid` and positions past K give zeros. put(plane, e,
+// codes) stores 8 code bytes of the elements e .. e + 7 of the super-chunk, put_scale(plane, e, byte) the
+// scale of the block holding e. x3r (non-null): also the third term of the flagged blocks (quant3_block4)
+// into the row's X3 row: the codes and scales only when some block of the chunk is flagged (readers use
+// them only then), the chunk's flag byte always. Eight values per lane share what the maxima and scales
+// cost (2 per lane before): 256 rows to each of 32 experts (7168 fp32) 720 -> 702 us for the forward call,
+// one token's 8 experts (bf16) 64.5 -> 60.1, a product of 200 rows x 2048 27.9 -> 25.4.
 constexpr int kQuantSteps = kChunkBlocks / 4;
 template <bool BF16, class Put, class PutScale>
 MX_DEV void quant_row_chunk(const void* x, long long at, int K, int c, bool valid, uint8_t* x3r, int* x3_any, Put put,
