@@ -297,9 +297,13 @@ constexpr int kQuantResidentBlocks = 1536;  // resident grid of quant_tiles over
 // The order of pairs inside a bucket is left to atomics; nothing downstream depends on it,
 // because every row of a product is computed independently and the combine gathers each
 // token's slots in slot order.
+// An expert id; one that 32 bits don't hold is as invalid as any other outside [0, E): -1, not its
+// low half, which may be some expert's id.
 __device__ __forceinline__ int read_idx(const void* idx, int idx64, long long p)
 {
-  return idx64 ? (int)reinterpret_cast<const long long*>(idx)[p] : reinterpret_cast<const int*>(idx)[p];
+  if (!idx64) return reinterpret_cast<const int*>(idx)[p];
+  const long long v = reinterpret_cast<const long long*>(idx)[p];
+  return v == (int)v ? (int)v : -1;
 }
 
 // counter[e] += 1 for every lane with `valid` set; returns the lane's slot (the counter's old value
@@ -353,10 +357,10 @@ __global__ __launch_bounds__(256) void route_count_kernel(const void* idx, int i
                                                           int* meta)
 {
   const int p = blockIdx.x * 256 + threadIdx.x;
-  const long long raw = p < P ? (idx64 ? reinterpret_cast<const long long*>(idx)[p] : reinterpret_cast<const int*>(idx)[p]) : 0;
+  const int raw = p < P ? read_idx(idx, idx64, p) : 0;
   const bool valid = p < P && raw >= 0 && raw < E;
   if (p < P && !valid) atomicOr(&meta[1], 1);
-  wave_bucket_add(counts, valid ? (int)raw : 0, valid);
+  wave_bucket_add(counts, valid ? raw : 0, valid);
 }
 
 // Sum over the 16 lanes of a lane group, on DPP lane moves (as group16_sum).
@@ -565,9 +569,9 @@ __global__ __launch_bounds__(256) void route_place_kernel(const void* idx, int i
                                                           int* pair_of)
 {
   const int p = blockIdx.x * 256 + threadIdx.x;
-  const long long raw = p < P ? (idx64 ? reinterpret_cast<const long long*>(idx)[p] : reinterpret_cast<const int*>(idx)[p]) : 0;
+  const int raw = p < P ? read_idx(idx, idx64, p) : 0;
   const bool valid = p < P && raw >= 0 && raw < E;
-  const int pos = wave_bucket_add(cursor, valid ? (int)raw : 0, valid);
+  const int pos = wave_bucket_add(cursor, valid ? raw : 0, valid);
   if (p >= P) return;
   if (!valid) {
     pair_of[p] = -1;

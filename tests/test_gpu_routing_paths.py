@@ -63,3 +63,30 @@ def test_multi_launch_routing(k, E, D, F, N, topk, zipf):
     assert_close(np.where(bad, 0.0, gwn), np.where(bad, 0.0, want[1]), "grad_w")
     del L
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("E,N,topk", ((16, 40, 4), (16, 9000, 8)))  # one work-group; several launches
+def test_ids_beyond_32_bits(k, E, N, topk):
+    """64-bit ids whose low 32 bits are an expert's id are outside the layer all the same."""
+    from lazylora_amd.experts import ExpertLayer
+    print(f"\n[case] ids beyond 32 bits, {N * topk} pairs", flush=True)
+    rng = np.random.default_rng(N)
+    D, F = 128, 96
+    ex = oracle.random_experts(rng, E, D, F, 118, 122)
+    L = ExpertLayer(*[torch.from_numpy(np.ascontiguousarray(a)).cuda()
+                      for a in (ex.w1p, ex.w1s, ex.w3p, ex.w3s, ex.w2p, ex.w2s)])
+    idx, w = oracle.softmax_topk(rng.standard_normal((N, E)).astype(np.float32), topk)
+    idx = idx.astype(np.int64)
+    far = idx.copy()
+    bad = rng.random(idx.shape) < 0.1
+    far[bad] += rng.choice([-2 ** 32, 2 ** 32, 3 * 2 ** 32, -2 ** 63], int(bad.sum()))
+    h = rng.standard_normal((N, D)).astype(np.float32)
+    H, I, W = (torch.from_numpy(a).cuda() for a in (h, far, w))
+    ws = torch.empty(k.moe_workspace_bytes(N, topk, E, D, F), dtype=torch.uint8, device="cuda")
+    out = k.routed_forward(H, I, W, L, workspace=ws)
+    assert k.route_status(ws) & 1
+    # the same rows as with an id that is plainly outside, bit for bit (each token's slots are added in order)
+    want = k.routed_forward(H, torch.from_numpy(np.where(bad, -1, idx)).cuda(), W, L)
+    assert torch.equal(out, want)
+    assert_close(out.cpu().numpy(), oracle.routed_forward(h, idx, np.where(bad, 0.0, w).astype(np.float32), ex, "swiglu"),
+                 "fwd")
