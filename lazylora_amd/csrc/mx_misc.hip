@@ -297,14 +297,22 @@ constexpr int kQuantResidentBlocks = 1536;  // resident grid of quant_tiles over
 // The order of pairs inside a bucket is left to atomics; nothing downstream depends on it,
 // because every row of a product is computed independently and the combine gathers each
 // token's slots in slot order.
-// An expert id; one that 32 bits don't hold is as invalid as any other outside [0, E): -1, not its
-// low half, which may be some expert's id.
-__device__ __forceinline__ int read_idx(const void* idx, int idx64, long long p)
+// An expert id as its 32-bit words (the same one twice for 32-bit ids), and its value: one that 32 bits
+// don't hold is as invalid as any other outside [0, E): -1, not its low half, which may be some
+// expert's id. Apart, so that a thread's loads are all issued before the first is looked at.
+struct IdWords {
+  int lo, hi;
+};
+__device__ __forceinline__ IdWords load_id(const void* idx, int idx64, int p)
 {
-  if (!idx64) return reinterpret_cast<const int*>(idx)[p];
-  const long long v = reinterpret_cast<const long long*>(idx)[p];
-  return v == (int)v ? (int)v : -1;
+  if (idx64) {  // uniform
+    const int2 v = reinterpret_cast<const int2*>(idx)[p];
+    return IdWords{v.x, v.y};
+  }
+  const int v = reinterpret_cast<const int*>(idx)[p];
+  return IdWords{v, v};
 }
+__device__ __forceinline__ int id_value(IdWords w, int idx64) { return !idx64 || w.hi == w.lo >> 31 ? w.lo : -1; }
 
 // counter[e] += 1 for every lane with `valid` set; returns the lane's slot (the counter's old value
 // plus the lane's rank among the wave's lanes with the same e). The lanes of the first
@@ -357,7 +365,7 @@ __global__ __launch_bounds__(256) void route_count_kernel(const void* idx, int i
                                                           int* meta)
 {
   const int p = blockIdx.x * 256 + threadIdx.x;
-  const int raw = p < P ? read_idx(idx, idx64, p) : 0;
+  const int raw = p < P ? id_value(load_id(idx, idx64, p), idx64) : 0;
   const bool valid = p < P && raw >= 0 && raw < E;
   if (p < P && !valid) atomicOr(&meta[1], 1);
   wave_bucket_add(counts, valid ? raw : 0, valid);
@@ -504,18 +512,19 @@ __global__ __launch_bounds__(1024) void route_one_kernel(const void* idx, int id
   __syncthreads();
   // 8 pairs per thread and round, their index loads all issued before the atomics
   for (int p0 = 0; p0 < P; p0 += 8 * 1024) {
-    int raw[8];
+    IdWords id[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < 8; ++u) {  // a wave without pairs loads nothing
       const int p = p0 + u * 1024 + t;
-      raw[u] = p < P ? read_idx(idx, idx64, p) : 0;
+      id[u] = p < P ? load_id(idx, idx64, p) : IdWords{0, 0};
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {  // wave-aggregated: pairs of one expert in a wave add once
+      const int raw = id_value(id[u], idx64);
       const bool in = p0 + u * 1024 + t < P;
-      const bool valid = in && raw[u] >= 0 && raw[u] < E;
+      const bool valid = in && raw >= 0 && raw < E;
       if (in && !valid) s_bad = 1;
-      lds_bucket_add(s_cnt, valid ? raw[u] : 0, valid);
+      lds_bucket_add(s_cnt, valid ? raw : 0, valid);
     }
   }
   __syncthreads();
@@ -527,19 +536,20 @@ __global__ __launch_bounds__(1024) void route_one_kernel(const void* idx, int id
   const int placed = route_scan(s_cnt, E, s_cnt, o, s_tot);  // pairs with a valid expert id
   __syncthreads();
   for (int p0 = 0; p0 < P; p0 += 8 * 1024) {
-    int raw[8];
+    IdWords id[8];
     float wv[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int p = min(p0 + u * 1024 + t, P - 1);
-      raw[u] = read_idx(idx, idx64, p);
-      wv[u] = w[p];
+      const int p = p0 + u * 1024 + t;
+      id[u] = p < P ? load_id(idx, idx64, p) : IdWords{0, 0};
+      wv[u] = p < P ? w[p] : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int p = p0 + u * 1024 + t;
-      const bool valid = p < P && raw[u] >= 0 && raw[u] < E;
-      const int pos = lds_bucket_add(s_cnt, valid ? raw[u] : 0, valid);
+      const int raw = id_value(id[u], idx64);
+      const bool valid = p < P && raw >= 0 && raw < E;
+      const int pos = lds_bucket_add(s_cnt, valid ? raw : 0, valid);
       if (p >= P) continue;
       if (!valid) {
         pair_of[p] = -1;
@@ -569,7 +579,7 @@ __global__ __launch_bounds__(256) void route_place_kernel(const void* idx, int i
                                                           int* pair_of)
 {
   const int p = blockIdx.x * 256 + threadIdx.x;
-  const int raw = p < P ? read_idx(idx, idx64, p) : 0;
+  const int raw = p < P ? id_value(load_id(idx, idx64, p), idx64) : 0;
   const bool valid = p < P && raw >= 0 && raw < E;
   const int pos = wave_bucket_add(cursor, valid ? raw : 0, valid);
   if (p >= P) return;
