@@ -430,29 +430,6 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
                           at<float>(ws, L.pair_w), at<int>(ws, L.pair_of), s),
          "route");
   MX_PHASE("route", s);
-  // h once per token in the XT layout (with a zero row N for the unused slots of a tile), which
-  // the one-tile work-groups gather; when the gate/up product splits its buckets, the tiles of
-  // large buckets also in the AT layout, which the grouped work-groups re-read for every column
-  // tile, and the XT rows are skipped when no bucket is small (the routing's meta says so on
-  // the device). Without the split every tile reads the XT rows, so they are always written.
-  const bool gu_split = mx::fwd_bucket_split(F, D) && !mx::fwd_few_rows((int)P, F / 32, F, D);
-  // Beyond top-1 they are written in any case: a token in several tiles is then quantised once and
-  // copied (1000 tokens in 16 tiles each: 97 us for its tiles, 46 with the rows).
-  const int* xt_meta = gu_split && k == 1 ? at<int>(ws, L.meta) : nullptr;
-  MX_TRY(mx::launch_quant_rows(h, h_dtype == MXFP4_BF16, D, N, D, xt_meta, at<uint8_t>(ws, L.xt_x),
-                               at<uint8_t>(ws, L.x3_x), at<int>(ws, L.meta) + 6, s),
-         "quantise h");
-  if (gu_split) {
-    MX_TRY(mx::launch_quant_tiles(h, h_dtype == MXFP4_BF16, D, N, D, at<int4>(ws, L.tiles), at<int>(ws, L.meta),
-                                  L.max_tiles, at<int>(ws, L.pair_token), at<uint8_t>(ws, L.xt_x),
-                                  xt_meta, at<uint8_t>(ws, L.at_x), at<uint8_t>(ws, L.x3_x),
-                                  at<int>(ws, L.meta) + 6, s, at<int4>(ws, L.wgroups), at<int>(ws, L.meta) + 4),
-           "quantise h tiles");
-  }
-  MX_PHASE("quant_h", s);
-  if (F % mx::kChunk) {  // padding blocks of the act buffer are read by the down product
-    MX_TRY(mx::launch_zero(at<void>(ws, L.at_act), at_bytes(L.max_tiles, F), s), "zero act");
-  }
   mx::FwdArgs a = {};
   a.wp0 = wts[0]; a.ws0 = wts[1]; a.wp1 = wts[2]; a.ws1 = wts[3];
   a.wp_estride = (long long)F * D / 2;
@@ -478,6 +455,29 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
   a.wcounter = at<int>(ws, L.meta) + 8;
   a.save = (save || lo.r) ? at<float>(ws, L.saved) : nullptr;
   a.act_kind = act_kind;
+  // h once per token in the XT layout (with a zero row N for the unused slots of a tile), which
+  // the one-tile work-groups gather; when the gate/up product splits its buckets, the tiles of
+  // large buckets also in the AT layout, which the grouped work-groups re-read for every column
+  // tile, and the XT rows are skipped when no bucket is small (the routing's meta says so on
+  // the device). Without the split every tile reads the XT rows, so they are always written.
+  const bool gu_split = mx::fwd_bucket_split(F, D) && !mx::fwd_few_rows(a, mx::kFwdGateUp, L.max_tiles);
+  // Beyond top-1 they are written in any case: a token in several tiles is then quantised once and
+  // copied (1000 tokens in 16 tiles each: 97 us for its tiles, 46 with the rows).
+  const int* xt_meta = gu_split && k == 1 ? at<int>(ws, L.meta) : nullptr;
+  MX_TRY(mx::launch_quant_rows(h, h_dtype == MXFP4_BF16, D, N, D, xt_meta, at<uint8_t>(ws, L.xt_x),
+                               at<uint8_t>(ws, L.x3_x), at<int>(ws, L.meta) + 6, s),
+         "quantise h");
+  if (gu_split) {
+    MX_TRY(mx::launch_quant_tiles(h, h_dtype == MXFP4_BF16, D, N, D, at<int4>(ws, L.tiles), at<int>(ws, L.meta),
+                                  L.max_tiles, at<int>(ws, L.pair_token), at<uint8_t>(ws, L.xt_x),
+                                  xt_meta, at<uint8_t>(ws, L.at_x), at<uint8_t>(ws, L.x3_x),
+                                  at<int>(ws, L.meta) + 6, s, at<int4>(ws, L.wgroups), at<int>(ws, L.meta) + 4),
+           "quantise h tiles");
+  }
+  MX_PHASE("quant_h", s);
+  if (F % mx::kChunk) {  // padding blocks of the act buffer are read by the down product
+    MX_TRY(mx::launch_zero(at<void>(ws, L.at_act), at_bytes(L.max_tiles, F), s), "zero act");
+  }
   const int r = lo.r;
   LoraPtrs lp = {};
   mx::LoraPartial parts[4];

@@ -1436,9 +1436,23 @@ bool fast_path(int R, int K) { return K > 0 && (K % kChunk) == 0 && (long long)R
 
 bool fwd_bucket_split(int R, int K) { return fast_path(R, K); }
 
-bool fwd_few_rows(int rows, int n_ct, int R, int K)
+// Both work-group shapes of a routed product read the forward layout when every matrix of the product
+// has one (and its byte count fits a buffer resource, as for the checkpoint layout).
+static bool reads_forward_layout(const FwdArgs& a, int mode)
 {
-  return (long long)rows * ((n_ct + 7) / 8) <= 128 && (long long)R * (K / 2) < (1LL << 32);
+  return fast_path(a.R, a.K) && mode != kFwdPlain && a.fl0 && (mode != kFwdGateUp || a.fl1) &&
+         forward_layout_bytes(a.R, a.K) < (1LL << 32);
+}
+
+// Column tiles per work-group of the split-K items: up to four super-chunks half the waves take another one.
+static int split_columns(int K) { return at_nchunks(K) <= 4 ? 2 : 1; }
+
+constexpr int kSplitMaxGroups = 3 * 256;
+bool fwd_few_rows(const FwdArgs& a, int mode, int max_tiles)
+{
+  if ((long long)a.M * ((a.n_ct + 7) / 8) > 128 || (long long)a.R * (a.K / 2) >= (1LL << 32)) return false;
+  const int cols = split_columns(a.K);
+  return reads_forward_layout(a, mode) || std::min(a.M, max_tiles) * ((a.n_ct + cols - 1) / cols) <= kSplitMaxGroups;
 }
 
 // The split-K launch of a routed product: one tile (at most one per row) x 64 weight rows per item
@@ -1452,10 +1466,10 @@ static hipError_t launch_fwd_split_routed(const FwdArgs& a, int mode, int max_ti
     if (fl) hipLaunchKernelGGL((fwd_split_kernel<M, true, 4, 1, KS>), blocks(kSplitWaves / KS), block, 0, s, a); \
     else hipLaunchKernelGGL((fwd_split_kernel<M, false, 4, 1, KS>), blocks(kSplitWaves / KS), block, 0, s, a); \
   } while (0)
-  // up to four super-chunks: half the waves take another column tile
-  if (mode == kFwdGateUp && at_nchunks(a.K) <= 4) MX_SPLIT(kFwdGateUp, 4);
+  const bool two = split_columns(a.K) == 2;
+  if (mode == kFwdGateUp && two) MX_SPLIT(kFwdGateUp, 4);
   else if (mode == kFwdGateUp) MX_SPLIT(kFwdGateUp, 8);
-  else if (at_nchunks(a.K) <= 4) MX_SPLIT(kFwdDown, 4);
+  else if (two) MX_SPLIT(kFwdDown, 4);
   else MX_SPLIT(kFwdDown, 8);
 #undef MX_SPLIT
   return hipGetLastError();
@@ -1505,13 +1519,10 @@ hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s)
     b.small_tiles = nullptr;
     b.wgroups = nullptr;
   }
-  // both work-group shapes read the forward layout when every matrix of the product has one
-  // (and its byte count fits a buffer resource, as for the checkpoint layout)
-  const bool fl = fast && mode != kFwdPlain && a.fl0 && (mode != kFwdGateUp || a.fl1) &&
-                  forward_layout_bytes(a.R, a.K) < (1LL << 32);
+  const bool fl = reads_forward_layout(a, mode);
   // both bucket kinds in one launch: eight-wave one-tile items and wide large-bucket items
   const bool fused = fl && a.n_ct % 8 == 0 && split;
-  if (a.tiles && fwd_few_rows(a.M, a.n_ct, a.R, a.K)) return launch_fwd_split_routed(a, mode, max_tiles, fl, s);
+  if (a.tiles && fwd_few_rows(a, mode, max_tiles)) return launch_fwd_split_routed(a, mode, max_tiles, fl, s);
   const bool only_wide = split && a.all_wide;
   dim3 grid((unsigned)blocks), block(64 * kWavesPerGroup);
 #define MX_LAUNCH(M, F, L) hipLaunchKernelGGL((fwd_kernel<M, F, L>), grid, block, 0, s, b)

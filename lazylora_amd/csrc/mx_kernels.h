@@ -159,14 +159,18 @@ constexpr int kBwdColsPerTile = 256;  // output columns of one transposed-produc
 // resource addressing the whole matrix). Without the split every tile takes the one-tile
 // work-groups, whose gate/up product reads the token-major (XT) rows of x for every tile.
 bool fwd_bucket_split(int R, int K);
-// Whether a routed product of at most `rows` pair rows (so at most as many tiles) over W [R, K] runs
-// as split-K items of one tile x 64 weight rows, whatever its buckets: while its eight-column-tile
-// items (rows * ceil(n_ct / 8) of them at most) would leave half of the 256 CUs without one. Its
-// gate/up product then reads the token-major (XT) rows of x for every tile. Measured (us, gate/up
-// and down of 7168 / 2048 experts, one token's 8 experts, then two tokens' 16): forward layout 51 +
-// 20 -> 30 + 15, 57 + 26 -> 56 + 28; checkpoint layout 43 + 19 -> 32 + 18, 53 + 32 -> 65 + 34: the
-// line lies between one and two tokens.
-bool fwd_few_rows(int rows, int n_ct, int R, int K);
+// Whether the routed product `a` (of max_tiles tiles at most) runs as split-K items of one tile x 64
+// weight rows, whatever its buckets. Its gate/up product then reads the token-major (XT) rows of x for
+// every tile. The line: while its eight-column-tile items (at most rows * ceil(n_ct / 8)) would leave
+// half of the 256 CUs without one and, from the checkpoint layout, while the split work-groups are at
+// most three per CU: the one-tile items take one pass over the weights whatever the rows, the split ones
+// a round more every 256. Measured (us, the product with x's quantisation, as one-tile items / split, pairs
+// of distinct experts), gate/up of 7168 / 2048 from the checkpoint layout: 8 pairs (two rounds) 55 / 44, 9 to
+// 12 (three) 56 / 57 to 58 / 59, 14 (four) 59 / 72, 16 62 / 75; its down product: 8 pairs 20 / 22, 10 30 / 30;
+// gate/up of 3584 / 3072: 8 (three) 39 / 40, 10 (four) 40 / 48; its down product: 9 (two) 24 / 19, 13 (three)
+// 25 / 25, 16 (four) 26 / 31. From the forward layout, whose one-tile items are eight waves: gate/up of 7168 / 2048
+// 8 pairs 63 / 39, 16 68 / 64, 17 68 / 66.
+bool fwd_few_rows(const FwdArgs& a, int mode, int max_tiles);
 hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s);
 hipError_t launch_bwd(const BwdArgs& a, int mode, int max_tiles, hipStream_t s);
 // The dense transposed product (kBwdPlain) straight from the fp32 rows x [M, R] (4-byte aligned),

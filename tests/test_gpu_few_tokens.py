@@ -60,3 +60,23 @@ def test_few_pairs(k, D, F, N, topk, kind):
     keep = (idx >= 0) & (idx < E)
     want = oracle.routed_forward(h, np.where(keep, idx, 0), np.where(keep, w, 0), ex, act=act, lora=lo)
     assert_close(got, want, "out")
+
+
+def test_line_from_the_checkpoint_layout(k):
+    """Two tokens at top-8 of 7168 / 2048 experts are past the line: split-K items of the gate/up product
+    would be four rounds of the chip. They take the one-tile items that a larger batch takes, and a row's
+    result does not depend on the rows beside it there, so it is the batch's bit for bit (split-K adds
+    the products of a row in another order)."""
+    from lazylora_amd.experts import ExpertLayer
+    E, D, F, N, topk = 16, 7168, 2048, 18, 8
+    print(f"\n[case] 2 of {N} tokens, top-{topk} of {E}, D {D} F {F}", flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    mat = lambda R, K: (torch.randint(0, 256, (E, R, K // 2), dtype=torch.uint8, device="cuda", generator=gen),
+                        torch.randint(117, 122, (E, R, K // 32), dtype=torch.uint8, device="cuda", generator=gen))
+    L = ExpertLayer(*mat(F, D), *mat(F, D), *mat(D, F))
+    h = torch.randn((N, D), device="cuda", generator=gen)
+    w, idx = torch.topk(torch.rand((N, E), device="cuda", generator=gen), topk)
+    w, idx = w.contiguous(), idx.contiguous()
+    all_rows = k.routed_forward(h, idx, w, L)
+    assert torch.equal(k.routed_forward(h[:2].contiguous(), idx[:2].contiguous(), w[:2].contiguous(), L), all_rows[:2])
