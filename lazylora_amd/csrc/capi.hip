@@ -400,15 +400,27 @@ int check_forward_layout(const uint8_t* const* fl, int D, int F, int flags)
   return MXFP4_OK;
 }
 
-// Whether the buckets of a routed call are large from fewer tiles on (kFewerMinRows), and whether every
-// bucket of its forward is one.
+// Whether the buckets of a routed call are large from fewer tiles on (kFewerMinRows).
 bool moe_fewer(long long P, int E, int D, int F)
 {
   return P >= (long long)mx::kFewerMinRows * E && (long long)D * F >= mx::kFewerMinWeights;
 }
+// The eight-column items of a tile, both forward products together.
+int moe_items(int D, int F) { return (F + 255) / 256 + (D + 511) / 512; }
+// If so: the tiles past each expert's first up to which its short buckets stay with the forward's one-tile
+// items (kJudgeItems), which the routing's counts decide, or -1 where they take wide items in any case.
+int moe_judge(long long P, int E, int D, int F, bool layout)
+{
+  if (!moe_fewer(P, E, D, F) || P > 48LL * E) return -1;
+  const int items = moe_items(D, F);
+  if (layout) return mx::kJudgeItemsLayout / items;
+  return (P - 11LL * E) * items < 12LL * mx::kSureItems ? mx::kJudgeItems / items : -1;
+}
+bool moe_layout_copy(const uint8_t* const* fl) { return fl && (fl[0] || fl[2]); }
+// Whether every bucket of a routed call's forward takes wide items.
 bool moe_all_wide(long long P, int E, int D, int F, const uint8_t* const* fl)
 {
-  return moe_fewer(P, E, D, F) && !(fl && (fl[0] || fl[2]));
+  return moe_fewer(P, E, D, F) && !moe_layout_copy(fl) && moe_judge(P, E, D, F, false) < 0;
 }
 
 // Routing + quantised x + gate/up (+GLU) into the workspace. With LoRA also the per-token
@@ -421,13 +433,13 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
 {
   const long long P = (long long)N * k;
   const bool fewer = moe_fewer(P, E, D, F);
-  const bool all_wide = moe_all_wide(P, E, D, F, fl);
+  const bool layout = moe_layout_copy(fl);
   MX_TRY(mx::launch_route(idx, idx_dtype == MXFP4_I64, w, N, k, E, at<int>(ws, L.counts), at<int>(ws, L.offsets),
                           at<int>(ws, L.cursor), at<int4>(ws, L.tiles), at<int>(ws, L.small_tiles),
                           at<int>(ws, L.bsmall_tiles), at<int4>(ws, L.groups), at<int4>(ws, L.wgroups),
-                          at<int>(ws, L.meta), all_wide ? 1 : fewer ? mx::kWideMinTiles : mx::kLargeMinTiles,
-                          fewer ? mx::kGroupMinTiles : mx::kLargeMinTiles, at<int>(ws, L.pair_token),
-                          at<float>(ws, L.pair_w), at<int>(ws, L.pair_of), s),
+                          at<int>(ws, L.meta), !fewer ? mx::kLargeMinTiles : layout ? mx::kWideMinTiles : 1,
+                          fewer ? mx::kGroupMinTiles : mx::kLargeMinTiles, moe_judge(P, E, D, F, layout),
+                          at<int>(ws, L.pair_token), at<float>(ws, L.pair_w), at<int>(ws, L.pair_of), s),
          "route");
   MX_PHASE("route", s);
   mx::FwdArgs a = {};
@@ -444,7 +456,7 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
   a.x3_any = at<int>(ws, L.meta) + 6;
   a.row_token = at<int>(ws, L.pair_token);
   a.tiles = at<int4>(ws, L.tiles); a.n_tiles = at<int>(ws, L.meta); a.M = (int)P;
-  a.all_wide = all_wide;
+  a.all_wide = moe_all_wide(P, E, D, F, fl);
   a.n_ct = F / 32;
   a.q_tiles = at<uint8_t>(ws, L.at_act);
   set_buckets(a, ws, L);

@@ -138,19 +138,31 @@ constexpr int kGroupTiles = 4;     // row tiles of one large-bucket group
 constexpr int kWideGroupTiles = 8;  // row tiles of one wide group (the large-bucket forward)
 // Experts with at least this many tiles take the large-bucket path: usually four; where the buckets average
 // kFewerMinRows rows, two in the forward (a wide item of two tiles reads the weights once and takes little
-// longer than a one-tile item; with few such experts, as under uniform routing of small batches, the extra
-// items would only lengthen the launch's tail) and three in the transposed products (whose items always
-// compute four tiles). From the checkpoint layout the forward then has no one-tile items at all: a launch
+// longer than a one-tile item) and three in the transposed products (whose items always compute four
+// tiles). From the checkpoint layout the forward then has no one-tile items at all: a launch
 // of their own for the few short buckets costs more than their wide items (3584 / 3072, 64 experts, top-8,
-// whole forward, us, with them then without: 8 rows per bucket 252 / 296, 12 rows 352 / 306, 20 rows 375 /
-// 314, 64 rows 419 / 412; Zipf 20 rows 363 / 349, 64 rows 538 / 506; 7168 / 2048, 128 experts, 16 rows 748
-// / 699). With a forward layout both kinds share one launch, and the one-tile items stay (12 rows 233 /
-// 239, Zipf 64 rows 430 / 440). 128 tokens, top-16 of 64 experts (32 rows on average, 3584 / 3072,
-// checkpoint layout), four everywhere, then this: gate/up 0.33 -> 0.24 ms, down 0.18 -> 0.13, W1 | W3
-// transposed 0.38 -> 0.29, W2 0.20 -> 0.20.
+// whole forward, us, with them then without: 20 rows per bucket 375 / 314, 64 rows 419 / 412; Zipf 20 rows
+// 363 / 349, 64 rows 538 / 506; 7168 / 2048, 128 experts, 16 rows 748 / 699). With a forward layout both
+// kinds share one launch, and the one-tile items stay (Zipf 64 rows 430 / 440). 128 tokens, top-16 of 64
+// experts (32 rows on average, 3584 / 3072, checkpoint layout), four everywhere, then this: gate/up 0.33 ->
+// 0.24 ms, down 0.18 -> 0.13, W1 | W3 transposed 0.38 -> 0.29, W2 0.20 -> 0.20.
 constexpr int kLargeMinTiles = 4, kWideMinTiles = 2, kGroupMinTiles = 3;
 constexpr int kFewerMinRows = 12;
 constexpr long long kFewerMinWeights = 1 << 20;  // elements per matrix: below, both shapes are a launch's latency
+// Short buckets (none of kLargeMinTiles tiles) are another matter: a wide item waits out the same serial
+// quarters whether it has one tile or three, while one-tile items of one expert run side by side. Wide items
+// pay only from a number of weight readings saved: the tiles past each expert's first x the eight-column
+// items of a tile (both products) above kJudgeItems, with a forward layout kJudgeItemsLayout (one and a
+// half to two for each CU). Whole forward, us, as one-tile items / wide, uniform routing: 7168 / 2048 from the
+// checkpoint layout, 16 experts of 16 rows (158 items saved) 143 / 156, of 32 (510) 193 / 167, 32 of 20 (563)
+// 270 / 218; forward layout, 16 of 16 121 / 140, of 32 187 / 148; 3584 / 3072, checkpoint layout, 16 of 24 (304)
+// 119 / 137, 64 of 12 (152) 264 / 290, of 16 (547) 329 / 297; 2048 / 1024, 32 of 24 (256) 64 / 83, 128 of 20
+// (820) 178 / 158. The routing's counts decide it on the device unless some bucket must be of four tiles (P >
+// 48 E). From the checkpoint layout, where leaving both kinds possible costs an empty launch of each
+// product (5 us), the wide items are taken for sure where uniform routing would save more than kSureItems,
+// its tiles past the first being about (P - 11 E) / 12.
+constexpr int kJudgeItems = 480, kJudgeItemsLayout = 390;
+constexpr int kSureItems = 420;
 constexpr int kFwdColsPerTile = 64;  // kFwdPlain / kFwdDown; kFwdGateUp covers 32 features
 constexpr int kBwdColsPerTile = 256;  // output columns of one transposed-product wave
 
@@ -225,11 +237,12 @@ hipError_t launch_dequant(void* out, int out_bf16, const uint8_t* packed, const 
 // an id outside [0, E)), small tiles (forward), groups, wide groups, full wide groups, third term
 // present (set by the quantisers), small tiles (transposed), then the work queues (2 ints each) of
 // the wide-group launches of the forward gate/up and down products, ...} (16 ints, all zeroed
-// here), and the pair maps.
+// here), and the pair maps. judge (>= 0): where no expert has kLargeMinTiles tiles and no more than `judge`
+// tiles lie past an expert's first, kLargeMinTiles stands for wide_min.
 hipError_t launch_route(const void* topk_idx, int idx64, const float* topk_w, int N, int k, int E, int* counts,
                         int* offsets, int* cursor, int4* tiles, int* small_tiles, int* bsmall_tiles, int4* groups,
-                        int4* wgroups, int* meta, int wide_min, int group_min, int* pair_token, float* pair_w,
-                        int* pair_of, hipStream_t s);
+                        int4* wgroups, int* meta, int wide_min, int group_min, int judge, int* pair_token,
+                        float* pair_w, int* pair_of, hipStream_t s);
 hipError_t launch_combine(float* out, const float* ypair, long long ldy, const int* pair_of, int N, int k,
                           int D, hipStream_t s);
 // Top-1 routing (the down product writes token rows itself): zeros into the rows of tokens with no

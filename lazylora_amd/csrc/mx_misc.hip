@@ -381,6 +381,12 @@ MX_DEV int group16_isum(int v)
 {
   return dpp_add<kDppMirror>(dpp_add<kDppHalfMirror>(dpp_add<kDppXor2>(dpp_add<kDppXor1>(v))));
 }
+MX_DEV int wave_isum(int v)
+{
+  v = group16_isum(v);
+  return (__builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16)) +
+         (__builtin_amdgcn_readlane(v, 32) + __builtin_amdgcn_readlane(v, 48));
+}
 
 // Single work-group of 1024: exclusive scan of counts and of per-expert tile counts, tile list. An
 // expert with at least group_min tiles (a large bucket of the transposed products) also gets its
@@ -392,9 +398,15 @@ MX_DEV int group16_isum(int v)
 // (forward), groups, wide groups, full wide groups, -, small tiles (transposed)}. cursor[e] gets
 // offsets[e] (cursor may be counts itself: each expert's count is read before its cursor is written,
 // by the same thread). The scan is within each wave by lane moves and across the 16 waves through
-// their totals: two barriers (one for 20 in LDS took 4 us of this latency-bound kernel's 20).
+// their totals: one barrier (20 in LDS took 4 us of this latency-bound kernel's 20). With `judge`
+// (>= 0: the buckets may be short) the counts are first looked at as a whole, one more barrier (LDS
+// atomics for its sums took 4 us).
 // Returns the number of rows (pairs with an expert).
 constexpr int kScan = 7;  // rows, tiles, small (forward), groups, full wide groups, partial ones, small (transposed)
+struct ScanLds {
+  int tot[kScan][16];  // the waves' totals
+  int judge[2][16];    // of the tiles past an expert's first, experts of kLargeMinTiles tiles
+};
 struct RouteOut {
   int* offsets;
   int4* tiles;
@@ -403,19 +415,38 @@ struct RouteOut {
   int4* groups;
   int4* wgroups;
   int* meta;
-  int wide_min, group_min;
+  int wide_min, group_min, judge;
 };
-__device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor, const RouteOut& o, int (*s_tot)[16])
+__device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor, const RouteOut& o, ScanLds& lds)
 {
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int per = (E + 1023) / 1024;
   const int e0 = min(t * per, E), e1 = min(e0 + per, E);
+  int wide_min = o.wide_min;
+  if (o.judge >= 0) {  // uniform
+    int past = 0, large = 0;
+    for (int e = e0; e < e1; ++e) {
+      const int et = (counts[e] + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
+      past += max(et - 1, 0);
+      large |= et >= kLargeMinTiles ? 1 : 0;
+    }
+    past = wave_isum(past);
+    large = wave_isum(large);
+    if (lane == 63) {
+      lds.judge[0][wave] = past;
+      lds.judge[1][wave] = large;
+    }
+    __syncthreads();
+    past = group16_isum(lds.judge[0][lane & 15]);
+    large = group16_isum(lds.judge[1][lane & 15]);
+    if (large == 0 && past <= o.judge) wide_min = kLargeMinTiles;
+  }
   int v[kScan] = {};
   for (int e = e0; e < e1; ++e) {
     const int et = (counts[e] + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
     v[0] += counts[e];
     v[1] += et;
-    if (et >= o.wide_min) {
+    if (et >= wide_min) {
       v[4] += et / kWideGroupTiles;
       v[5] += et % kWideGroupTiles ? 1 : 0;
     } else {
@@ -436,12 +467,12 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
     }
   if (lane == 63)
 #pragma unroll
-    for (int i = 0; i < kScan; ++i) s_tot[i][wave] = inc[i];
+    for (int i = 0; i < kScan; ++i) lds.tot[i][wave] = inc[i];
   __syncthreads();
   int off[kScan], total[kScan];  // exclusive offsets and totals
 #pragma unroll
   for (int i = 0; i < kScan; ++i) {
-    const int w = s_tot[i][lane & 15];
+    const int w = lds.tot[i][lane & 15];
     total[i] = group16_isum(w);
     off[i] = group16_isum((lane & 15) < wave ? w : 0) + inc[i] - v[i];
   }
@@ -456,7 +487,7 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
       for (int g = 0; g < et; g += kGroupTiles) o.groups[group_off++] = make_int4(e, tile_off + g, min(kGroupTiles, et - g), 0);
     else
       for (int m = 0; m < et; ++m) o.bsmall_tiles[bsmall_off++] = tile_off + m;
-    if (et >= o.wide_min) {
+    if (et >= wide_min) {
       for (int g = 0; g + kWideGroupTiles <= et; g += kWideGroupTiles)
         o.wgroups[wgroup_off++] = make_int4(e, tile_off + g, kWideGroupTiles, 0);
       if (et % kWideGroupTiles)
@@ -481,8 +512,8 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
 
 __global__ __launch_bounds__(1024) void route_scan_kernel(const int* counts, int E, int* cursor, RouteOut o)
 {
-  __shared__ int s_tot[kScan][16];
-  route_scan(counts, E, cursor, o, s_tot);
+  __shared__ ScanLds lds;
+  route_scan(counts, E, cursor, o, lds);
 }
 
 // The whole routing in one work-group (P <= kRouteOneP pairs, E <= kRouteOneE experts): counts
@@ -500,7 +531,7 @@ __global__ __launch_bounds__(1024) void route_one_kernel(const void* idx, int id
                                                          int E, int* counts, RouteOut o, int* pair_token,
                                                          float* pair_w, int* pair_of)
 {
-  __shared__ int s_tot[kScan][16];
+  __shared__ ScanLds lds;
   __shared__ int s_cnt[kRouteOneE];
   __shared__ uint16_t s_tok[kRouteStageP];  // tokens fit: no more of them than pairs, at most 2^16
   __shared__ float s_w[kRouteStageP];
@@ -533,7 +564,7 @@ __global__ __launch_bounds__(1024) void route_one_kernel(const void* idx, int id
   // flags and work-queue counters, which start at zero) are written here
   if (t == 1) o.meta[1] = s_bad;
   if (t == 6 || (t >= 8 && t < 16)) o.meta[t] = 0;
-  const int placed = route_scan(s_cnt, E, s_cnt, o, s_tot);  // pairs with a valid expert id
+  const int placed = route_scan(s_cnt, E, s_cnt, o, lds);  // pairs with a valid expert id
   __syncthreads();
   for (int p0 = 0; p0 < P; p0 += 8 * 1024) {
     IdWords id[8];
@@ -777,11 +808,11 @@ hipError_t launch_zero(void* p, size_t bytes, hipStream_t s)
 
 hipError_t launch_route(const void* topk_idx, int idx64, const float* topk_w, int N, int k, int E, int* counts,
                         int* offsets, int* cursor, int4* tiles, int* small_tiles, int* bsmall_tiles, int4* groups,
-                        int4* wgroups, int* meta, int wide_min, int group_min, int* pair_token, float* pair_w,
-                        int* pair_of, hipStream_t s)
+                        int4* wgroups, int* meta, int wide_min, int group_min, int judge, int* pair_token,
+                        float* pair_w, int* pair_of, hipStream_t s)
 {
   const int P = N * k;
-  const RouteOut o{offsets, tiles, small_tiles, bsmall_tiles, groups, wgroups, meta, wide_min, group_min};
+  const RouteOut o{offsets, tiles, small_tiles, bsmall_tiles, groups, wgroups, meta, wide_min, group_min, judge};
   if (P <= kRouteOneP && E <= kRouteOneE) {
     hipLaunchKernelGGL(route_one_kernel, dim3(1), dim3(1024), 0, s, topk_idx, idx64, topk_w, P, k, E, counts, o,
                        pair_token, pair_w, pair_of);

@@ -55,8 +55,8 @@ def test_bucket_sizes(k, D, F, inputs, forward_layout):
 @pytest.mark.parametrize("D,F", ((1024, 1056), (1056, 1024), (1536, 1024)))
 @pytest.mark.parametrize("rank", (0, 8))
 def test_no_one_tile_items(k, D, F, rank, pairs_over_line):
-    """Top-3, on both sides of the 12 rows per expert from which a forward from the checkpoint layout
-    gives every bucket wide items (some of one row, one of none), and where only one of the two products
+    """Top-3, on both sides of the 12 rows per expert from which the routing's counts decide whether a
+    forward's buckets take wide items (short ones, as here, do not), and where only one of the two products
     has them (the other's K is no multiple of 512)."""
     import types
 
@@ -83,6 +83,60 @@ def test_no_one_tile_items(k, D, F, rank, pairs_over_line):
     out = k.routed_forward(c(h), c(idx), c(w), L, lora=adapters)
     got = k.routed_backward(c(h), c(idx), c(w), L, c(g), lora=adapters)
     assert_close(out.cpu().numpy(), oracle.routed_forward(h, idx, w, ex, lora=lo), "out")
+    want = oracle.routed_backward(h, idx, w, ex, g, lora=lo)
+    for name, a, b in zip(("grad_h", "grad_w"), got, want):
+        assert_close(a.cpu().numpy(), b, name)
+
+
+SHORT = (16, 17, 1, 20, 32, 15, 48, 16, 0, 33, 8, 16, 30, 2, 16, 5)
+
+
+# (rows of expert 0, 1, .., wide groups from the checkpoint layout, from the forward layout)
+@pytest.mark.parametrize("rows,none,forward", (
+    (SHORT, 0, 0),                   # no bucket of four tiles, few tiles past the first: one-tile items
+    (SHORT[:-1] + (49,), 15, 7),     # one large bucket: all that have rows, and those of two tiles and more
+    ((17,) * 65 + (12,) * 10, 0, 0),   # 65 tiles past the first: below both lines
+    ((17,) * 66 + (12,) * 10, 0, 66),  # past the forward layout's
+    ((17,) * 80 + (12,) * 10, 0, 80),  # 80: at the checkpoint layout's
+    ((17,) * 81 + (12,) * 10, 91, 81),  # past it
+    ((22,) * 80, 80, 80),            # averages that settle it from the checkpoint layout
+    (tuple(8 + n % 90 for n in range(90)), 90, 81),  # 52 rows on average: large whatever the counts
+))
+@pytest.mark.parametrize("forward_layout,rank", ((False, 8), (True, 0)))
+def test_short_buckets(k, rows, none, forward, forward_layout, rank):
+    """Which buckets take wide items (meta word 4, at the start of the workspace, counts their groups), and
+    the results, on both sides of each line of that rule; buckets of one row among those that do."""
+    import types
+
+    from lazylora_amd.experts import ExpertLayer
+    print(f"\n[case] {len(rows)} experts, {sum(rows)} rows, forward layout {forward_layout}, rank {rank}", flush=True)
+    E, N, D, F = len(rows), sum(rows), 1024, 1024
+    rng = np.random.default_rng(N)
+    ex = oracle.random_experts(rng, E, D, F, 117, 121)
+    h, g = (rng.standard_normal((N, D)).astype(np.float32) for _ in range(2))
+    idx = np.repeat(np.arange(E), rows)[rng.permutation(N)].reshape(N, 1)
+    w = rng.uniform(0.5, 1.0, (N, 1)).astype(np.float32)
+    lo = adapters = None
+    if rank:
+        A = lambda n_in, n_out: (0.05 * rng.standard_normal((rank, n_in)).astype(np.float32),
+                                 0.05 * rng.standard_normal((n_out, rank)).astype(np.float32))
+        parts = A(D, F), A(D, F), A(F, D)
+        lo = oracle.LoRA(*[v for p in parts for v in p])
+        adapters = tuple(types.SimpleNamespace(lora_A=torch.from_numpy(a).cuda(), lora_B=torch.from_numpy(b).cuda(),
+                                               scaling=2.0, dropout_rate=0.0) for a, b in parts)
+    L = ExpertLayer(*[torch.from_numpy(a).cuda() for a in (ex.w1p, ex.w1s, ex.w3p, ex.w3s, ex.w2p, ex.w2s)])
+    if forward_layout:
+        L.prepare_forward_layout()
+    c = lambda a: torch.from_numpy(a).cuda()
+    ws = torch.empty(k.moe_workspace_bytes(N, 1, E, D, F), dtype=torch.uint8, device="cuda")
+    out = k.routed_forward(c(h), c(idx), c(w), L, lora=adapters, save_for_backward=True, workspace=ws)
+    assert int(ws[:64].view(torch.int32)[4]) == (forward if forward_layout else none)
+    want = oracle.routed_forward(h, idx, w, ex, lora=lo)
+    got = out.cpu().numpy()
+    for e in range(E):  # no bucket hides in the others
+        if rows[e]:
+            assert_close(got[idx[:, 0] == e], want[idx[:, 0] == e], f"expert with {rows[e]} rows")
+    got = k.routed_backward(c(h), c(idx), c(w), L, c(g), lora=adapters, reuse_forward=True, workspace=ws)
     want = oracle.routed_backward(h, idx, w, ex, g, lora=lo)
     for name, a, b in zip(("grad_h", "grad_w"), got, want):
         assert_close(a.cpu().numpy(), b, name)
