@@ -416,6 +416,11 @@ int moe_judge(long long P, int E, int D, int F, bool layout)
   if (layout) return mx::kJudgeItemsLayout / items;
   return (P - 11LL * E) * items < 12LL * mx::kSureItems ? mx::kJudgeItems / items : -1;
 }
+// The same for the transposed products: the experts of kGroupMinTiles tiles up to which they take one-tile items.
+int moe_judge_groups(long long P, int E, int D, int F)
+{
+  return moe_fewer(P, E, D, F) && P <= 48LL * E ? mx::kJudgeGroupItems / moe_items(D, F) : -1;
+}
 bool moe_layout_copy(const uint8_t* const* fl) { return fl && (fl[0] || fl[2]); }
 // Whether every bucket of a routed call's forward takes wide items.
 bool moe_all_wide(long long P, int E, int D, int F, const uint8_t* const* fl)
@@ -439,7 +444,8 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
                           at<int>(ws, L.bsmall_tiles), at<int4>(ws, L.groups), at<int4>(ws, L.wgroups),
                           at<int>(ws, L.meta), !fewer ? mx::kLargeMinTiles : layout ? mx::kWideMinTiles : 1,
                           fewer ? mx::kGroupMinTiles : mx::kLargeMinTiles, moe_judge(P, E, D, F, layout),
-                          at<int>(ws, L.pair_token), at<float>(ws, L.pair_w), at<int>(ws, L.pair_of), s),
+                          moe_judge_groups(P, E, D, F), at<int>(ws, L.pair_token), at<float>(ws, L.pair_w),
+                          at<int>(ws, L.pair_of), s),
          "route");
   MX_PHASE("route", s);
   mx::FwdArgs a = {};

@@ -163,6 +163,13 @@ constexpr long long kFewerMinWeights = 1 << 20;  // elements per matrix: below, 
 // its tiles past the first being about (P - 11 E) / 12.
 constexpr int kJudgeItems = 480, kJudgeItemsLayout = 390;
 constexpr int kSureItems = 420;
+// The transposed products likewise: a group item of three tiles decodes once but takes longer than a one-tile
+// item, so a few of them only lengthen a launch whose other items are done after one round. They pay where
+// some bucket has such items anyway, or from that many experts of three tiles x the items above. Both
+// products, us, as one-tile items / groups, 7168 / 2048, checkpoint layout, uniform routing: 64 experts of 24
+// rows (3 of three tiles) 556 / 702, of 32 (29) 759 / 698; 32 of 32 (14) 436 / 436, 16 of 32 (7) 330 / 415;
+// 3584 / 3072: 32 of 32 338 / 435, 64 of 32 566 / 461; 2048 / 1024: 64 of 32 147 / 177, 128 of 32 (58) 250 / 234.
+constexpr int kJudgeGroupItems = 400;
 constexpr int kFwdColsPerTile = 64;  // kFwdPlain / kFwdDown; kFwdGateUp covers 32 features
 constexpr int kBwdColsPerTile = 256;  // output columns of one transposed-product wave
 
@@ -238,11 +245,12 @@ hipError_t launch_dequant(void* out, int out_bf16, const uint8_t* packed, const 
 // present (set by the quantisers), small tiles (transposed), then the work queues (2 ints each) of
 // the wide-group launches of the forward gate/up and down products, ...} (16 ints, all zeroed
 // here), and the pair maps. judge (>= 0): where no expert has kLargeMinTiles tiles and no more than `judge`
-// tiles lie past an expert's first, kLargeMinTiles stands for wide_min.
+// tiles lie past an expert's first, kLargeMinTiles stands for wide_min; judge_groups (>= 0): where no expert
+// has kLargeMinTiles tiles and no more than that many have kGroupMinTiles, kLargeMinTiles stands for group_min.
 hipError_t launch_route(const void* topk_idx, int idx64, const float* topk_w, int N, int k, int E, int* counts,
                         int* offsets, int* cursor, int4* tiles, int* small_tiles, int* bsmall_tiles, int4* groups,
-                        int4* wgroups, int* meta, int wide_min, int group_min, int judge, int* pair_token,
-                        float* pair_w, int* pair_of, hipStream_t s);
+                        int4* wgroups, int* meta, int wide_min, int group_min, int judge, int judge_groups,
+                        int* pair_token, float* pair_w, int* pair_of, hipStream_t s);
 hipError_t launch_combine(float* out, const float* ypair, long long ldy, const int* pair_of, int N, int k,
                           int D, hipStream_t s);
 // Top-1 routing (the down product writes token rows itself): zeros into the rows of tokens with no

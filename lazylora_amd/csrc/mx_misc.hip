@@ -398,14 +398,14 @@ MX_DEV int wave_isum(int v)
 // (forward), groups, wide groups, full wide groups, -, small tiles (transposed)}. cursor[e] gets
 // offsets[e] (cursor may be counts itself: each expert's count is read before its cursor is written,
 // by the same thread). The scan is within each wave by lane moves and across the 16 waves through
-// their totals: one barrier (20 in LDS took 4 us of this latency-bound kernel's 20). With `judge`
-// (>= 0: the buckets may be short) the counts are first looked at as a whole, one more barrier (LDS
-// atomics for its sums took 4 us).
+// their totals: one barrier (20 in LDS took 4 us of this latency-bound kernel's 20). With `judge` or
+// `judge_groups` (>= 0: the buckets may be short) the counts are first looked at as a whole, one more
+// barrier (LDS atomics for its three sums took 4 us).
 // Returns the number of rows (pairs with an expert).
 constexpr int kScan = 7;  // rows, tiles, small (forward), groups, full wide groups, partial ones, small (transposed)
 struct ScanLds {
   int tot[kScan][16];  // the waves' totals
-  int judge[2][16];    // of the tiles past an expert's first, experts of kLargeMinTiles tiles
+  int judge[3][16];    // of the tiles past an expert's first, experts of kLargeMinTiles and of kGroupMinTiles tiles
 };
 struct RouteOut {
   int* offsets;
@@ -415,31 +415,36 @@ struct RouteOut {
   int4* groups;
   int4* wgroups;
   int* meta;
-  int wide_min, group_min, judge;
+  int wide_min, group_min, judge, judge_groups;
 };
 __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor, const RouteOut& o, ScanLds& lds)
 {
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int per = (E + 1023) / 1024;
   const int e0 = min(t * per, E), e1 = min(e0 + per, E);
-  int wide_min = o.wide_min;
-  if (o.judge >= 0) {  // uniform
-    int past = 0, large = 0;
+  int wide_min = o.wide_min, group_min = o.group_min;
+  if (o.judge >= 0 || o.judge_groups >= 0) {  // uniform
+    int past = 0, large = 0, group = 0;
     for (int e = e0; e < e1; ++e) {
       const int et = (counts[e] + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
       past += max(et - 1, 0);
       large |= et >= kLargeMinTiles ? 1 : 0;
+      group += et == kGroupMinTiles ? 1 : 0;
     }
     past = wave_isum(past);
     large = wave_isum(large);
+    group = wave_isum(group);
     if (lane == 63) {
       lds.judge[0][wave] = past;
       lds.judge[1][wave] = large;
+      lds.judge[2][wave] = group;
     }
     __syncthreads();
     past = group16_isum(lds.judge[0][lane & 15]);
     large = group16_isum(lds.judge[1][lane & 15]);
+    group = group16_isum(lds.judge[2][lane & 15]);
     if (large == 0 && past <= o.judge) wide_min = kLargeMinTiles;
+    if (large == 0 && group <= o.judge_groups) group_min = kLargeMinTiles;
   }
   int v[kScan] = {};
   for (int e = e0; e < e1; ++e) {
@@ -452,7 +457,7 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
     } else {
       v[2] += et;
     }
-    if (et >= o.group_min) v[3] += (et + kGroupTiles - 1) / kGroupTiles;
+    if (et >= group_min) v[3] += (et + kGroupTiles - 1) / kGroupTiles;
     else v[6] += et;
   }
   int inc[kScan];  // inclusive sums
@@ -483,7 +488,7 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
     const int et = (c + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
     o.offsets[e] = row_off;
     cursor[e] = row_off;
-    if (et >= o.group_min)
+    if (et >= group_min)
       for (int g = 0; g < et; g += kGroupTiles) o.groups[group_off++] = make_int4(e, tile_off + g, min(kGroupTiles, et - g), 0);
     else
       for (int m = 0; m < et; ++m) o.bsmall_tiles[bsmall_off++] = tile_off + m;
@@ -808,11 +813,12 @@ hipError_t launch_zero(void* p, size_t bytes, hipStream_t s)
 
 hipError_t launch_route(const void* topk_idx, int idx64, const float* topk_w, int N, int k, int E, int* counts,
                         int* offsets, int* cursor, int4* tiles, int* small_tiles, int* bsmall_tiles, int4* groups,
-                        int4* wgroups, int* meta, int wide_min, int group_min, int judge, int* pair_token,
-                        float* pair_w, int* pair_of, hipStream_t s)
+                        int4* wgroups, int* meta, int wide_min, int group_min, int judge, int judge_groups,
+                        int* pair_token, float* pair_w, int* pair_of, hipStream_t s)
 {
   const int P = N * k;
-  const RouteOut o{offsets, tiles, small_tiles, bsmall_tiles, groups, wgroups, meta, wide_min, group_min, judge};
+  const RouteOut o{offsets, tiles, small_tiles, bsmall_tiles, groups, wgroups, meta, wide_min, group_min, judge,
+                   judge_groups};
   if (P <= kRouteOneP && E <= kRouteOneE) {
     hipLaunchKernelGGL(route_one_kernel, dim3(1), dim3(1024), 0, s, topk_idx, idx64, topk_w, P, k, E, counts, o,
                        pair_token, pair_w, pair_of);

@@ -140,3 +140,38 @@ def test_short_buckets(k, rows, none, forward, forward_layout, rank):
     want = oracle.routed_backward(h, idx, w, ex, g, lora=lo)
     for name, a, b in zip(("grad_h", "grad_w"), got, want):
         assert_close(a.cpu().numpy(), b, name)
+
+
+# (rows of expert 0, 1, .., groups of the transposed products' large buckets)
+@pytest.mark.parametrize("rows,groups", (
+    (SHORT, 0),                      # two experts of three tiles, none of four
+    (SHORT[:-1] + (49,), 3),         # one of four: three groups
+    ((33, 40, 48) * 22, 0),          # 66 of three tiles
+    ((33, 40, 48) * 22 + (35,), 67),  # 67
+    (tuple(8 + n % 90 for n in range(90)), 98),  # over 48 rows on average
+))
+@pytest.mark.parametrize("layout", (False, True))
+def test_three_tile_groups(k, rows, groups, layout):
+    """Which buckets of three tiles the transposed products give their large-bucket items (meta word 3, at the
+    start of the workspace, counts the groups), and the gradients, on both sides of each line of that rule."""
+    from lazylora_amd.experts import ExpertLayer
+    print(f"\n[case] {len(rows)} experts, {sum(rows)} rows, backward layout {layout}", flush=True)
+    E, N, D, F = len(rows), sum(rows), 1024, 1024
+    rng = np.random.default_rng(N)
+    ex = oracle.random_experts(rng, E, D, F, 117, 121)
+    h, g = (rng.standard_normal((N, D)).astype(np.float32) for _ in range(2))
+    idx = np.repeat(np.arange(E), rows)[rng.permutation(N)].reshape(N, 1)
+    w = rng.uniform(0.5, 1.0, (N, 1)).astype(np.float32)
+    L = ExpertLayer(*[torch.from_numpy(a).cuda() for a in (ex.w1p, ex.w1s, ex.w3p, ex.w3s, ex.w2p, ex.w2s)])
+    if layout:
+        L.prepare_backward_layout()
+    c = lambda a: torch.from_numpy(a).cuda()
+    ws = torch.empty(k.moe_workspace_bytes(N, 1, E, D, F), dtype=torch.uint8, device="cuda")
+    gh, gw = k.routed_backward(c(h), c(idx), c(w), L, c(g), workspace=ws)
+    assert int(ws[:64].view(torch.int32)[3]) == groups
+    gh, gw = gh.cpu().numpy(), gw.cpu().numpy()
+    want = oracle.routed_backward(h, idx, w, ex, g)
+    for e in range(E):
+        if rows[e]:
+            assert_close(gh[idx[:, 0] == e], want[0][idx[:, 0] == e], f"grad_h of the expert with {rows[e]} rows")
+    assert_close(gw, want[1], "grad_w")
