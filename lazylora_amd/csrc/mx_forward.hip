@@ -1146,18 +1146,23 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, int expert, int 
 // skipped), so the work-groups take them from a work counter in list order: the full groups' items first,
 // then the partial groups', which fill in behind them. Consecutive items are the eight column blocks of one
 // group, which run at about the same time and share its activations. The items past the last whole round of
-// the grid are cut into two or four runs of tiles where that many work-groups per item would idle: a run of
+// the grid are cut into two or four runs of tiles where work-groups for all of these would idle: a run of
 // two of eight tiles reads the weights again but takes about half the time (whole forward from the
 // checkpoint layout, top-8, Zipf routing: 1024 pairs over 128 experts, 7168 / 2048, 535 -> 443 us; 512 over
-// 64, 3584 / 3072, 312 -> 281; 256 rows to each of 32 experts from the forward layout 701 -> 691).
+// 64, 3584 / 3072, 312 -> 281; 256 rows to each of 32 experts from the forward layout 701 -> 691). An item
+// of one tile is one run: eight experts of 8 or 9 tiles are 144 items of gate/up, 96 to be cut and up to 48 not.
 template <int MODE, bool FL>
 __device__ __forceinline__ void fwd_wide_items(const FwdArgs& a, int wave, int lane, WideLds& lds, int* s_item)
 {
-  const int ng = *(cint_ptr)a.n_wgroups;
+  const cint_ptr m = (cint_ptr)a.n_wgroups;  // meta words 4, 5 .. and 12, 13 (see launch_route)
+  const int ng = m[0];
   if (ng == 0) return;  // no large buckets: the whole grid leaves without touching the queue
   const int nfb = (a.n_ct + kWgWaves - 1) / kWgWaves;
   const int total = ng * nfb, rem = total % (int)gridDim.x, whole = total - rem;
-  const int sh = rem * 4 <= (int)gridDim.x ? 2 : rem * 2 <= (int)gridDim.x ? 1 : 0;  // log2 of the runs
+  // the items of the partial groups, which come last, have no more runs than tiles
+  const int full = rem - (ng - m[1]) * nfb;
+  auto runs = [&](int s) { return full < 0 ? rem << s : (full << s) + m[7 + s] * nfb; };
+  const int sh = runs(2) <= (int)gridDim.x ? 2 : runs(1) <= (int)gridDim.x ? 1 : 0;  // log2 of the runs
   const int end = whole + (rem << sh);
   for (;;) {
     const int it = queue_next(a.wcounter, s_item);  // also: every wave is done with the LDS before

@@ -243,7 +243,8 @@ hipError_t launch_dequant(void* out, int out_bf16, const uint8_t* packed, const 
 // of up to kGroupTiles and their other tiles' indices (bsmall_tiles), meta = {tiles, flags (bit 0:
 // an id outside [0, E)), small tiles (forward), groups, wide groups, full wide groups, third term
 // present (set by the quantisers), small tiles (transposed), then the work queues (2 ints each) of
-// the wide-group launches of the forward gate/up and down products, ...} (16 ints, all zeroed
+// the wide-group launches of the forward gate/up and down products, the runs of the partial wide groups
+// when each is cut into two or four (at most its tiles), -, -} (16 ints, all zeroed or written
 // here), and the pair maps. judge (>= 0): where no expert has kLargeMinTiles tiles and no more than `judge`
 // tiles lie past an expert's first, kLargeMinTiles stands for wide_min; judge_groups (>= 0): where no expert
 // has kLargeMinTiles tiles and no more than that many have kGroupMinTiles, kLargeMinTiles stands for group_min.

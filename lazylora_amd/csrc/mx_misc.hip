@@ -395,7 +395,8 @@ MX_DEV int wave_isum(int v)
 // gets wide groups of up to kWideGroupTiles: every full wide group first (expert order), then the
 // experts' last, partial ones, so that a work queue taking them in order hands out the largest
 // items first; the other experts' tile indices go to small_tiles. meta = {tiles, flags, small tiles
-// (forward), groups, wide groups, full wide groups, -, small tiles (transposed)}. cursor[e] gets
+// (forward), groups, wide groups, full wide groups, -, small tiles (transposed)} and words 12 and 13, the
+// partial wide groups' runs when each is cut into two or four (a run has a tile at least). cursor[e] gets
 // offsets[e] (cursor may be counts itself: each expert's count is read before its cursor is written,
 // by the same thread). The scan is within each wave by lane moves and across the 16 waves through
 // their totals: one barrier (20 in LDS took 4 us of this latency-bound kernel's 20). With `judge` or
@@ -405,6 +406,7 @@ MX_DEV int wave_isum(int v)
 constexpr int kScan = 7;  // rows, tiles, small (forward), groups, full wide groups, partial ones, small (transposed)
 struct ScanLds {
   int tot[kScan][16];  // the waves' totals
+  int runs[2][16];     // of the partial wide groups' runs
   int judge[3][16];    // of the tiles past an expert's first, experts of kLargeMinTiles and of kGroupMinTiles tiles
 };
 struct RouteOut {
@@ -446,7 +448,7 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
     if (large == 0 && past <= o.judge) wide_min = kLargeMinTiles;
     if (large == 0 && group <= o.judge_groups) group_min = kLargeMinTiles;
   }
-  int v[kScan] = {};
+  int v[kScan] = {}, run2 = 0, run4 = 0;
   for (int e = e0; e < e1; ++e) {
     const int et = (counts[e] + kFwdRowsPerTile - 1) / kFwdRowsPerTile;
     v[0] += counts[e];
@@ -454,6 +456,8 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
     if (et >= wide_min) {
       v[4] += et / kWideGroupTiles;
       v[5] += et % kWideGroupTiles ? 1 : 0;
+      run2 += min(et % kWideGroupTiles, 2);
+      run4 += min(et % kWideGroupTiles, 4);
     } else {
       v[2] += et;
     }
@@ -470,9 +474,14 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
       const int u = __shfl_up(inc[i], d, 64);
       inc[i] += lane >= d ? u : 0;
     }
-  if (lane == 63)
+  run2 = wave_isum(run2);
+  run4 = wave_isum(run4);
+  if (lane == 63) {
 #pragma unroll
     for (int i = 0; i < kScan; ++i) lds.tot[i][wave] = inc[i];
+    lds.runs[0][wave] = run2;
+    lds.runs[1][wave] = run4;
+  }
   __syncthreads();
   int off[kScan], total[kScan];  // exclusive offsets and totals
 #pragma unroll
@@ -503,6 +512,10 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
     for (int m = 0; m < c; m += kFwdRowsPerTile) o.tiles[tile_off++] = make_int4(e, row_off + m, min(kFwdRowsPerTile, c - m), 0);
     row_off += c;
   }
+  if (wave == 15) {
+    run2 = group16_isum(lds.runs[0][lane & 15]);
+    run4 = group16_isum(lds.runs[1][lane & 15]);
+  }
   if (t == 1023) {
     o.offsets[E] = total[0];
     o.meta[0] = total[1];
@@ -511,6 +524,8 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
     o.meta[4] = total[4] + total[5];
     o.meta[5] = total[4];
     o.meta[7] = total[6];
+    o.meta[12] = run2;
+    o.meta[13] = run4;
   }
   return total[0];
 }
@@ -565,10 +580,10 @@ __global__ __launch_bounds__(1024) void route_one_kernel(const void* idx, int id
   }
   __syncthreads();
   for (int e = t; e < E; e += 1024) counts[e] = s_cnt[e];
-  // meta: the scan writes words 0, 2..5 and 7; the flags word, word 6 and words 8..15 (the products'
-  // flags and work-queue counters, which start at zero) are written here
+  // meta: the scan writes words 0, 2..5, 7, 12 and 13; the flags word, word 6 and the other words of
+  // 8..15 (the products' flags and work-queue counters, which start at zero) are written here
   if (t == 1) o.meta[1] = s_bad;
-  if (t == 6 || (t >= 8 && t < 16)) o.meta[t] = 0;
+  if (t == 6 || (t >= 8 && t < 12) || t == 14 || t == 15) o.meta[t] = 0;
   const int placed = route_scan(s_cnt, E, s_cnt, o, lds);  // pairs with a valid expert id
   __syncthreads();
   for (int p0 = 0; p0 < P; p0 += 8 * 1024) {

@@ -175,3 +175,39 @@ def test_three_tile_groups(k, rows, groups, layout):
         if rows[e]:
             assert_close(gh[idx[:, 0] == e], want[0][idx[:, 0] == e], f"grad_h of the expert with {rows[e]} rows")
     assert_close(gw, want[1], "grad_w")
+
+
+# tokens of expert 0, 1, ..: items of 12 column blocks in a grid of 256 work-groups
+@pytest.mark.parametrize("rows", (
+    (128, 129, 144, 128, 140, 130, 127, 113),  # 12 groups, 4 of one tile: 7 full ones cut in two
+    (256, 16, 33),                             # two full groups, one and three tiles: cut in four
+    (300,) * 8,                                # 24 groups, 288 items: a whole round, then partial groups only
+    (128,) * 9 + (17,),                        # full groups and one of two tiles, cut in two
+))
+@pytest.mark.parametrize("forward_layout", (False, True))
+def test_last_round_runs(k, rows, forward_layout):
+    """The last round of the wide items cut into runs of tiles where work-groups for all of these would idle:
+    the runs of the partial groups (meta words 12 and 13, at the start of the workspace) are no more than
+    their tiles."""
+    from lazylora_amd.experts import ExpertLayer
+    print(f"\n[case] {rows} forward layout {forward_layout}", flush=True)
+    E, N, D, F = len(rows), sum(rows), 512, 3072
+    rng = np.random.default_rng(N)
+    ex = oracle.random_experts(rng, E, D, F, 117, 121)
+    h = rng.standard_normal((N, D)).astype(np.float32)
+    idx = np.repeat(np.arange(E), rows)[rng.permutation(N)].reshape(N, 1)
+    w = rng.uniform(0.5, 1.0, (N, 1)).astype(np.float32)
+    L = ExpertLayer(*[torch.from_numpy(a).cuda() for a in (ex.w1p, ex.w1s, ex.w3p, ex.w3s, ex.w2p, ex.w2s)])
+    if forward_layout:
+        L.prepare_forward_layout()
+    c = lambda a: torch.from_numpy(a).cuda()
+    ws = torch.empty(k.moe_workspace_bytes(N, 1, E, D, F), dtype=torch.uint8, device="cuda")
+    got = k.routed_forward(c(h), c(idx), c(w), L, workspace=ws).cpu().numpy()
+    tiles = [-(-n // 16) for n in rows]
+    wide = [t for t in tiles if t >= (2 if forward_layout else 1)]
+    meta = ws[:64].view(torch.int32).tolist()
+    assert meta[4:6] == [sum(-(-t // 8) for t in wide), sum(t // 8 for t in wide)]
+    assert meta[12:14] == [sum(min(t % 8, n) for t in wide) for n in (2, 4)]
+    want = oracle.routed_forward(h, idx, w, ex)
+    for e, n in enumerate(rows):
+        assert_close(got[idx[:, 0] == e], want[idx[:, 0] == e], f"expert with {n} rows")
