@@ -58,13 +58,15 @@ __global__ __launch_bounds__(256) void router_topk_kernel(long long* __restrict_
   float score[PER_LANE];
   uint32_t key[PER_LANE];  // 0: absent or already chosen
   uint32_t best = 0;
-#pragma unroll
-  for (int m = 0; m < PER_LANE; ++m) {
+  // (static_for: the arrays' indices are constants from the start, so they are registers of their own and
+  // not one tuple that every branch below copies)
+  static_for<PER_LANE>([&](auto mc) {
+    constexpr int m = decltype(mc)::value;
     const int e = lane + 64 * m;
     score[m] = e < E ? row[e] : 0.f;
-  }
-#pragma unroll
-  for (int m = 0; m < PER_LANE; ++m) {
+  });
+  static_for<PER_LANE>([&](auto mc) {
+    constexpr int m = decltype(mc)::value;
     const int e = lane + 64 * m;
     key[m] = 0;
     if (e < E) {
@@ -72,7 +74,7 @@ __global__ __launch_bounds__(256) void router_topk_kernel(long long* __restrict_
       key[m] = order_key(bias ? score[m] + bias[e] : score[m]);
     }
     best = max(best, key[m]);
-  }
+  });
 
   float sum = 0.f;
   float mine = 0.f;  // lane t keeps the t-th chosen score
@@ -83,12 +85,12 @@ __global__ __launch_bounds__(256) void router_topk_kernel(long long* __restrict_
     // several lanes hold one, the lowest id
     int mm = PER_LANE;
     float s_mm = 0.f;
-#pragma unroll
-    for (int m = PER_LANE - 1; m >= 0; --m) {
+    static_for<PER_LANE>([&](auto mc) {
+      constexpr int m = PER_LANE - 1 - decltype(mc)::value;
       const bool hit = key[m] == win;
       mm = hit ? m : mm;
       s_mm = hit ? score[m] : s_mm;
-    }
+    });
     const uint64_t holders = __builtin_amdgcn_ballot_w64(best == win);
     int owner = __builtin_ctzll(holders);
     if (holders & (holders - 1)) {  // uniform, rare
@@ -102,11 +104,11 @@ __global__ __launch_bounds__(256) void router_topk_kernel(long long* __restrict_
     const float s = bits_f((uint32_t)__builtin_amdgcn_readlane((int)f_bits(s_mm), owner));  // the unbiased score
     // the owner retires it
     uint32_t nb = 0;
-#pragma unroll
-    for (int m = 0; m < PER_LANE; ++m) {
+    static_for<PER_LANE>([&](auto mc) {
+      constexpr int m = decltype(mc)::value;
       key[m] = lane == owner && m == mm ? 0u : key[m];
       nb = max(nb, key[m]);
-    }
+    });
     best = nb;
     sum += s;
     if (lane == t) {
