@@ -479,9 +479,12 @@ int moe_front(const void* h, int h_dtype, const void* idx, int idx_dtype, const 
   // tile, and the XT rows are skipped when no bucket is small (the routing's meta says so on
   // the device). Without the split every tile reads the XT rows, so they are always written.
   const bool gu_split = mx::fwd_bucket_split(F, D) && !mx::fwd_few_rows(a, mx::kFwdGateUp, L.max_tiles);
-  // Beyond top-1 they are written in any case: a token in several tiles is then quantised once and
-  // copied (1000 tokens in 16 tiles each: 97 us for its tiles, 46 with the rows).
-  const int* xt_meta = gu_split && k == 1 ? at<int>(ws, L.meta) : nullptr;
+  // From kXtMinSlots slots on they are written in any case: a token in several tiles is then quantised once
+  // and copied. 16 experts, all buckets large, us, copied / quantised for every tile, 2048 tokens of 7168 fp32:
+  // top-2 43 / 37, top-4 61 / 62, top-6 78 / 88, top-8 95 / 113, top-16 161 / 210; bf16 40 / 31, 58 / 58, 76 / 78, 93 / 96,
+  // 159 / 164; the widest case against it 8192 tokens, fp32, top-6 373 / 341 (16,384: 722 / 778).
+  constexpr int kXtMinSlots = 5;
+  const int* xt_meta = gu_split && k < kXtMinSlots ? at<int>(ws, L.meta) : nullptr;
   MX_TRY(mx::launch_quant_rows(h, h_dtype == MXFP4_BF16, D, N, D, xt_meta, at<uint8_t>(ws, L.xt_x),
                                at<uint8_t>(ws, L.x3_x), at<int>(ws, L.meta) + 6, s),
          "quantise h");

@@ -211,3 +211,28 @@ def test_last_round_runs(k, rows, forward_layout):
     want = oracle.routed_forward(h, idx, w, ex)
     for e, n in enumerate(rows):
         assert_close(got[idx[:, 0] == e], want[idx[:, 0] == e], f"expert with {n} rows")
+
+
+@pytest.mark.parametrize("topk", (2, 4, 5, 8))
+@pytest.mark.parametrize("D", (512, 1056))
+@pytest.mark.parametrize("bf16", (False, True))
+def test_only_large_buckets(k, topk, D, bf16):
+    """Every bucket large and every token in several tiles: up to four slots its tiles are quantised one by
+    one and its row in the token-major layout is not written, from five on they are copied from it (at a width
+    that the large-bucket items do not take there are no tiles). Outlier channels, whose blocks have a third
+    term."""
+    from lazylora_amd.experts import ExpertLayer
+    print(f"\n[case] top-{topk} D {D} bf16 {bf16}", flush=True)
+    E, N, F = 8, 300, 64
+    rng = np.random.default_rng(topk + D)
+    ex = oracle.random_experts(rng, E, D, F, 117, 121)
+    h = rng.standard_normal((N, D)).astype(np.float32)
+    h[:, 5::97] *= 1000.0
+    H = torch.from_numpy(h).cuda().to(torch.bfloat16 if bf16 else torch.float32)
+    idx = np.stack([(np.arange(topk) + t) % E for t in range(N)])
+    w = rng.uniform(0.5, 1.0, (N, topk)).astype(np.float32)
+    L = ExpertLayer(*[torch.from_numpy(a).cuda() for a in (ex.w1p, ex.w1s, ex.w3p, ex.w3s, ex.w2p, ex.w2s)])
+    ws = torch.empty(k.moe_workspace_bytes(N, topk, E, D, F), dtype=torch.uint8, device="cuda").random_(0, 256)
+    got = k.routed_forward(H, torch.from_numpy(idx).cuda(), torch.from_numpy(w).cuda(), L, workspace=ws)
+    assert ws[:64].view(torch.int32)[2] == 0  # no bucket is small
+    assert_close(got.cpu().numpy(), oracle.routed_forward(H.float().cpu().numpy(), idx, w, ex), "out")
