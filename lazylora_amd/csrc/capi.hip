@@ -679,7 +679,7 @@ int mxfp4_gemm_t(float* y, const float* dy, const uint8_t* packed, const uint8_t
   a.M = M;
   a.n_ct = (K + mx::kBwdColsPerTile - 1) / mx::kBwdColsPerTile;
   a.y = y; a.ldy = K; a.accumulate = 1;
-  if (M <= mx::kBwdFewRows) {
+  if (M <= mx::kBwdFewRows) {  // (the workspace is not used: it is asked for whatever the rows)
     MX_TRY(mx::launch_bwd_few(a, dy, stream), "gemm_t: product");
     return MXFP4_OK;
   }

@@ -22,8 +22,8 @@
 // waves of a work-group take four neighbouring stripes of one row tile and share its A operands:
 // the work-group copies them into LDS (global_load_lds, 16 steps at a time, double-buffered),
 // so A costs one read per 1024 columns instead of one per 256, and one barrier per 16 steps.
-// Large buckets (experts with many 16-row tiles) take items of T row tiles, which reuse every
-// decoded operand for all T tiles.
+// Large buckets (experts with many 16-row tiles) take items of four row tiles, which reuse every
+// decoded operand for all of them (bwd_group_item).
 //
 // The whole contraction range (nseg * R rows) stays in one wave, so every output element has
 // exactly one writer and the sum order is fixed: results are deterministic.
@@ -48,13 +48,10 @@ constexpr int kWaves = 4;  // waves (stripes) per work-group
 constexpr int kWideWaves = 8;
 constexpr int kWideMinItems = 512;
 
-// One work item: the NW stripes from NW * ct4 on of up to T row tiles of one expert (T = 1: a
-// small-bucket tile; T > 1: part of a large-bucket group, whose tiles share every decoded
-// operand).
-template <int T>
+// One one-tile work item: the NW stripes from NW * ct4 on of a row tile of one expert.
 struct WorkItem {
-  int expert, ct4, ntl;
-  int row0[T], nrows[T];
+  int expert, ct4;
+  int row0, nrows;
 };
 
 // The one-tile work list: the small-bucket tiles (with no large-bucket groups, every tile in
@@ -72,10 +69,9 @@ __device__ __forceinline__ int one_tile_count(const BwdArgs& a)
 // The work item of one-tile work-group `bid` among items of NW stripes (items are dealt round-robin
 // over the XCDs, bid % 8, each XCD taking one contiguous run, so the stripe blocks of one tile,
 // which read the same A rows, run on one XCD). Returns whether there is one.
-template <int T, int NW>
-__device__ __forceinline__ bool decode_work(const BwdArgs& a, int bid, WorkItem<T>& w)
+template <int NW>
+__device__ __forceinline__ bool decode_work(const BwdArgs& a, int bid, WorkItem& w)
 {
-  static_assert(T == 1, "large buckets take bwd_group_item");
   const bool use_small = use_small_list(a);
   const int count = one_tile_count(a);
   const int n_ct4 = (a.n_ct + NW - 1) / NW;
@@ -86,21 +82,16 @@ __device__ __forceinline__ bool decode_work(const BwdArgs& a, int bid, WorkItem<
   if (slot >= per_xcd || item >= total) return false;
   const int i = item / n_ct4;
   w.ct4 = item - i * n_ct4;
-  const int t0 = use_small ? ((cint_ptr)a.small_tiles)[i] : i;
-  w.ntl = 1;
-#pragma unroll
-  for (int tt = 0; tt < T; ++tt) {
-    const int t = t0 + (tt < w.ntl ? tt : 0);
-    if (a.tiles) {
-      const cint_ptr tl = (cint_ptr)(a.tiles + t);
-      w.expert = tl[0];
-      w.row0[tt] = tl[1];
-      w.nrows[tt] = tl[2];
-    } else {
-      w.expert = 0;
-      w.row0[tt] = t * kFwdRowsPerTile;
-      w.nrows[tt] = min(kFwdRowsPerTile, a.M - w.row0[tt]);
-    }
+  const int t = use_small ? ((cint_ptr)a.small_tiles)[i] : i;
+  if (a.tiles) {
+    const cint_ptr tl = (cint_ptr)(a.tiles + t);
+    w.expert = tl[0];
+    w.row0 = tl[1];
+    w.nrows = tl[2];
+  } else {
+    w.expert = 0;
+    w.row0 = t * kFwdRowsPerTile;
+    w.nrows = min(kFwdRowsPerTile, a.M - w.row0);
   }
   return true;
 }
@@ -138,26 +129,11 @@ MX_DEV void decode_pair(const StepRaw& r, const float (&sf)[8], bf16x8& b0, bf16
 }
 
 // Ring depth (steps of weights in flight per wave, each 4 KiB per wave) and A chunk (steps whose
-// A operands one LDS buffer holds: kChunk x T tiles x 2 terms x 1 KiB). T > 1 items do T times
-// the matrix work per step, so a shorter ring hides the loads. kChunk is a multiple of kRing.
-#ifndef MX_BWD_RING
-#define MX_BWD_RING 4
-#endif
-template <int T>
-struct Cfg {
-  static constexpr int kRing = MX_BWD_RING;
-  static constexpr int kChunk = 16 / T;
-  static constexpr int kChunkBytes = kChunk * T * 2 * 1024;
-};
-
-// Orders this wave's LDS writes before its later LDS reads (and the other way round): the lanes of
-// one wave exchange data through LDS without a work-group barrier (LDS operations of a wave
-// complete in order; this keeps the compiler's order).
-MX_DEV void wave_lds_fence()
-{
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
+// A operands one LDS buffer holds, 2 terms x 1 KiB each; a multiple of the ring).
+constexpr int kRing = 4;
+constexpr int kChunkSteps = 16;
+constexpr int kChunkBytes = kChunkSteps * 2 * 1024;
+static_assert(kChunkSteps % kRing == 0, "a ring pass never straddles an A chunk");
 
 // Four staged columns of the W2 transposed product: h = g . W2 (with the LoRA term) at columns col ..
 // col + 3 of pair row p, against the saved gate | up: writes the bf16 hi + lo gradients of gate and
@@ -189,13 +165,10 @@ MX_DEV float lane_f(float v, int l) { return __builtin_bit_cast(float, __builtin
 // a stripe is 4 KiB of codes read by four 16-byte loads per lane (each instruction 1 KiB
 // contiguous) and 256 B of scales read by one 8-byte load per lane, instead of eight 8-byte
 // loads from eight rows and eight scale-byte loads.
-template <int MODE, int T, bool BL, int NW>
-__device__ __forceinline__ void bwd_item(const BwdArgs& a, const WorkItem<T>& w, uint8_t* abuf)
+template <int MODE, bool BL, int NW>
+__device__ __forceinline__ void bwd_item(const BwdArgs& a, const WorkItem& w, uint8_t* abuf)
 {
-  constexpr int kRing = Cfg<T>::kRing;
-  constexpr int kChunk = Cfg<T>::kChunk;
-  constexpr int kChunkBytes = Cfg<T>::kChunkBytes;
-  static_assert(kChunk % kRing == 0, "a ring pass never straddles an A chunk");
+  constexpr int kChunk = kChunkSteps;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, g = lane >> 4;
@@ -269,45 +242,32 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, const WorkItem<T>& w,
   constexpr int kStepLoads = BL ? 5 : 16;  // load instructions per step and lane
 
   // A operands: MFMA lane (i = n, g) takes elements 8g..8g+7 of the step's 32 contraction
-  // indices of row i of each tile, hi and lo terms (16 bytes each). The work-group copies them
-  // into abuf chunk by chunk: unit u = (step in chunk, tile, term) is 1 KiB, lane l's operand at
+  // indices of row i of the tile, hi and lo terms (16 bytes each). The work-group copies them
+  // into abuf chunk by chunk: unit u = (step in chunk, term) is 1 KiB, lane l's operand at
   // 16 l, exactly as a ds_read_b128 of the MFMA lanes wants it; wave w copies units w, w + 4, ...
   // Rows past a tile's end repeat its last row (never stored). Padding steps meet zero weights,
   // so their A (the last real step's, copied again) adds zero.
-  const uint16_t* pa[T][2];
-#pragma unroll
-  for (int tt = 0; tt < T; ++tt) {
-    const int ri = w.row0[tt] + min(n, w.nrows[tt] - 1);
-    const long long arow = a.a_row_map ? a.a_row_map[ri] : ri;
-    pa[tt][0] = a.a_hi + arow * a.lda + 8 * g;
-    pa[tt][1] = a.a_lo + arow * a.lda + 8 * g;
-  }
+  const int ri = w.row0 + min(n, w.nrows - 1);
+  const long long arow = a.a_row_map ? a.a_row_map[ri] : ri;
+  const uint16_t* const pa_hi = a.a_hi + arow * a.lda + 8 * g;
+  const uint16_t* const pa_lo = a.a_lo + arow * a.lda + 8 * g;
   // The copies are issued from inline assembly (the compiler does not see them, so it does not
   // drain every load in flight at each barrier); each chunk is waited for explicitly.
   auto copy_chunk = [&](int chunk) {
     uint8_t* dst = abuf + (chunk & 1) * kChunkBytes;
-    static_assert(kChunk * T * 2 % NW == 0, "the A units split evenly over the waves");
+    static_assert(kChunk * 2 % NW == 0, "the A units split evenly over the waves");
 #pragma unroll
-    for (int k = 0; k < kChunk * T * 2 / NW; ++k) {
+    for (int k = 0; k < kChunk * 2 / NW; ++k) {
       const int u = k * NW + wave;
-      const int si = u / (2 * T), tt = (u >> 1) % T, term = u & 1;
-      const int so = min(chunk * kChunk + si, nsteps - 1) * kStepRows;
-      // select tile tt's pointer without indexing (keeps pa in registers)
-      const uint16_t* src = pa[0][0];
-#pragma unroll
-      for (int t2 = 0; t2 < T; ++t2)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          if (tt == t2 && term == h) src = pa[t2][h];
+      const int so = min(chunk * kChunk + u / 2, nsteps - 1) * kStepRows;
+      const uint16_t* src = (u & 1) ? pa_lo : pa_hi;
       dma16_async(src + so, dst + u * 1024);
     }
   };
 
-  f32x4 acc[T][16];
+  f32x4 acc[16];
 #pragma unroll
-  for (int tt = 0; tt < T; ++tt)
-#pragma unroll
-    for (int t = 0; t < 16; ++t) acc[tt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < 16; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   StepRaw ring[kRing];
   // issue order is pinned (the first A chunk, then the ring slot by slot) so that each step
@@ -339,12 +299,8 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, const WorkItem<T>& w,
       const int si = s % kChunk;
       StepRaw& r = ring[p];
       // this step's A operands from the chunk in LDS
-      i32x4 ah[T], al[T];
-#pragma unroll
-      for (int tt = 0; tt < T; ++tt) {
-        ah[tt] = *reinterpret_cast<const i32x4*>(ab + ((si * T + tt) * 2) * 1024);
-        al[tt] = *reinterpret_cast<const i32x4*>(ab + ((si * T + tt) * 2 + 1) * 1024);
-      }
+      const i32x4 ah = *reinterpret_cast<const i32x4*>(ab + si * 2 * 1024);
+      const i32x4 al = *reinterpret_cast<const i32x4*>(ab + (si * 2 + 1) * 1024);
       // scales of this step's rows as E8M0 operands of the conversion; a scale byte >= 253
       // makes its row contribute zero
       float sf[8];
@@ -363,17 +319,11 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, const WorkItem<T>& w,
         decode_pair<p2>(r, sf, b[0], b[1]);
         decode_pair<p2 + 1>(r, sf, b[2], b[3]);
 #pragma unroll
-        for (int tt = 0; tt < T; ++tt)
-          if (tt < w.ntl)
+        for (int j = 0; j < 4; ++j)
+          acc[2 * p2 + j] = mfma_bf16(__builtin_bit_cast(bf16x8, ah), b[j], acc[2 * p2 + j]);
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-              acc[tt][2 * p2 + j] = mfma_bf16(__builtin_bit_cast(bf16x8, ah[tt]), b[j], acc[tt][2 * p2 + j]);
-#pragma unroll
-        for (int tt = 0; tt < T; ++tt)
-          if (tt < w.ntl)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              acc[tt][2 * p2 + j] = mfma_bf16(__builtin_bit_cast(bf16x8, al[tt]), b[j], acc[tt][2 * p2 + j]);
+        for (int j = 0; j < 4; ++j)
+          acc[2 * p2 + j] = mfma_bf16(__builtin_bit_cast(bf16x8, al), b[j], acc[2 * p2 + j]);
       };
       bytes(std::integral_constant<int, 0>{});
       bytes(std::integral_constant<int, 2>{});
@@ -394,13 +344,12 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, const WorkItem<T>& w,
   // lanes of one LDS pass hit all banks. With the grouped kernel's the same way: W2 transposed of
   // 16,000 pairs in large buckets (3584 x 3072, SiTU) 1.07 -> 0.90 ms, the Zipf
   // step 3.10 -> 3.00 ms; uniform buckets of 9 rows unchanged (bound by the weights).
-  static_assert(T == 1, "one tile per item");
   static_assert(NW * 8192 <= 2 * kChunkBytes, "the staged rows fit the A buffers");
   __syncthreads();  // every wave is done with the last chunk's A operands
   f32x4* const stage = reinterpret_cast<f32x4*>(abuf + wave * 8192);
   const int lcol = c0 + 4 * lane;
   const bool lcol_ok = stripe_ok && lcol < a.C;  // C is a multiple of 32: all 4 columns or none
-  const int row0 = w.row0[0], nrows = stripe_ok ? w.nrows[0] : 0;
+  const int row0 = w.row0, nrows = stripe_ok ? w.nrows : 0;
   static_for<2>([&](auto hc) {
     constexpr int half = decltype(hc)::value;
     if ((g >> 1) == half)
@@ -409,7 +358,7 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, const WorkItem<T>& w,
 #pragma unroll
         for (int c4 = 0; c4 < 4; ++c4)
           stage[((g & 1) * 4 + v) * 64 + 4 * n + (c4 ^ ((n >> 1) & 3))] =
-              f32x4{acc[0][4 * c4][v], acc[0][4 * c4 + 1][v], acc[0][4 * c4 + 2][v], acc[0][4 * c4 + 3][v]};
+              f32x4{acc[4 * c4][v], acc[4 * c4 + 1][v], acc[4 * c4 + 2][v], acc[4 * c4 + 3][v]};
     wave_lds_fence();
     const int left = nrows - 8 * half;
     auto staged = [&](int r) { return stage[r * 64 + (lane ^ ((lane >> 3) & 3))]; };
@@ -457,38 +406,24 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, const WorkItem<T>& w,
 
 // ---------------------------------------------------------------- large buckets
 // An expert with many rows would stream (and decode) its weights once per row tile. Its tiles
-// come in groups of up to kGroupTiles (4) consecutive tiles; a work item is GT of them (a part of
-// a group when GT is smaller) x a block of 4 GS columns: every wave decodes a GS-column stripe of
-// each 32-row step once and applies it to all GT row tiles, and the item's A operands (GT tiles x
-// hi/lo, 2 GT KiB per step) come through LDS for the four waves. Each weight byte is read once per 16 GT rows
-// instead of once per 16, and each A fragment read from LDS feeds GS / 16 MFMAs.
+// come in groups of up to kGroupTiles (4) consecutive tiles; a work item is one group x a block of
+// 512 columns: every wave decodes a 128-column stripe of each 32-row step once and applies it to all
+// four row tiles, and the item's A operands (4 tiles x hi/lo, 8 KiB per step) come through LDS for the
+// four waves. Each weight byte is read once per 64 rows instead of once per 16, and each A fragment
+// read from LDS feeds 8 MFMAs.
 //
-// Lane (n, g) of a wave holds columns (GS / 16) n .. + GS / 16 - 1 of its stripe, whose weights
-// are GS / 32 bytes of each of its 8 rows: with GS = 128 the lane's own dword, with GS = 64 half
-// of the dword its lane pair shares. Byte p gives MFMAs 2p and 2p + 1. Scales come as the dword
-// holding the lane's scale byte, so the kernel requires C % 128 == 0 (whole dwords of scales per
-// row); launch_bwd sends other shapes through the one-tile kernel.
-#ifndef MX_BWD_GT
-#define MX_BWD_GT 4
-#endif
-#ifndef MX_BWD_GS
-#define MX_BWD_GS 128
-#endif
-#ifndef MX_BWD_GRING
-#define MX_BWD_GRING 2
-#endif
-#ifndef MX_BWD_GPER_CU
-#define MX_BWD_GPER_CU 2
-#endif
-constexpr int kGT = MX_BWD_GT;                // row tiles per item
-constexpr int kGS = MX_BWD_GS;                // columns per wave
-constexpr int kGParts = kGroupTiles / kGT;    // items per group and column block
-constexpr int kGCols = kWaves * kGS;          // columns per item
-constexpr int kGRing = MX_BWD_GRING;          // steps of weights in flight per wave
-constexpr int kGChunk = MX_BWD_GRING;         // steps per LDS A chunk (a multiple of kGRing)
-constexpr int kGUnit = 1024;                  // one tile x one term x one step of A
+// Lane (n, g) of a wave holds columns 8n .. 8n + 7 of its stripe, whose weights are its own dword of
+// each of its 8 rows. Byte p gives MFMAs 2p and 2p + 1. Scales come as the dword holding the lane's
+// scale byte, so the kernel requires C % 128 == 0 (whole dwords of scales per row); launch_bwd sends
+// other shapes through the one-tile items.
+constexpr int kGT = kGroupTiles;      // row tiles per item
+constexpr int kGS = 128;              // columns per wave
+constexpr int kGCols = kWaves * kGS;  // columns per item
+constexpr int kGRing = 2;             // steps of weights in flight per wave
+constexpr int kGChunk = 2;            // steps per LDS A chunk (a multiple of kGRing)
+constexpr int kGPerCu = 2;            // work-groups per CU
+constexpr int kGUnit = 1024;          // one tile x one term x one step of A
 constexpr int kGChunkBytes = kGChunk * kGT * 2 * kGUnit;
-constexpr int kGBytes = kGS / 32;             // weight bytes per row and lane
 static_assert(kGCols % kBwdColsPerTile == 0, "an item covers whole 256-column grad_w partials");
 
 struct GStep {
@@ -690,7 +625,7 @@ __device__ __forceinline__ void bwd_group_item(const BwdArgs& a, int expert, int
         constexpr int P = decltype(pc)::value;
         gdecode_pair<P>(wl, sf, b[2 * P], b[2 * P + 1]);
       });
-      // every tile slot computes (a short part's empty slots work on copies of its first tile's
+      // every tile slot computes (a short group's empty slots work on copies of its first tile's
       // rows and are never stored): no branch, so the A reads of the next tiles are issued while
       // the MFMAs of the current ones run
 #pragma unroll
@@ -788,7 +723,7 @@ __device__ __forceinline__ void bwd_group_item(const BwdArgs& a, int expert, int
 }
 
 // Both bucket kinds in one launch. The first `gblocks` work-groups (a multiple of 8; 0 without a
-// bucket split) are a resident grid over the large-bucket items (group, part, column block), dealt
+// bucket split) are a resident grid over the large-bucket items (group, column block), dealt
 // round-robin over the XCDs like the one-tile items: the longer items start first and the one-tile
 // items fill the slots beside and behind them (128 tokens, top-16 of 64 experts, 3584 / 3072: the
 // two transposed products 0.32 and 0.46 ms in two launches each, 0.20 and 0.38 in one), and a routing without large buckets
@@ -797,37 +732,32 @@ __device__ __forceinline__ void bwd_group_item(const BwdArgs& a, int expert, int
 // (bwd_wide_kernel) and run only when there are fewer than kWideMinItems eight-stripe items. BL:
 // the weights come from the backward layout.
 template <int MODE, bool BL>
-__global__ __launch_bounds__(64 * kWaves, MX_BWD_GPER_CU) void bwd_kernel(BwdArgs a, int wide, int gblocks)
+__global__ __launch_bounds__(64 * kWaves, kGPerCu) void bwd_kernel(BwdArgs a, int wide, int gblocks)
 {
-  static_assert(2 * kGChunkBytes <= 2 * Cfg<1>::kChunkBytes, "the A buffers serve both kinds");
-  __shared__ __attribute__((aligned(16))) uint8_t abuf[2 * Cfg<1>::kChunkBytes];
+  static_assert(2 * kGChunkBytes <= 2 * kChunkBytes, "the A buffers serve both kinds");
+  __shared__ __attribute__((aligned(16))) uint8_t abuf[2 * kChunkBytes];
   if constexpr (MODE != kBwdPlain) {
     if ((int)blockIdx.x < gblocks) {
       __shared__ float red[kWaves * kGT * 16];
       const int ng = *(cint_ptr)a.n_groups;
       const int ncb = (a.C + kGCols - 1) / kGCols;
-      const int total = ng * kGParts * ncb;
+      const int total = ng * ncb;
       const int per_xcd = (total + 7) >> 3;
-      bool busy = false;
       for (int it = 0;; ++it) {
         const int slot = (int)(blockIdx.x >> 3) + it * (gblocks >> 3);
         const int item = (int)(blockIdx.x & 7) * per_xcd + slot;
         if (slot >= per_xcd || item >= total) break;
-        const int gp = item / ncb, cb = item - gp * ncb;
-        const int gi = gp / kGParts, part = gp - gi * kGParts;
+        const int gi = item / ncb, cb = item - gi * ncb;
         const cint_ptr gg = (cint_ptr)(a.groups + gi);
-        const int ntl = gg[2] - part * kGT;
-        if (ntl <= 0) continue;  // the empty part of a short group
-        if (busy) __syncthreads();  // every wave has finished reading the previous item's LDS
-        bwd_group_item<MODE, BL>(a, gg[0], gg[1] + part * kGT, min(ntl, kGT), cb, abuf, red);
-        busy = true;
+        if (it > 0) __syncthreads();  // every wave has finished reading the previous item's LDS
+        bwd_group_item<MODE, BL>(a, gg[0], gg[1], gg[2], cb, abuf, red);
       }
       return;
     }
   }
   if (wide && one_tile_count(a) * ((a.n_ct + kWideWaves - 1) / kWideWaves) >= kWideMinItems) return;
-  WorkItem<1> w;
-  if (decode_work<1, kWaves>(a, (int)blockIdx.x - gblocks, w)) bwd_item<MODE, 1, BL, kWaves>(a, w, abuf);
+  WorkItem w;
+  if (decode_work<kWaves>(a, (int)blockIdx.x - gblocks, w)) bwd_item<MODE, BL, kWaves>(a, w, abuf);
 }
 
 // The one-tile items with eight stripes (one work-group per CU; the grid covers every item); it runs
@@ -835,10 +765,10 @@ __global__ __launch_bounds__(64 * kWaves, MX_BWD_GPER_CU) void bwd_kernel(BwdArg
 template <int MODE, bool BL>
 __global__ __launch_bounds__(64 * kWideWaves, 1) void bwd_wide_kernel(BwdArgs a)
 {
-  __shared__ __attribute__((aligned(16))) uint8_t abuf[2 * Cfg<1>::kChunkBytes];
+  __shared__ __attribute__((aligned(16))) uint8_t abuf[2 * kChunkBytes];
   if (one_tile_count(a) * ((a.n_ct + kWideWaves - 1) / kWideWaves) < kWideMinItems) return;
-  WorkItem<1> w;
-  if (decode_work<1, kWideWaves>(a, (int)blockIdx.x, w)) bwd_item<MODE, 1, BL, kWideWaves>(a, w, abuf);
+  WorkItem w;
+  if (decode_work<kWideWaves>(a, (int)blockIdx.x, w)) bwd_item<MODE, BL, kWideWaves>(a, w, abuf);
 }
 
 // ---------------------------------------------------------------- few rows
@@ -1017,8 +947,8 @@ hipError_t launch_bwd(const BwdArgs& a, int mode, int max_tiles, hipStream_t s)
   // groups come from experts with more than two tiles: at most one per 32 rows (one from 33, two from 65)
   long long gblocks = 0;
   if (split) {
-    const long long gtotal = (long long)(a.M / 32) * kGParts * ((a.C + kGCols - 1) / kGCols);
-    gblocks = std::min<long long>((gtotal + 7) / 8 * 8, resident_groups(MX_BWD_GPER_CU));
+    const long long gtotal = (long long)(a.M / 32) * ((a.C + kGCols - 1) / kGCols);
+    gblocks = std::min<long long>((gtotal + 7) / 8 * 8, resident_groups(kGPerCu));
   }
   dim3 grid((unsigned)(gblocks + blocks)), block(64 * kWaves);
 #define MX_LAUNCH(M, L) hipLaunchKernelGGL((bwd_kernel<M, L>), grid, block, 0, s, b, wide, (int)gblocks)
@@ -1039,7 +969,8 @@ hipError_t launch_bwd(const BwdArgs& a, int mode, int max_tiles, hipStream_t s)
 // left; four spill. Measured against the split pass + bwd_kernel (us, M = 1 / 22 / 100 / 256):
 // W [2048, 7168] 46 / 50 / 52 / 54 -> 15 / 15 / 28 / 43, [3072, 3584] 66 / 71 / 72 / 74 -> 18 / 20 /
 // 20 / 38, [7168, 2048] 146 / 150 / 153 / 157 -> 39 / 41 / 39 / 42, [7168, 7168] 147 / 150 / 155 /
-// 159 -> 43 / 47 / 91 / 137; the lines meet between 256 and 512 rows.
+// 159 -> 43 / 47 / 91 / 137. kBwdFewRows is as far as every shape was measured; the lines meet further out
+// (before 512 rows).
 constexpr int kFewMinGroups = 256;
 hipError_t launch_bwd_few(const BwdArgs& a, const float* x, hipStream_t s)
 {

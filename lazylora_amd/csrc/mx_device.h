@@ -390,16 +390,6 @@ MX_DEV void dma16_async_s(const void* base, uint32_t voff, void* lds)
   const uint64_t bs = ((uint64_t)bhi << 32) | blo;
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(bs), "s"(m0) : "memory");
 }
-// dma16_async_s with the streaming (nt) hint, for bytes each copied exactly once, by whole lines.
-MX_DEV void dma16_async_s_nt(const void* base, uint32_t voff, void* lds)
-{
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(
-      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds);
-  const uint64_t b = (uint64_t)(uintptr_t)base;
-  const uint32_t blo = __builtin_amdgcn_readfirstlane((uint32_t)b), bhi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
-  const uint64_t bs = ((uint64_t)bhi << 32) | blo;
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(bs), "s"(m0) : "memory");
-}
 // The 4-byte form (global_load_lds_dword): lane l's 4 bytes land at lds + 4 l.
 MX_DEV void dma4_async(const void* src, void* lds)
 {
@@ -441,6 +431,15 @@ MX_DEV void queue_leave(int* counter)
     atomicExch(counter, 0);
     atomicExch(counter + 1, 0);
   }
+}
+
+// Orders this wave's LDS writes before its later LDS reads (and the other way round): the lanes of
+// one wave exchange data through LDS without a work-group barrier (LDS operations of a wave
+// complete in order; this keeps the compiler's order).
+MX_DEV void wave_lds_fence()
+{
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
 // bf16 helpers (round to nearest even, as v_cvt_pk_bf16_f32 does)

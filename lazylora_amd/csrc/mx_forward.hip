@@ -413,14 +413,6 @@ __device__ __forceinline__ void epilogue_direct(const FwdArgs& a, const WorkItem
 }
 
 
-// Orders this wave's LDS writes before its later LDS reads (and the other way round): the lanes of
-// one wave exchange data through LDS without a work-group barrier.
-__device__ __forceinline__ void wave_lds_fence()
-{
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // Epilogue of one wave's tile through 8 KiB of LDS of its own (st; no work-group barrier): the same
 // results as epilogue_direct, written as 16-byte pieces that cover 128- or 256-byte runs instead of
 // single bytes and dwords (16 and 16 store instructions for a tile's act codes and gate | up, 16 for
@@ -827,21 +819,21 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const WorkItem& w, in
   if (w.active) epilogue_direct<MODE>(a, w, lane, acc, tw);
 }
 
-template <int MODE, bool FAST, bool FL, int NW = kWavesPerGroup>
-__global__ __launch_bounds__(64 * NW, NW == kWavesPerGroup ? 2 : 1) void fwd_kernel(FwdArgs a)
+template <int MODE, bool FAST, bool FL>
+__global__ __launch_bounds__(64 * kWavesPerGroup, 2) void fwd_kernel(FwdArgs a)
 {
   __shared__ FwdLds lds;  // used by the fast path only
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: keeps control flow scalar
   WorkItem w;
-  for (int it = 0; decode_work(a.tiles, a.n_tiles, a.small_tiles, a.n_small, a.n_wgroups, a.M, a.n_ct, wave, it, w, NW); ++it) {
+  for (int it = 0; decode_work(a.tiles, a.n_tiles, a.small_tiles, a.n_small, a.n_wgroups, a.M, a.n_ct, wave, it, w); ++it) {
     // the previous item's reads of LDS are complete before this item's copies land there;
     // its output stores drain while this item's first loads are in flight
     if (FAST && it > 0) __syncthreads();
     // recompute lane-derived addresses per item instead of holding them across items
     int l = lane;
     asm volatile("" : "+v"(l));
-    fwd_item<MODE, FAST, FL, NW>(a, w, wave, l, lds);
+    fwd_item<MODE, FAST, FL>(a, w, wave, l, lds);
   }
 }
 
@@ -1190,7 +1182,7 @@ __global__ __launch_bounds__(64 * kWgWaves, 1) void fwd_wide_kernel(FwdArgs a)
 
 // Both bucket kinds of a routed product from the forward layout in one launch of eight-wave
 // work-groups (one per CU, the shape of both kernels above): each work-group runs its one-tile
-// items (fwd_kernel<MODE, true, true, 8>) and then takes large-bucket items from the work queue
+// items (of eight column tiles) and then takes large-bucket items from the work queue
 // (fwd_wide_kernel), so the large items fill the slots that the one-tile items' last round leaves
 // idle, and a routing without large buckets pays for no second launch. Same items, same
 // arithmetic: the results are those of the two launches.
@@ -1486,7 +1478,7 @@ static hipError_t launch_fwd_split_routed(const FwdArgs& a, int mode, int max_ti
 // tiles: measured against fwd_kernel, quantisation included (us, M = 1 / 16 / 48 / 100 / 256):
 // [2048, 7168] 38 / 39 / 39 / 40 / 41 before, 13 / 13 / 16 / 20 / 27 here; [7168, 2048] 18 / 19 /
 // 19 / 21 / 30, 11 / 11 / 16 / 18 / 29; [7168, 7168] 38 / 39 / 40 / 43 / 76, 17 / 18 / 29 / 37 / 65;
-// the lines meet at about 400 rows.
+// that is as far as every shape was measured, the lines meet further out (at about 400 rows).
 constexpr int kSplitMinGroups = 192;
 constexpr int kSplitMaxTiles = 16;
 static hipError_t launch_fwd_split_plain(const FwdArgs& a, hipStream_t s)
@@ -1513,7 +1505,7 @@ hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s)
   if (mode == kFwdPlain && max_tiles <= kSplitMaxTiles && (long long)a.R * (a.K / 2) < (1LL << 32))
     return launch_fwd_split_plain(a, s);
   const long long blocks = std::min<long long>((total + 7) / 8 * 8, resident_groups());
-  // the down product from the forward layout: eight column tiles per work-group, one per CU
+  // both bucket kinds from the forward layout: eight column tiles per work-group, one per CU
   const long long n_cg8 = (a.n_ct + 7) / 8;
   const long long blocks8 = std::min<long long>(((long long)max_tiles * n_cg8 + 7) / 8 * 8, resident_groups() / 16 * 8);
   const bool fast = fast_path(a.R, a.K);
@@ -1540,15 +1532,11 @@ hipError_t launch_fwd(const FwdArgs& a, int mode, int max_tiles, hipStream_t s)
     else hipLaunchKernelGGL((fwd_fused_kernel<kFwdDown>), dim3((unsigned)blocks8), dim3(512), 0, s, b);
     return hipGetLastError();
   } else if (mode == kFwdGateUp) {
-    if (fl && a.n_ct % 8 == 0)
-      hipLaunchKernelGGL((fwd_kernel<kFwdGateUp, true, true, 8>), dim3((unsigned)blocks8), dim3(512), 0, s, b);
-    else if (fl) MX_LAUNCH(kFwdGateUp, true, true);
+    if (fl) MX_LAUNCH(kFwdGateUp, true, true);
     else if (fast) MX_LAUNCH(kFwdGateUp, true, false);
     else MX_LAUNCH(kFwdGateUp, false, false);
   } else {
-    if (fl && a.n_ct % 8 == 0)
-      hipLaunchKernelGGL((fwd_kernel<kFwdDown, true, true, 8>), dim3((unsigned)blocks8), dim3(512), 0, s, b);
-    else if (fl) MX_LAUNCH(kFwdDown, true, true);
+    if (fl) MX_LAUNCH(kFwdDown, true, true);
     else if (fast) MX_LAUNCH(kFwdDown, true, false);
     else MX_LAUNCH(kFwdDown, false, false);
   }

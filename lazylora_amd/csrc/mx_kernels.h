@@ -30,7 +30,7 @@ struct FwdArgs {
   const uint8_t* a_rows;
   long long a_row_bytes;
   int a_zero_row;
-  // work: tiles[t] = {expert, first row, row count <= 16, 1 in a large bucket}; null = dense, rows 16t.. of M
+  // work: tiles[t] = {expert, first row, row count <= 16, 0}; null = dense, rows 16t.. of M
   const int4* tiles;
   const int* n_tiles;
   int M;  // rows: all of them, or with a tile list at most

@@ -92,7 +92,6 @@ MX_DEV void quant_tile_chunk(const void* x, long long ldx, int rows, int K, int 
                              const int* row_map, const uint8_t* xt, const int* meta, uint8_t* out, uint8_t* x3,
                              int* x3_any, uint8_t* chunk)
 {
-  const int nsc = at_nchunks(K);
   const int i = threadIdx.x >> 4;
   const long long cbase = (long long)c * kAtChunkBytes;  // at_*_off are tile-relative
   if (xt && !(meta && meta[2] == 0 && meta[4] > 0)) {
