@@ -273,7 +273,8 @@ int check_moe_args(const void* h, int h_dtype, const void* idx, int idx_dtype, c
     if (!wts[i]) return fail(MXFP4_EINVAL, "moe: null expert weight pointer%s");
     if (!aligned16(wts[i])) return fail(MXFP4_EINVAL, "moe: packed weights and scales must be 16-byte aligned%s");
   }
-  // the activation quantisers read h two elements at a time
+  // the activation quantisers read h eight elements at a time, copied out byte for byte (no vector
+  // dereference), so that 8 and 4 bytes are enough
   if (N > 0 && ((uintptr_t)h & (h_dtype == MXFP4_BF16 ? 3 : 7)))
     return fail(MXFP4_EINVAL, "moe: h must be 8-byte (fp32) or 4-byte (bf16) aligned%s");
   if ((long long)N * k > (1ll << 30)) return fail(MXFP4_EINVAL, "moe: too many (token, slot) pairs%s");

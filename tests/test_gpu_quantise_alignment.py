@@ -1,7 +1,8 @@
 """The quantisers read x in 32-byte (fp32) and 16-byte (bf16) pieces, and x need only be 8- and 4-byte
 aligned: the routed forward at the C entry with x at such addresses, at widths around a super-chunk,
 with outlier channels (third terms), token rows and bucket tiles alike, bit for bit the result from
-an aligned x."""
+an aligned x. The single-matrix products likewise: x at every 8 bytes, and the transposed product's
+gradient, which it reads in 32-byte pieces or splits in a pass of its own, at every 4."""
 import numpy as np
 import pytest
 import torch
@@ -49,3 +50,29 @@ def test_offsets(k, D, E, N, topk, bf16):
         outs.append(out)
     for off, out in zip((2, 4, 6), outs[1:]):
         assert torch.equal(out, outs[0]), off
+
+
+@pytest.mark.parametrize("M", (1, 17, 256, 257))  # both sides of the products' few-row kernels
+@pytest.mark.parametrize("R,K", ((512, 96), (500, 512), (96, 1056)))
+def test_product_offsets(k, R, K, M):
+    print(f"\n[case] M {M} R {R} K {K}", flush=True)
+    rng = np.random.default_rng(M + R + K)
+    packed, scales = (torch.from_numpy(a).cuda() for a in (rng.integers(0, 256, (R, K // 2), dtype=np.uint8),
+                                                           rng.integers(117, 122, (R, K // 32), dtype=np.uint8)))
+    stream = torch.cuda.current_stream().cuda_stream
+    for name, n_in, n_out, step in (("gemm", K, R, 2), ("gemm_t", R, K, 1)):
+        x = torch.from_numpy(rng.standard_normal((M, n_in)).astype(np.float32)).cuda()
+        nws = int(getattr(k.lib, f"mxfp4_{name}_workspace_size")(M, K, R))
+        outs = []
+        for off in range(0, 8, step):  # elements of 4 bytes
+            buf = torch.zeros(M * n_in + 16, dtype=torch.float32, device="cuda")
+            buf[off:off + M * n_in] = x.reshape(-1)
+            ws = torch.empty(nws, dtype=torch.uint8, device="cuda")
+            y = torch.zeros((M, n_out), dtype=torch.float32, device="cuda")
+            rc = getattr(k.lib, f"mxfp4_{name}")(y.data_ptr(), buf.data_ptr() + 4 * off, packed.data_ptr(),
+                                                 scales.data_ptr(), M, K, R, ws.data_ptr(), nws, stream)
+            assert rc == 0
+            outs.append(y)
+        assert torch.isfinite(outs[0]).all() and outs[0].abs().max() > 0
+        for off, y in zip(range(step, 8, step), outs[1:]):
+            assert torch.equal(y, outs[0]), (name, off)
