@@ -426,6 +426,7 @@ struct RouteOut {
   int4* wgroups;
   int* meta;
   int wide_min, group_min, judge, judge_groups;
+  bool runs;  // there may be wide groups
 };
 __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor, const RouteOut& o, ScanLds& lds)
 {
@@ -482,8 +483,10 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
       const int u = __shfl_up(inc[i], d, 64);
       inc[i] += lane >= d ? u : 0;
     }
-  run2 = wave_isum(run2);
-  run4 = wave_isum(run4);
+  if (o.runs) {  // uniform
+    run2 = wave_isum(run2);
+    run4 = wave_isum(run4);
+  }
   if (lane == 63) {
 #pragma unroll
     for (int i = 0; i < kScan; ++i) lds.tot[i][wave] = inc[i];
@@ -520,7 +523,7 @@ __device__ __forceinline__ int route_scan(const int* counts, int E, int* cursor,
     for (int m = 0; m < c; m += kFwdRowsPerTile) o.tiles[tile_off++] = make_int4(e, row_off + m, min(kFwdRowsPerTile, c - m), 0);
     row_off += c;
   }
-  if (wave == 15) {
+  if (o.runs && wave == 15) {
     run2 = group16_isum(lds.runs[0][lane & 15]);
     run4 = group16_isum(lds.runs[1][lane & 15]);
   }
@@ -841,7 +844,7 @@ hipError_t launch_route(const void* topk_idx, int idx64, const float* topk_w, in
 {
   const int P = N * k;
   const RouteOut o{offsets, tiles, small_tiles, bsmall_tiles, groups, wgroups, meta, wide_min, group_min, judge,
-                   judge_groups};
+                   judge_groups, wide_min < kLargeMinTiles || P > (kLargeMinTiles - 1) * kFwdRowsPerTile};
   if (P <= kRouteOneP && E <= kRouteOneE) {
     hipLaunchKernelGGL(route_one_kernel, dim3(1), dim3(1024), 0, s, topk_idx, idx64, topk_w, P, k, E, counts, o,
                        pair_token, pair_w, pair_of);
