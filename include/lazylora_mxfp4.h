@@ -199,7 +199,9 @@ int mxfp4_backward_layout(uint8_t *dst, const uint8_t *packed, const uint8_t *sc
  * MXFP4_MOE_BWD_LAYOUT in flags the array holds 6 pointers: those 3, then the
  * mxfp4_backward_layout of w1p, w3p, w2p (again W1 and W3 both or neither; W1 and W3 need D a
  * multiple of 256, W2 needs F a multiple of 256), which the backward's transposed products read
- * (the forward ignores them). Results are bit-identical to the calls without layouts; w1p..w2s
+ * (the forward ignores them). The transposed products' results are bit-identical to those without
+ * layouts, and so are the forward products' where an expert's rows go tile by tile both ways; for
+ * large buckets and for calls of a few pairs the layout sets the order of their fp32 sums. w1p..w2s
  * are still read where a product has no layout copy. */
 int mxfp4_moe_forward_fl(float *out, const void *h, int h_dtype, const void *topk_idx,
                          int idx_dtype, const float *topk_w, int N, int k, const uint8_t *w1p,

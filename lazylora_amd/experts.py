@@ -99,9 +99,10 @@ class ExpertLayer:
 
     def prepare_forward_layout(self) -> int:
         """Builds the forward-layout copies of W1, W3 (when D is a multiple of 512) and W2 (when F
-        is), which the routed forward's small-bucket work-groups then read with whole 1 KiB loads
+        is), which the routed forward then reads with whole 1 KiB loads
         of codes and whole-line loads of scales (mxfp4_forward_layout; results are
-        bit-identical). Each copy holds the packed codes and E8M0 scales it copies with the rows
+        bit-identical where both ways take one-tile items, and differ in the order of fp32 sums
+        where they take others: large buckets, and calls of a few pairs). Each copy holds the packed codes and E8M0 scales it copies with the rows
         padded to a multiple of 16 (ceil(R / 16) * 16 * (K / 2 + K / 32) bytes per expert: the
         same size when R is a multiple of 16); returns the bytes added.
 
@@ -131,8 +132,8 @@ class ExpertLayer:
         """Builds the backward-layout copies of W1, W3 (when D is a multiple of 256) and W2 (when
         F is), which the routed backward's transposed products then read with four 1 KiB loads
         of codes and one 512-byte load of scales per wave and 32-row step (sixteen loads of
-        pieces of eight rows otherwise; mxfp4_backward_layout; results are bit-identical). Each copy holds the codes and scales it copies: R * (K / 2 + K / 32)
-        bytes per expert; returns the bytes added. Stale copies are detected and dropped like
+        pieces of eight rows otherwise; mxfp4_backward_layout; results are bit-identical). Each
+        copy holds the codes and scales it copies: R * (K / 2 + K / 32) bytes per expert; returns the bytes added. Stale copies are detected and dropped like
         the forward layout's (prepare_forward_layout)."""
         from lazylora_amd.native import kernel
 

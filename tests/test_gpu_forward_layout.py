@@ -1,9 +1,9 @@
 """The forward layout (mxfp4_forward_layout, ExpertLayer.prepare_forward_layout): its bytes
 against a NumPy construction from the definition in include/lazylora_mxfp4.h, and the routed
 layer with it against the same layer without it. The one-tile forward work-groups read the same
-code bytes from either layout, in the same order, so every result is bit-identical, at small
-shapes (uniform routing, large buckets, LoRA, only W1|W3 laid out) and at the BASELINE config-4
-size."""
+code bytes from either layout, in the same order, so their results are bit-identical; large
+buckets sum in another order and agree to rounding. At small shapes (uniform routing, large
+buckets, LoRA, only W1|W3 laid out) and at the BASELINE config-4 size."""
 import numpy as np
 import pytest
 import torch
@@ -126,8 +126,8 @@ def test_routed_layer_small_buckets(k, act):
 
 
 def test_routed_layer_large_buckets_and_lora(k):
-    """Buckets of 150, 70, 30 and 6 rows: the large ones take the GEMM-shaped work-groups, the
-    small ones the one-tile work-groups, both reading the forward layout (each its own way); LoRA
+    """Buckets of 150, 70, 30 and 6 rows: the large ones take wide items of several tiles, the
+    small ones one-tile items, both reading the forward layout (each its own way); LoRA
     deltas join both epilogues."""
     case("routed layer with/without forward layout, large buckets + LoRA r=8")
     rng = np.random.default_rng(62)
